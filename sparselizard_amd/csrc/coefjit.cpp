@@ -30,7 +30,8 @@ std::map<std::string, hipFunction_t> g_cache;  // key: device id + source
 
 }  // namespace
 
-std::string coef_kernel_source(const slx_instr* prog, int n, bool fp64, bool runs, const std::vector<int>& field_nff) {
+std::string coef_kernel_source(const slx_instr* prog, int n, bool fp64, bool runs, const std::vector<int>& field_nff,
+                               const CoefPack& pack) {
     std::ostringstream o;
     // fields whose values a thread gathers once per element (runs of Gauss
     // points, at most SLX_JIT_GATHER_NFF form functions)
@@ -85,6 +86,20 @@ std::string coef_kernel_source(const slx_instr* prog, int n, bool fp64, bool run
          "    {\n"
          "#pragma clang fp contract(off)\n";
     std::vector<std::string> cur(SLX_MAX_PROG_REGS, "(T)0");
+    // records: 16-byte stores, each as soon as its entries are known
+    const int vw = fp64 ? 2 : 4;
+    std::vector<std::string> rec(pack.erec);
+    std::vector<int> open(pack.erec / vw + 1, vw);
+    auto put = [&](int k, const std::string& v) {
+        rec[k] = v;
+        if (--open[k / vw] > 0) return;
+        const int k0 = k / vw * vw;
+        o << "        *(" << (fp64 ? "double2" : "float4") << "*)(ctab + (size_t)e * " << pack.erec << " + " << k0 << ") = "
+          << (fp64 ? "make_double2(" : "make_float4(");
+        for (int c = 0; c < vw; c++) o << (c ? ", " : "") << rec[k0 + c];
+        o << ");\n";
+    };
+    for (int k : pack.pads) put(k, "(T)0");
     for (int pc = 0; pc < n; pc++) {
         const slx_instr& x = prog[pc];
         const std::string a = (x.a >= 0 && x.a < SLX_MAX_PROG_REGS) ? cur[x.a] : "(T)0";
@@ -118,7 +133,11 @@ std::string coef_kernel_source(const slx_instr* prog, int n, bool fp64, bool run
             case SLX_OP_MUL: rhs = a + " * " + bb; break;
             case SLX_OP_POW: rhs = "pow(" + a + ", " + bb + ")"; break;
             case SLX_OP_OUT:
-                o << "        ctab[(size_t)" << x.imm << " * stride + oi] = " << a << " * adet;\n";
+                if (pack.erec > 0) {
+                    if (pack.pos[x.imm] >= 0) put(pack.pos[x.imm], a + " * adet");
+                } else {
+                    o << "        ctab[(size_t)" << x.imm << " * stride + oi] = " << a << " * adet;\n";
+                }
                 continue;
             default: rhs = "apply_unary<T>(" + std::to_string(x.op) + ", " + a + ")"; break;
         }
@@ -130,14 +149,14 @@ std::string coef_kernel_source(const slx_instr* prog, int n, bool fp64, bool run
 }
 
 bool coef_compile(const slx_instr* prog, int n_instr, bool fp64, bool runs, const std::vector<int>& field_nff, hipFunction_t* fn,
-                  std::string* err) {
+                  std::string* err, const CoefPack& pack) {
     *fn = nullptr;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) {
         if (err) *err = "no current device";
         return false;
     }
-    const std::string src = coef_kernel_source(prog, n_instr, fp64, runs, field_nff);
+    const std::string src = coef_kernel_source(prog, n_instr, fp64, runs, field_nff, pack);
     const std::string key = std::to_string(dev) + "\n" + src;
     {
         std::lock_guard<std::mutex> lk(g_mu);

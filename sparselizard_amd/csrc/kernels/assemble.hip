@@ -7,7 +7,8 @@
 //   |det J| (contribution.cpp:147, 200), into the table
 //   ctab[(slot * nq + q) * n_elem + e]  (element fastest: coalesced for kernels
 //   that map lanes to elements), or with qfast ctab[(slot * n_elem + e) * nq + q]
-//   (Gauss point fastest: contiguous per element, for the factorized kernel).
+//   (Gauss point fastest: contiguous per element, for the factorized kernel);
+//   qfast 2 writes the per-element records of DevPack (row-wise assembly).
 // elem_cols: lanes = (element, dof column); per slice, TI tf rows at a time:
 //   Ke[i][j] = sum_q sum_t tf_t[i][q] w_q C_t(e,q) dof_t[j][q]
 //   (contribution.cpp:172-246; the per-term dgemm of densemat.cpp:228-311 with
@@ -39,7 +40,7 @@ typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
 // ctab[(slot * nq + q) * n_elem + e] multiplied by |det J|.
 template <typename T, int V>
 __device__ void run_program(const DevBucket& b, const DevInputs& in, const int (&e)[V], const int (&q)[V], const Geo (&g)[V],
-                            const bool (&on)[V], int nq, int qfast, T* __restrict__ ctab) {
+                            const bool (&on)[V], int nq, int qfast, const DevPack& pk, T* __restrict__ ctab) {
     T reg[SLX_MAX_REGS][V];
     const int64_t stride = (int64_t)nq * b.n_elem;
     for (int pc = 0; pc < b.n_instr; pc++) {
@@ -97,6 +98,13 @@ __device__ void run_program(const DevBucket& b, const DevInputs& in, const int (
                 for (int v = 0; v < V; v++) r[v] = pow(reg[ia][v], reg[ib][v]);
                 break;
             case SLX_OP_OUT:
+                if (qfast == 2) {
+                    const int at = pk.pos[ins.imm];
+#pragma unroll
+                    for (int v = 0; v < V; v++)
+                        if (on[v] && at >= 0) ctab[(size_t)e[v] * pk.erec + at] = reg[ia][v] * (T)fabs(g[v].det);
+                    continue;
+                }
 #pragma unroll
                 for (int v = 0; v < V; v++)
                     if (on[v])
@@ -117,7 +125,7 @@ __device__ void run_program(const DevBucket& b, const DevInputs& in, const int (
 // over the Gauss points); each thread takes V consecutive (element, Gauss
 // point) pairs, element fastest.
 template <typename T, int V>
-__global__ void __launch_bounds__(256) coef_kernel(DevBucket b, DevInputs in, int nq, int qfast, T* __restrict__ ctab) {
+__global__ void __launch_bounds__(256) coef_kernel(DevBucket b, DevInputs in, int nq, int qfast, DevPack pk, T* __restrict__ ctab) {
     const int64_t total = (int64_t)b.n_elem * nq;
     const int64_t idx0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * V;
     if (idx0 >= total) return;
@@ -129,11 +137,17 @@ __global__ void __launch_bounds__(256) coef_kernel(DevBucket b, DevInputs in, in
         const int64_t idx = idx0 + v;
         on[v] = idx < total;
         const int64_t id = on[v] ? idx : idx0;
+        // (records have nq = 1)
         e[v] = qfast ? (int)(id / nq) : (int)(id % b.n_elem);
         q[v] = qfast ? (int)(id % nq) : (int)(id / b.n_elem);
         geometry(b, in.xyz, e[v], q[v], g[v]);
     }
-    run_program<T, V>(b, in, e, q, g, on, nq, qfast, ctab);
+    if (qfast == 2)
+        for (int k = 0; k < pk.n_pads; k++)
+#pragma unroll
+            for (int v = 0; v < V; v++)
+                if (on[v]) ctab[(size_t)e[v] * pk.erec + pk.pads[k]] = (T)0;
+    run_program<T, V>(b, in, e, q, g, on, nq, qfast, pk, ctab);
 }
 
 // Element matrices, one lane per (element, dof column): `jc` consecutive
@@ -563,16 +577,16 @@ __global__ void reduce_rhs(DevReduce rd, const KT* __restrict__ ke, double* __re
 
 // ---------------------------------------------------------------- launchers --
 
-hipError_t launch_coef(const DevBucket& b, const DevInputs& in, bool fp64, void* ctab, hipStream_t st, int qfast) {
+hipError_t launch_coef(const DevBucket& b, const DevInputs& in, bool fp64, void* ctab, hipStream_t st, int qfast, const DevPack& pk) {
     if (b.n_elem == 0 || b.n_coefs == 0) return hipSuccess;
     const int nq = b.q_inv ? 1 : b.n_gp;
     const int64_t n = (int64_t)b.n_elem * nq;
     if (fp64) {
         const unsigned grid = (unsigned)((n + 2 * 256 - 1) / (2 * 256));
-        hipLaunchKernelGGL((coef_kernel<double, 2>), dim3(grid), dim3(256), 0, st, b, in, nq, qfast, (double*)ctab);
+        hipLaunchKernelGGL((coef_kernel<double, 2>), dim3(grid), dim3(256), 0, st, b, in, nq, qfast, pk, (double*)ctab);
     } else {
         const unsigned grid = (unsigned)((n + 4 * 256 - 1) / (4 * 256));
-        hipLaunchKernelGGL((coef_kernel<float, 4>), dim3(grid), dim3(256), 0, st, b, in, nq, qfast, (float*)ctab);
+        hipLaunchKernelGGL((coef_kernel<float, 4>), dim3(grid), dim3(256), 0, st, b, in, nq, qfast, pk, (float*)ctab);
     }
     return hipGetLastError();
 }

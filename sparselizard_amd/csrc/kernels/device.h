@@ -51,6 +51,14 @@ struct DevInputs {
     const double* field_data[SLX_MAX_FIELDS];
 };
 
+// Record layout of a bucket's coefficients: slot s of element e at
+// e * erec + pos[s] (pos < 0: not stored), zeros at the pads.
+struct DevPack {
+    const int32_t* pos;
+    const int32_t* pads;
+    int32_t n_pads, erec;
+};
+
 // Reduction maps of the cached CSR pattern.
 struct DevReduce {
     int64_t nrows;                  // free rows

@@ -19,6 +19,7 @@
 #include "kernels/mfma.h"
 #include "kernels/factor.h"
 #include "kernels/tile.h"
+#include "kernels/direct.h"
 #include "kernels/solve.h"
 #include "kernels/symbolic.h"
 #include "coefjit.h"
@@ -29,7 +30,7 @@
 #include <dlfcn.h>
 
 namespace slx {
-hipError_t launch_coef(const DevBucket& b, const DevInputs& in, bool fp64, void* ctab, hipStream_t st, int qfast);
+hipError_t launch_coef(const DevBucket& b, const DevInputs& in, bool fp64, void* ctab, hipStream_t st, int qfast, const DevPack& pk);
 hipError_t launch_elem(const DevBucket& b, const void* ctab, int precision, void* ke, hipStream_t st, uint32_t slice_mask, int qfast);
 hipError_t scratch_init(int device);
 hipError_t launch_reduce(const DevReduce& rd, int max_erow_len, bool ke_fp64, const void* ke, double* Aval, double* Dval,
@@ -221,6 +222,16 @@ struct slx_plan_s {
     const void* last_ctab = nullptr;   // coefficient table of the last bucket assembled
     int n_cu = 256;
 
+    // row-wise assembly (kernels/direct.hip): the matrix bucket, and the bucket
+    // of the right-hand side when it is summed in the same launch (-1: not)
+    bool direct = false;
+    int direct_bucket = -1, direct_rhs_bucket = -1;
+    bool needs_ke = true;              // some kernel of the numeric phase writes element matrices
+    DirectDev dd{};
+    DirectBuild dbuild{};
+    CoefPack pack;                     // record layout of the matrix bucket's coefficients
+    DevPack dpack{};
+
     DBuf* newbuf() {
         bufs.emplace_back(new DBuf());
         return bufs.back().get();
@@ -393,7 +404,7 @@ void finish_plan(slx_plan_s& P, const slx_plan_desc& d, int slot_bytes, int maxr
     }
     // Ke buffer (FP64 capacity serves every precision)
     P.ke_capacity_bytes = std::max<int64_t>(P.n_ke, 1) * sizeof(double);
-    P.d_ke.alloc(P.ke_capacity_bytes);
+    if (P.needs_ke) P.d_ke.alloc(P.ke_capacity_bytes);
 }
 
 // Symbolic phase on the host: element-row lists in the reference
@@ -1494,7 +1505,7 @@ void build_tile(slx_plan_s& P, const slx_bucket_desc& bd, int b, const KeLayout&
     }
 }
 
-void compile_coef_programs(slx_plan_s& P, const slx_plan_desc& d);
+
 
 // The fused launch (kernels/factor.hip, launch_factor_fused): when two or more
 // buckets have factorized slices, their coefficient tables get regions of
@@ -1569,6 +1580,251 @@ void build_fused(slx_plan_s& P, const slx_plan_desc& d) {
         P.fused_lds[a] = lds;
         if (!tab.empty()) upload(P.d_fused[a], tab.data(), tab.size(), P.stream);
     }
+}
+
+// Bits that number n values.
+int bits_for(int64_t n) {
+    int b = 0;
+    while ((int64_t(1) << b) < n) b++;
+    return b;
+}
+
+// Row-wise assembly (kernels/direct.hip) replaces the element kernels and the
+// reduction of a plan when
+//  - one bucket holds every matrix slice and its coefficients are constant over
+//    the Gauss points (affine elements, element-wise material);
+//  - its slices share one tf and one dof table and form equal segment groups
+//    (at most SLX_DIRECT_MAXB dof fields, SLX_DIRECT_MAXP derivative pairs),
+//    with one coefficient slot per (slice, derivative pair) and no signs;
+//  - the segment words fit 32 bits and the Gauss-point sums 32 KB of LDS.
+// The right-hand side joins the launch when its slices sit in one such bucket
+// with one term each; otherwise it keeps its kernels (and then must not share
+// the matrix bucket).  Measured against the element kernels with the
+// reduction, whole assemblies: 48^3 x 6 P2 elasticity 1.19 vs 1.90 ms (FP16
+// split), 21^3 x 6 in FP64 0.145 vs 0.72 ms, 200^2 x 2 P1 Poisson 0.011 vs
+// 0.040 ms (three launches instead of six and no side stream); no class
+// measured slower.
+// SLX_TUNE_DIRECT=0 and SLX_TUNE_TABLE=none keep the element kernels.
+void choose_direct(slx_plan_s& P, const slx_plan_desc& d, const KeLayout& L) {
+    P.direct = false;
+    P.needs_ke = true;
+    if (const char* t = std::getenv("SLX_TUNE_DIRECT"))
+        if (std::atoi(t) == 0) return;
+    if (const char* t = std::getenv("SLX_TUNE_TABLE"))
+        if (std::string(t) == "none") return;
+    if (!d.has_matrix) return;
+    int mb = -1;
+    for (int b = 0; b < d.n_buckets; b++)
+        for (int s = 0; s < d.buckets[b].n_slices; s++)
+            if (!d.buckets[b].slices[s].is_rhs && mb != b) {
+                if (mb >= 0) return;
+                mb = b;
+            }
+    if (mb < 0) return;
+    const slx_bucket_desc& bd = d.buckets[mb];
+    if (bd.n_elem == 0 || !bd.q_invariant) return;
+    std::vector<const SegGroup*> groups;
+    for (const SegGroup& G : L.groups)
+        if (G.bucket == mb && !G.rhs) groups.push_back(&G);
+    const SegGroup& g0 = *groups[0];
+    const slx_slice_desc& s0 = bd.slices[g0.slices[0]];
+    if (groups.size() > 8) return;
+    std::vector<std::pair<int, int>> pairs;
+    for (const SegGroup* G : groups) {
+        if (G->n_tf != g0.n_tf || G->slices.size() != g0.slices.size() || G->ld != g0.ld) return;
+        for (int s : G->slices) {
+            const slx_slice_desc& sd = bd.slices[s];
+            if (sd.n_dof != s0.n_dof || sd.tf_table != s0.tf_table || sd.dof_table != s0.dof_table || sd.tf_sign || sd.dof_sign) return;
+            for (int t = 0; t < sd.n_terms; t++) {
+                const std::pair<int, int> pr(sd.terms[t].tf_deriv, sd.terms[t].dof_deriv);
+                if (std::find(pairs.begin(), pairs.end(), pr) == pairs.end()) pairs.push_back(pr);
+            }
+        }
+    }
+    if (pairs.empty() || pairs.size() > SLX_DIRECT_MAXP) return;
+    DirectDev dd{};
+    dd.n_tf = g0.n_tf;
+    dd.n_dof = s0.n_dof;
+    dd.na = (int)groups.size();
+    dd.nb = (int)g0.slices.size();
+    if (!direct_shape(dd, (int)pairs.size())) return;
+    dd.ib = bits_for(dd.n_tf);
+    if (dd.ib > 12 || (int64_t(1) << (32 - dd.ib)) < (int64_t)bd.n_elem * dd.na) return;
+    const int kc = (dd.nb * dd.P + 3) / 4 * 4;
+    // right-hand-side coefficients of the same bucket follow the groups' own
+    int n_rhs_slots = 0;
+    for (int s = 0; s < bd.n_slices; s++) n_rhs_slots += bd.slices[s].is_rhs ? 1 : 0;
+    const int rtail = (n_rhs_slots + dd.na - 1) / dd.na;
+    dd.rec = kc + (rtail + 3) / 4 * 4;
+    dd.n_cu = P.n_cu;
+    CoefPack pack;
+    pack.pos.assign(std::max(bd.n_coefs, 1), -1);
+    for (int a = 0; a < dd.na; a++)
+        for (int f = 0; f < dd.nb; f++) {
+            const slx_slice_desc& sd = bd.slices[groups[a]->slices[f]];
+            // the segment's columns: slice f at f * n_dof
+            if (L.ke_base[mb][groups[a]->slices[f]] - groups[a]->base != (int64_t)f * dd.n_dof) return;
+            std::vector<uint8_t> have(pairs.size(), 0);
+            for (int t = 0; t < sd.n_terms; t++) {
+                const std::pair<int, int> pr(sd.terms[t].tf_deriv, sd.terms[t].dof_deriv);
+                const int p = (int)(std::find(pairs.begin(), pairs.end(), pr) - pairs.begin());
+                int& at = pack.pos[sd.terms[t].coef];
+                if (have[p] || at >= 0) return;
+                have[p] = 1;
+                at = a * dd.rec + f * dd.P + p;
+            }
+        }
+    // right-hand side: one bucket, constant coefficients, one term per slice
+    int rb = -1;
+    bool rhs_ok = true, rhs_any = false;
+    for (int b = 0; b < d.n_buckets; b++)
+        for (int s = 0; s < d.buckets[b].n_slices; s++) {
+            const slx_slice_desc& sd = d.buckets[b].slices[s];
+            if (!sd.is_rhs) continue;
+            rhs_any = true;
+            if (rb < 0) rb = b;
+            if (rb != b || !d.buckets[b].q_invariant || sd.n_terms != 1 || sd.tf_sign) rhs_ok = false;
+        }
+    int64_t nk = 0;
+    if (rb >= 0 && rhs_ok) {
+        for (int s = 0; s < d.buckets[rb].n_slices; s++)
+            if (d.buckets[rb].slices[s].is_rhs) nk += d.buckets[rb].slices[s].n_tf;
+        dd.rib = bits_for(nk);
+        if (dd.rib > 12 || (int64_t(1) << (32 - dd.rib)) < d.buckets[rb].n_elem) rhs_ok = false;
+    }
+    pack.erec = dd.na * dd.rec;
+    if (n_rhs_slots > 0) {
+        // without this launch those slices' kernels need the bucket's slot layout
+        if (rb != mb || !rhs_ok || !d.has_rhs) return;
+        int n = 0;
+        for (int s = 0; s < bd.n_slices; s++)
+            if (bd.slices[s].is_rhs) {
+                int& at = pack.pos[bd.slices[s].terms[0].coef];
+                if (at < 0) {
+                    at = n / rtail * dd.rec + kc + n % rtail;
+                    n++;
+                } else if (at % dd.rec < kc) {
+                    return;
+                }
+            }
+    }
+    std::vector<uint8_t> used(pack.erec, 0);
+    for (int at : pack.pos)
+        if (at >= 0) used[at] = 1;
+    for (int k = 0; k < pack.erec; k++)
+        if (!used[k]) pack.pads.push_back(k);
+    dd.has_rhs = d.has_rhs && rhs_ok ? 1 : 0;
+    P.direct = true;
+    P.direct_bucket = mb;
+    P.direct_rhs_bucket = dd.has_rhs ? rb : -1;
+    P.needs_ke = d.has_rhs && !dd.has_rhs;
+    P.pack = pack;
+    P.dd = dd;
+    // Gauss-point sums, in FP64
+    const double* tf = bd.tables[s0.tf_table];
+    const double* df = bd.tables[s0.dof_table];
+    const int ngp = bd.n_gp;
+    std::vector<double> phi((size_t)dd.n_tf * dd.G * dd.phi_row, 0.0);
+    for (int i = 0; i < dd.n_tf; i++)
+        for (int j = 0; j < dd.n_dof; j++)
+            for (size_t p = 0; p < pairs.size(); p++) {
+                double s = 0.0;
+                for (int q = 0; q < ngp; q++)
+                    s += bd.gp_weights[q] * tf[((size_t)pairs[p].first * dd.n_tf + i) * ngp + q] *
+                         df[((size_t)pairs[p].second * dd.n_dof + j) * ngp + q];
+                phi[((size_t)i * dd.G + j / dd.JL) * dd.phi_row + p * dd.JL + j % dd.JL] = s;
+            }
+    const std::vector<float> phi32(phi.begin(), phi.end());
+    P.dd.phi64 = P.dev(phi.data(), phi.size());
+    P.dd.phi32 = P.dev(phi32.data(), phi32.size());
+    DirectBuild& B = P.dbuild;
+    B = DirectBuild{};
+    B.seg_len = (int)g0.len;
+    B.n_elem = bd.n_elem;
+    B.ld = (int)g0.ld;
+    for (int a = 0; a < dd.na; a++) B.group_base[a] = groups[a]->base;
+    if (dd.has_rhs && rb >= 0) {
+        const slx_bucket_desc& rd = d.buckets[rb];
+        std::vector<double> rphi;
+        std::vector<int64_t> rbase;
+        B.rn_elem = rd.n_elem;
+        for (const SegGroup& G : L.groups) {
+            if (G.bucket != rb || !G.rhs) continue;
+            const slx_slice_desc& sd = rd.slices[G.slices[0]];
+            B.rgroup_base[B.n_rgroups] = G.base;
+            B.rgroup_ntf[B.n_rgroups] = sd.n_tf;
+            B.rgroup_k[B.n_rgroups++] = (int)rphi.size();
+            const double* t = rd.tables[sd.tf_table];
+            for (int i = 0; i < sd.n_tf; i++) {
+                double s = 0.0;
+                for (int q = 0; q < rd.n_gp; q++) s += rd.gp_weights[q] * t[((size_t)sd.terms[0].tf_deriv * sd.n_tf + i) * rd.n_gp + q];
+                rphi.push_back(s);
+                rbase.push_back(rb == mb ? pack.pos[sd.terms[0].coef] : (int64_t)sd.terms[0].coef * rd.n_elem);
+            }
+        }
+        const std::vector<float> rphi32(rphi.begin(), rphi.end());
+        P.dd.rstride = rb == mb ? pack.erec : 1;
+        P.dd.rphi64 = P.dev(rphi.data(), rphi.size());
+        P.dd.rphi32 = P.dev(rphi32.data(), rphi32.size());
+        P.dd.rbase = P.dev(rbase.data(), rbase.size());
+    }
+    std::vector<int32_t> pos(pack.pos.begin(), pack.pos.end()), pads(pack.pads.begin(), pack.pads.end());
+    P.dpack.pos = P.dev(pos.data(), pos.size());
+    P.dpack.pads = pads.empty() ? nullptr : P.dev(pads.data(), pads.size());
+    P.dpack.n_pads = (int)pads.size();
+    P.dpack.erec = pack.erec;
+}
+
+// The row-wise maps, once the pattern is known; a pattern it cannot take
+// (32-bit slots, rows beyond the LDS accumulators) returns the bucket to the
+// element kernels.
+void build_direct(slx_plan_s& P, const slx_plan_desc& d, const KeLayout& L) {
+    if (!P.direct) return;
+    DirectDev& dd = P.dd;
+    if (P.rd.slot_bytes > 2 || P.rd.max_row_len > direct_max_row(dd) || P.nfree >= (int64_t(1) << 32) || P.red_classes.size() > 255) {
+        P.direct = false;
+        const slx_bucket_desc& bd = d.buckets[P.direct_bucket];
+        build_mfma(P, bd, P.direct_bucket, L);
+        build_tile(P, bd, P.direct_bucket, L);
+        build_factor(P, bd, P.direct_bucket, L);
+        if (!P.needs_ke) P.d_ke.alloc(P.ke_capacity_bytes);
+        P.needs_ke = true;
+        return;
+    }
+    DirectBuild& B = P.dbuild;
+    B.nrows = P.nfree;
+    B.n_erows = P.n_erows;
+    B.n_rhs = P.n_rhs_erows;
+    B.rdesc = P.d_rdesc.as<uint64_t>();
+    B.erows = P.d_erows.as<uint64_t>();
+    B.rhs_erows = P.d_rhs_erows.as<uint64_t>();
+    B.slots = P.d_slots.p;
+    B.slot_bytes = P.rd.slot_bytes;
+    dd.nrows = P.nfree;
+    dd.slot_bytes = P.rd.slot_bytes;
+    dd.slot_words = (dd.nb * dd.JL * dd.slot_bytes + 3) / 4;
+    dd.free_dofs = P.d_free.as<int64_t>();
+    dd.rptr = P.d_rhs_ptr.as<int64_t>();
+    const int64_t padl = (B.seg_len + 3) / 4 * 4, blocks = P.n_slots_w / padl;
+    DBuf* desc = P.newbuf();
+    DBuf* seg = P.newbuf();
+    DBuf* slots = P.newbuf();
+    DBuf* rseg = P.newbuf();
+    desc->alloc(std::max<int64_t>(4 * P.nfree, 4) * sizeof(uint64_t));
+    seg->alloc((P.n_erows + SLX_DIRECT_PAD) * sizeof(uint32_t));
+    slots->alloc((blocks + SLX_DIRECT_PAD) * dd.G * dd.slot_words * sizeof(uint32_t));
+    rseg->alloc(std::max<int64_t>(P.n_rhs_erows, 1) * sizeof(uint32_t));
+    std::vector<int64_t> cb, ce;
+    for (const RedClass& c : P.red_classes) {
+        cb.push_back(c.begin);
+        ce.push_back(c.end);
+    }
+    HIPCHECK(launch_direct_build(dd, B, desc->as<uint64_t>(), seg->as<uint32_t>(), slots->as<uint32_t>(), rseg->as<uint32_t>(), P.stream,
+                                 cb.data(), ce.data(), (int)cb.size()));
+    dd.desc = desc->as<uint64_t>();
+    dd.seg = seg->as<uint32_t>();
+    dd.slots = slots->as<uint32_t>();
+    dd.rseg = rseg->as<uint32_t>();
 }
 
 void upload_buckets(slx_plan_s& P, const slx_plan_desc& d, const KeLayout& L) {
@@ -1692,15 +1948,19 @@ void upload_buckets(slx_plan_s& P, const slx_plan_desc& d, const KeLayout& L) {
         // element node numbers must be in range of the node array
         for (size_t k = 0; k < (size_t)bd.n_elem * bd.n_geo; k++)
             SLX_CHECK(bd.geo_nodes[k] >= 0 && bd.geo_nodes[k] < d.n_nodes, "element node out of range");
-        build_mfma(P, bd, b, L);
-        build_tile(P, bd, b, L);
-        build_factor(P, bd, b, L);
+    }
+    choose_direct(P, d, L);
+    for (int b = 0; b < d.n_buckets; b++) {
+        if (P.direct && b == P.direct_bucket) continue;
+        build_mfma(P, d.buckets[b], b, L);
+        build_tile(P, d.buckets[b], b, L);
+        build_factor(P, d.buckets[b], b, L);
     }
     upload(P.consts, d.consts, (size_t)std::max(d.n_consts, 1), P.stream);
+    if (P.direct) ctab_words = std::max(ctab_words, (size_t)P.pack.erec * std::max(d.buckets[P.direct_bucket].n_elem, 1));
     P.d_ctab.alloc(ctab_words * sizeof(double));
     P.d_ctab_side.alloc(ctab_side_words * sizeof(double));
     build_fused(P, d);
-    compile_coef_programs(P, d);
     P.side_ok = d.has_matrix && d.has_rhs && any_rhs_only && !rhs_in_mixed;
     if (P.side_ok) {
         HIPCHECK(hipStreamCreateWithFlags(&P.side, hipStreamNonBlocking));
@@ -1736,7 +1996,9 @@ void compile_coef_programs(slx_plan_s& P, const slx_plan_desc& d) {
                 for (int f = 0; f < d.n_fields; f++) fnff[f] = d.field_nff[(size_t)f * d.n_buckets + todo[i].first];
                 hipFunction_t fn = nullptr;
                 std::string err;
-                if (coef_compile(bd.prog, bd.n_instr, todo[i].second != 0, bd.q_invariant == 0, fnff, &fn, &err)) {
+                const bool records = P.direct && todo[i].first == P.direct_bucket;
+                if (coef_compile(bd.prog, bd.n_instr, todo[i].second != 0, bd.q_invariant == 0, fnff, &fn, &err,
+                                 records ? P.pack : CoefPack())) {
                     P.coef_fn[todo[i].first][todo[i].second] = fn;
                 } else {
                     std::lock_guard<std::mutex> lk(mu);
@@ -1803,7 +2065,8 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
                       : precision == SLX_PREC_FP32_MFMA ? AR_F32 : -1;
     // fork: rhs-only buckets and the rhs reduction overlap the matrix work
     // (serial when every launch is timed)
-    const bool overlap = P.side_ok && !tm;
+    // (a row-wise right-hand side is part of the matrix launch)
+    const bool overlap = P.side_ok && !tm && !(P.direct && P.dd.has_rhs);
     if (overlap) {
         HIPCHECK(hipEventRecord(P.ev_fork, st));
         HIPCHECK(hipStreamWaitEvent(P.side, P.ev_fork, 0));
@@ -1836,7 +2099,7 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
             else {
                 SLX_CHECK(b.n_regs <= SLX_MAX_REGS, "coefficient program of " << b.n_regs << " registers has no compiled kernel and the interpreter holds "
                                                    << SLX_MAX_REGS << " (" << P.coef_jit_error << ")");
-                HIPCHECK(launch_coef(b, in, ke64, ctab, st, 1));
+                HIPCHECK(launch_coef(b, in, ke64, ctab, st, 1, P.dpack));
             }
             if (tm) tm->end();
         }
@@ -1854,8 +2117,10 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
         void* ctab = in_fused ? (void*)((char*)P.d_ctab_fused.p + P.fuse_off[bi]) : (P.rhs_only[bi] ? P.d_ctab_side.p : P.d_ctab.p);
         uint32_t all = (b.n_slices >= 32) ? 0xffffffffu : ((1u << b.n_slices) - 1u);
         uint32_t done = 0;
-        // the factorized kernel reads the coefficients of one element contiguously
-        const int qfast = fmask != 0 ? 1 : 0;
+        // the factorized kernel reads the coefficients of one element contiguously,
+        // the row-wise kernel reads records
+        const bool records = P.direct && (int)bi == P.direct_bucket;
+        const int qfast = records ? 2 : fmask != 0 ? 1 : 0;
         P.last_qfast = qfast;
         P.last_ctab = ctab;
         if (!in_fused) {
@@ -1865,10 +2130,11 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
             else {
                 SLX_CHECK(b.n_regs <= SLX_MAX_REGS, "coefficient program of " << b.n_regs << " registers has no compiled kernel and the interpreter holds "
                                                    << SLX_MAX_REGS << " (" << P.coef_jit_error << ")");
-                HIPCHECK(launch_coef(b, in, ke64, ctab, bst, qfast));
+                HIPCHECK(launch_coef(b, in, ke64, ctab, bst, qfast, P.dpack));
             }
             if (tm) tm->end();
         }
+        if (records || (P.direct && (int)bi == P.direct_rhs_bucket)) continue;  // the row-wise launch does the rest
         if (arith >= 0 && P.mfma[bi].M > 0 && ((P.mfma[bi].arith_ok >> arith) & 1u)) {
             if (tm) tm->begin(T_MFMA);
             HIPCHECK(launch_mfma(b, mfma_for(P.mfma[bi], arith), (const float*)ctab, P.d_ke.as<float>(), bst));
@@ -1911,11 +2177,16 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
             ce.push_back(c.end);
             cl.push_back(c.max_len);
         }
+        if (P.direct)
+            HIPCHECK(launch_direct(P.dd, ke64, P.d_ctab.p, P.direct_rhs_bucket == P.direct_bucket ? P.d_ctab.p : P.d_ctab_side.p,
+                                   P.d_Aval.as<double>(), P.d_Dval.as<double>(), P.d_rhs.as<double>(), st, cb.data(), ce.data(), cl.data(),
+                                   (int)cl.size()));
+        else
         HIPCHECK(launch_reduce(P.rd, P.max_erow_len, ke64, P.d_ke.p, P.d_Aval.as<double>(), P.d_Dval.as<double>(), P.d_rhs.as<double>(),
                                true, false, st, cb.data(), ce.data(), cl.data(), (int)cl.size()));
         if (tm) tm->end();
     }
-    if (P.has_rhs) {
+    if (P.has_rhs && !(P.direct && P.dd.has_rhs)) {
         if (tm) tm->begin(T_RHS);
         HIPCHECK(launch_reduce(P.rd, P.max_erow_len, ke64, P.d_ke.p, P.d_Aval.as<double>(), P.d_Dval.as<double>(), P.d_rhs.as<double>(),
                                false, true, overlap ? P.side : st, nullptr, nullptr, nullptr, 0));
@@ -1987,6 +2258,10 @@ slx_status slx_plan_create_ex(slx_ctx ctx, const slx_plan_desc* desc, int32_t fl
         if (!done) {
             check_addresses(desc);
             build_symbolic(*P, *desc, L);
+        }
+        if (!P->host_only) {
+            build_direct(*P, *desc, L);
+            compile_coef_programs(*P, *desc);
         }
         P->symbolic_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
         if (!P->host_only) HIPCHECK(hipStreamSynchronize(P->stream));
@@ -2495,11 +2770,12 @@ slx_status slx_plan_coefficients(slx_plan p, double* out, int64_t cap, int64_t* 
         SLX_CHECK(p->last_precision >= 0 && !p->dbuckets.empty(), "no assembly has run on this plan");
         const DevBucket& b = p->dbuckets.back();
         const void* ctab = p->last_ctab;
-        const int64_t n = (int64_t)b.n_coefs * (b.q_inv ? 1 : b.n_gp) * b.n_elem;
+        int64_t n = (int64_t)b.n_coefs * (b.q_inv ? 1 : b.n_gp) * b.n_elem;
         *n_out = n;
         if (!out) return;
         SLX_CHECK(cap >= n, "output holds " << cap << " entries, the table has " << n);
         HIPCHECK(hipStreamSynchronize(p->stream));
+        if (p->last_qfast == 2) n = (int64_t)p->pack.erec * b.n_elem;
         std::vector<double> tmp(n);
         if (p->last_precision == SLX_PREC_FP64) {
             HIPCHECK(hipMemcpy(tmp.data(), ctab, (size_t)n * sizeof(double), hipMemcpyDeviceToHost));
@@ -2509,7 +2785,11 @@ slx_status slx_plan_coefficients(slx_plan p, double* out, int64_t cap, int64_t* 
             for (int64_t i = 0; i < n; i++) tmp[i] = t32[i];
         }
         const int64_t nq = b.q_inv ? 1 : b.n_gp, ne = b.n_elem;
-        if (p->last_qfast) {
+        if (p->last_qfast == 2) {
+            // the row-wise kernel's records (element, position) -> (slot, element)
+            for (int c = 0; c < b.n_coefs; c++)
+                for (int64_t e = 0; e < ne; e++) out[c * ne + e] = p->pack.pos[c] >= 0 ? tmp[e * p->pack.erec + p->pack.pos[c]] : 0.0;
+        } else if (p->last_qfast) {
             // the factorized kernels' layout (slot, element, q) -> (slot, q, element)
             for (int64_t i = 0; i < n; i++) {
                 const int64_t c = i / (nq * ne), r = i % (nq * ne), e = r / nq, q = r % nq;
@@ -2528,6 +2808,13 @@ slx_status slx_plan_element_matrices(slx_plan p, double* out, int64_t cap) {
         SLX_CHECK(p->last_precision >= 0, "no assembly has run on this plan");
         SLX_CHECK(cap >= p->n_ke, "output holds " << cap << " entries, the element matrices have " << p->n_ke);
         HIPCHECK(hipStreamSynchronize(p->stream));
+        if (p->direct) {
+            // row-wise plans keep no element matrices: from the last assembly's coefficients
+            if (!p->d_ke.p) p->d_ke.alloc(p->ke_capacity_bytes);
+            HIPCHECK(launch_direct_ke(p->dd, p->dbuild, p->last_precision == SLX_PREC_FP64, p->d_ctab.p,
+                                      p->direct_rhs_bucket == p->direct_bucket ? p->d_ctab.p : p->d_ctab_side.p, p->d_ke.p, p->stream));
+            HIPCHECK(hipStreamSynchronize(p->stream));
+        }
         if (p->last_precision == SLX_PREC_FP64) {
             HIPCHECK(hipMemcpy(out, p->d_ke.p, (size_t)p->n_ke * sizeof(double), hipMemcpyDeviceToHost));
         } else {

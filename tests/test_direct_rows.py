@@ -1,0 +1,89 @@
+"""Row-wise assembly (kernels/direct.hip) against the oracle: every shape of
+the kernel (one or three dof fields, 4, 6, 9 and 12 derivative pairs, two or
+three columns per lane), one to many elements, compiled and interpreted
+coefficients, and the element kernels that SLX_TUNE_DIRECT=0 keeps.
+
+Gates: FP64 1e-12; the reduced modes run this kernel in FP32, whose entries are
+sums of at most 12 products of rounded factors (below 14 * 6e-8 of the sum of
+magnitudes), so 1e-6.
+"""
+import numpy as np
+import pytest
+
+import sparselizard_amd as sa
+from oracle import py_oracle
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    ("poisson2d", "n=2"),               # one free row
+    ("poisson2d", "n=9"),               # 3 x 3, 4 pairs, three columns per lane
+    ("poisson2d", "n=70"),              # compiled coefficients, several workgroups
+    ("poisson2d", "n=7;order=2"),       # 6 x 6, two lanes per row
+    ("convdiff2d", "n=8"),              # 6 pairs
+    ("convdiff2d", "n=6;order=2"),
+    ("elasticity3d", "n=2;order=1"),    # 4 x 4, three fields, 9 pairs
+    ("elasticity3d", "n=3"),            # 10 x 10, five lanes per row
+    ("elasticity3d", "n=10"),           # compiled records, three row classes
+    ("elasticity3d", "n=2;clamp=0"),    # no constrained column
+]
+
+
+def relerr(a, b):
+    return np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300)
+
+
+def check(prob, plan, tol):
+    info = prob.info()
+    got = plan.csr(info["ndofs"])
+    ref = py_oracle.assemble(prob.desc_ptr(), prob.numeric(), info["ndofs"], info["nfree"])
+    for name in ("Arow", "Acol", "Drow", "Dcol"):
+        assert np.array_equal(getattr(got, name), getattr(ref, name)), name
+    for name in ("Aval", "Dval", "rhs"):
+        assert relerr(getattr(got, name), getattr(ref, name)) <= tol, name
+    return got
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("f16split", 1e-6), ("bf16split", 1e-6), ("fp32mfma", 1e-6), ("fp32", 1e-6)])
+@pytest.mark.parametrize("kind,spec", CASES)
+def test_rows_match_oracle(ctx, kind, spec, precision, tol):
+    print("case direct", kind, spec, precision, flush=True)
+    prob = sa.Problem(ctx, kind, spec)
+    plan = prob.generate(precision)
+    assert plan.kernel_counts("f16split") == dict(batched=0, factorized=0)
+    a = check(prob, plan, tol)
+    b = prob.generate(precision).csr(prob.info()["ndofs"])
+    assert np.array_equal(a.Aval, b.Aval) and np.array_equal(a.Dval, b.Dval) and np.array_equal(a.rhs, b.rhs)
+
+
+@pytest.mark.parametrize("kind,spec", [("poisson2d", "n=9"), ("elasticity3d", "n=3")])
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("fp32", 1e-6)])
+def test_compiled_records(ctx, kind, spec, precision, tol):
+    prob = sa.Problem(ctx, kind, spec)
+    plan = prob.plan()
+    assert plan.coef_mode("compiled") > 0
+    check(prob, prob.generate(precision), tol)
+
+
+@pytest.mark.parametrize("kind,spec", [("poisson2d", "n=9"), ("convdiff2d", "n=8"), ("elasticity3d", "n=3")])
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-13), ("fp32", 1e-6)])
+def test_element_kernels_agree(ctx, kind, spec, precision, tol, monkeypatch):
+    """Element matrices, coefficients and system equal those of the element kernels."""
+    prob = sa.Problem(ctx, kind, spec)
+    plan = prob.generate(precision)
+    ke, co, got = plan.element_matrices(), plan.coefficients(), plan.csr(prob.info()["ndofs"])
+    monkeypatch.setenv("SLX_TUNE_DIRECT", "0")
+    prob2 = sa.Problem(ctx, kind, spec)
+    plan2 = prob2.generate(precision)
+    kb, kl = plan2.ke_layout()
+    d, sel, k = prob2.desc(), [], 0
+    for b in range(d.n_buckets):
+        for s in range(d.buckets[b].n_slices):
+            sd = d.buckets[b].slices[s]
+            e, i, j = np.meshgrid(np.arange(d.buckets[b].n_elem), np.arange(sd.n_tf), np.arange(1 if sd.is_rhs else sd.n_dof), indexing="ij")
+            sel.append((kb[k] + (e * sd.n_tf + i) * kl[k] + j).ravel())
+            k += 1
+    sel = np.concatenate(sel)
+    assert relerr(ke[sel], plan2.element_matrices()[sel]) <= tol
+    assert np.array_equal(co, plan2.coefficients())
+    assert relerr(got.Aval, plan2.csr(prob2.info()["ndofs"]).Aval) <= tol
