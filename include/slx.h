@@ -271,7 +271,9 @@ slx_status slx_plan_fused_info(slx_plan plan, int32_t precision, int32_t* n_slic
  * or after max_outer refinements; max_inner bounds the inner iterations of
  * one refinement.  Returns the counts, the final relative FP64 residual and
  * the method used; not reaching rel_tol is reported through rel_residual,
- * not as an error.  Allocates its device workspace per call.  x_out: host
+ * not as an error.  Its device workspace stays with the plan up to 256 MiB;
+ * a larger one, or one for a call that overlaps another solve of the same
+ * plan, is allocated for the call.  x_out: host
  * (d_x_out NULL) or device (x_out NULL) memory. */
 #define SLX_SOLVE_AUTO 0
 #define SLX_SOLVE_CG 1

@@ -11,7 +11,10 @@
         if (_e != hipSuccess) return _e;       \
     } while (0)
 
-#define SLX_SOLVE_BLOCKS 2048  // fixed grid of the partial-sum kernels
+#define SLX_SOLVE_BLOCKS 1024  // partial sums of one dot product at most
+#define SLX_SOLVE_PART 2048    // half the doubles of the partial sums in the workspace
+#define SLX_ROWS_MAX 1024      // longest row of the row-wise FP32 product
+#define SLX_GMRES_CHECK 8      // GMRES iterations between looks at the residual
 #define SLX_STREAM_NNZ 4096    // nonzeros of one row block of the streaming FP32 product
 #define SLX_GMRES_MAX 100        // Krylov vectors per GMRES cycle at most
 #define SLX_XCDS 8              // XCDs of the device (SLX_SOLVE_BLOCKS is a multiple)
@@ -28,6 +31,7 @@ struct SolveSystem {
     const int64_t* cons_dofs;   // [ncons] dof of each D column
     const int64_t* Ablk;        // [nblk + 1] row blocks of A (stream_row_blocks)
     int64_t nblk;
+    int max_row;                // longest row of A
 };
 
 struct SolveParams {
@@ -44,13 +48,13 @@ struct SolveStats {
 };
 
 // device workspace: nfree doubles f, r, x; ncons doubles xd; n_dofs doubles
-// xfull; 2 * SLX_SOLVE_BLOCKS + 8 doubles part / sc; nfree floats r32, z, p,
+// xfull; 2 * SLX_SOLVE_PART + 8 doubles part / sc; nfree floats r32, z, p,
 // q, d, dinv; nnzA floats val32 (16-byte aligned)
 struct SolveWork {
     double *f, *r, *x, *xd, *xfull, *part, *sc;
     float *r32, *z, *p, *q, *d, *dinv, *val32;
     // GMRES only: Krylov basis [restart + 1][nfree] floats, partial sums
-    // [restart + 1][SLX_SOLVE_BLOCKS] and restart + 1 coefficients (doubles)
+    // [restart + 1][SLX_SOLVE_PART] and restart + 1 coefficients (doubles)
     float* V;
     double *mpart, *hv;
 };
@@ -70,8 +74,8 @@ hipError_t eliminate_system(const SolveSystem& s, const double* b, double* out, 
 // (x, y: n_dofs entries; xa, ya: nfree work; xd: ncons work)
 hipError_t matvec_system(const SolveSystem& s, const double* x, double* y, double* xa, double* xd, double* ya, hipStream_t st);
 // y = A x with the streaming FP32 product on any CSR; sc[1] = x.y
-hipError_t spmv_stream_probe(int64_t nrows, const int64_t* rowp, const int32_t* col, const float* val, int64_t nnz, const int64_t* blk,
-                             int64_t nblk, const float* x, float* y, double* part, double* sc, hipStream_t st);
+hipError_t spmv_stream_probe(int64_t nrows, const int64_t* rowp, const int32_t* col, const float* val, int64_t nnz,
+                             int max_row, const int64_t* blk, int64_t nblk, const float* x, float* y, double* part, double* sc, hipStream_t st);
 
 hipError_t solve_system(const SolveSystem& s, const SolveParams& prm, SolveWork& w, SolveStats& out, hipStream_t st);
 

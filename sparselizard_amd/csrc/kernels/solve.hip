@@ -6,14 +6,15 @@
 // refinement (FP64 CSR residuals) around a Jacobi-preconditioned FP32
 // conjugate-gradient inner solve, for symmetric positive definite A.
 //
-// One inner iteration is three streaming kernels and two one-block sums:
+// One inner iteration is three kernels:
 //   K1  q = A p (FP32 values),             partials of p.q
-//   F   pq = ordered sum of the partials
 //   K2  d += a p, r -= a q, z = r / diag,  partials of r.z and r.r  (a = rz / pq)
-//   F   rz' and rr, beta = rz' / rz
-//   K3  p = z + beta p
-// Every reduction is deterministic: a fixed grid of partial sums, summed in a
-// fixed order by one block, and fixed lanes per row for the products.
+//   K3  p = z + beta p                     (beta = rz' / rz)
+// The partials are summed, in one order, by every block that needs the scalar
+// (at most SLX_SOLVE_BLOCKS values from the L2) instead of by one-block kernels
+// between them: at 16^3 x 6 P2 elasticity those took 10 of 44 us an iteration.
+// Every reduction is deterministic: a grid fixed by the system's sizes, partial
+// sums in a fixed order, and fixed lanes per row for the products.
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <cmath>
@@ -22,7 +23,7 @@
 
 namespace slx {
 
-enum { SC_RZ = 0, SC_PQ = 1, SC_RZN = 2, SC_RR = 3, SC_BETA = 4, SC_DOT = 5 };
+enum { SC_PQ = 1, SC_RR = 3, SC_DOT = 5 };
 
 // block sum of one double per thread (256 threads); result valid in thread 0
 __device__ inline double block_sum(double v, double* sh) {
@@ -34,6 +35,19 @@ __device__ inline double block_sum(double v, double* sh) {
     if (threadIdx.x == 0) s = (sh[0] + sh[1]) + (sh[2] + sh[3]);
     __syncthreads();
     return s;
+}
+
+// ordered sum of n partials, in every thread of a 256-thread block
+__device__ inline double all_sum(const double* __restrict__ part, int n, double* sh) {
+    double s = 0.0;
+    for (int i = threadIdx.x; i < n; i += 256) s += part[i];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+    __syncthreads();
+    const double t = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+    __syncthreads();
+    return t;
 }
 
 // y[r] = c0 f[r] - c1 (A x)[r] over one CSR matrix, LPR lanes per row (the
@@ -154,6 +168,99 @@ __global__ void __launch_bounds__(256) spmv_stream_f32(int64_t nblk, const int64
     if (threadIdx.x == 0) part[blockIdx.x] = t;
 }
 
+// q = A p over FP32 values, LPR lanes per row, U nonzeros of a lane in
+// flight at once (values and columns, then the eight gathers): the product of
+// the inner iterations for rows of ordinary length.  The streaming kernel
+// above waits for its row block's loads, the LDS exchange and the row sums in
+// turn: 26.9 us at 16^3 x 6 P2 elasticity (8.5e6 nonzeros, 81 a row), 23.9 us
+// here, bound by the L1's line accesses (1.3e7, most of them gathers of x).
+// Rows go to the XCDs in contiguous eighths, as above.
+template <int LPR, int U>
+__global__ void __launch_bounds__(512) spmv_rows_f32(int64_t nrows, const int64_t* __restrict__ rowp, const int32_t* __restrict__ col,
+                                                     const float* __restrict__ val, const float* __restrict__ x, float* __restrict__ y,
+                                                     double* __restrict__ part) {
+    constexpr int RPB = 512 / LPR;
+    __shared__ double sh[8];
+    const int l = threadIdx.x % LPR, g = threadIdx.x / LPR;
+    const int xcd = blockIdx.x % SLX_XCDS;
+    const int64_t nb = (nrows + RPB - 1) / RPB, b_end = nb * (xcd + 1) / SLX_XCDS;
+    double acc = 0.0;
+    for (int64_t b = nb * xcd / SLX_XCDS + blockIdx.x / SLX_XCDS; b < b_end; b += gridDim.x / SLX_XCDS) {
+        const int64_t r = b * RPB + g;
+        if (r < nrows) {
+            const int64_t k0 = rowp[r];
+            const int n = (int)(rowp[r + 1] - k0);
+            float s = 0.f;
+            for (int k = l; k < n; k += U * LPR) {
+                float v[U], xv[U];
+                int c[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int kk = k + u * LPR;
+                    const int64_t at = k0 + (kk < n ? kk : k);
+                    v[u] = kk < n ? val[at] : 0.f;
+                    c[u] = col[at];
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) xv[u] = x[c[u]];
+#pragma unroll
+                for (int u = 0; u < U; u++) s += v[u] * (k + u * LPR < n ? xv[u] : 0.f);
+            }
+#pragma unroll
+            for (int o = LPR / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, LPR);
+            if (l == 0) {
+                y[r] = s;
+                acc += (double)x[r] * (double)s;
+            }
+        }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0.0;
+#pragma unroll
+        for (int i = 0; i < 8; i++) t += sh[i];
+        part[blockIdx.x] = t;
+    }
+}
+
+// The FP32 product of the inner iterations: rows of at most SLX_ROWS_MAX
+// nonzeros on the row kernel, longer ones (a few lanes would walk them alone)
+// on the streaming kernel.  *npart: partial sums of x.y written.
+static hipError_t inner_product(int64_t nrows, int64_t nnz, int max_row, int64_t nblk, const int64_t* blk, const int64_t* rowp,
+                                const int32_t* col, const float* val, const float* x, float* y, double* part, int* npart, hipStream_t st) {
+    if (max_row > SLX_ROWS_MAX) {
+        *npart = SLX_SOLVE_BLOCKS;
+        hipLaunchKernelGGL(spmv_stream_f32, dim3(SLX_SOLVE_BLOCKS), dim3(256), 0, st, nblk, blk, rowp, col, val, nnz, x, y, part);
+        return hipGetLastError();
+    }
+    // the fewest lanes whose batches of six or eight hold the mean row
+    const int64_t avg = nrows ? (nnz + nrows - 1) / nrows : 1;
+    int lpr = 1;
+    while (lpr < 32 && lpr * 8 < avg) lpr *= 2;
+    const bool six = lpr * 6 >= avg;
+    const int64_t blocks = (nrows * lpr + 511) / 512;
+    const unsigned grid = (unsigned)std::min<int64_t>(SLX_SOLVE_BLOCKS, (blocks + SLX_XCDS - 1) / SLX_XCDS * SLX_XCDS);
+    *npart = (int)grid;
+#define SLX_ROWS_CASE(L)                                                                                                          \
+    case L:                                                                                                                       \
+        if (six) hipLaunchKernelGGL((spmv_rows_f32<L, 6>), dim3(grid), dim3(512), 0, st, nrows, rowp, col, val, x, y, part);      \
+        else hipLaunchKernelGGL((spmv_rows_f32<L, 8>), dim3(grid), dim3(512), 0, st, nrows, rowp, col, val, x, y, part);          \
+        break;
+    switch (lpr) {
+        SLX_ROWS_CASE(1)
+        SLX_ROWS_CASE(2)
+        SLX_ROWS_CASE(4)
+        SLX_ROWS_CASE(8)
+        SLX_ROWS_CASE(16)
+        SLX_ROWS_CASE(32)
+    }
+#undef SLX_ROWS_CASE
+    return hipGetLastError();
+}
+
 void stream_row_blocks(const int64_t* rowp, int64_t nrows, std::vector<int64_t>& out) {
     out.clear();
     out.push_back(0);
@@ -177,17 +284,24 @@ __global__ void scatter_kernel(int64_t n, const int64_t* __restrict__ idx, const
     if (i < n) dst[idx[i]] = src[i];
 }
 
-// Jacobi preconditioner (FP32) and the FP32 copy of the matrix values
-__global__ void prep_kernel(int64_t nrows, const int64_t* __restrict__ rowp, const int32_t* __restrict__ col, const double* __restrict__ val,
-                            float* __restrict__ val32, float* __restrict__ dinv) {
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// Jacobi preconditioner (FP32) and the FP32 copy of the matrix values, 16
+// lanes per row (one row per lane read the values a row apart: 0.29 ms
+// instead of 0.03 at 16^3 x 6 P2 elasticity)
+__global__ void __launch_bounds__(256) prep_kernel(int64_t nrows, const int64_t* __restrict__ rowp, const int32_t* __restrict__ col,
+                                                   const double* __restrict__ val, float* __restrict__ val32, float* __restrict__ dinv) {
+    const int64_t r = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / 16;
     if (r >= nrows) return;
+    const int l = threadIdx.x % 16;
     double d = 0.0;
-    for (int64_t k = rowp[r]; k < rowp[r + 1]; k++) {
-        val32[k] = (float)val[k];
-        if (col[k] == r) d = val[k];
+    for (int64_t k = rowp[r] + l; k < rowp[r + 1]; k += 16) {
+        const double v = val[k];
+        val32[k] = (float)v;
+        if (col[k] == r) d = v;
     }
-    dinv[r] = d != 0.0 ? (float)(1.0 / d) : 1.0f;
+    // the diagonal sits in one lane; the others hold zero
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) d += __shfl_xor(d, o, 16);
+    if (l == 0) dinv[r] = d != 0.0 ? (float)(1.0 / d) : 1.0f;
 }
 
 // partials of a.b (FP64 accumulation) over the fixed grid
@@ -200,31 +314,17 @@ __global__ void __launch_bounds__(256) dot_partial(int64_t n, const T* __restric
     if (threadIdx.x == 0) part[blockIdx.x] = t;
 }
 
-// sc[out0] (and sc[out1]) = ordered sums of one (two) partial arrays; mode 1
-// also sets beta = sc[SC_RZN] / sc[SC_RZ] and then sc[SC_RZ] = sc[SC_RZN]
-__global__ void __launch_bounds__(256) sum_partials(const double* __restrict__ part, int nsum, int out0, int out1, int mode,
-                                                    double* __restrict__ sc) {
+// sc[out] = ordered sum of n partials
+__global__ void __launch_bounds__(256) sum_partials(const double* __restrict__ part, int n, int out, double* __restrict__ sc) {
     __shared__ double sh[4];
-    double t[2] = {0.0, 0.0};
-    for (int j = 0; j < nsum; j++) {
-        double s = 0.0;
-        for (int i = threadIdx.x; i < SLX_SOLVE_BLOCKS; i += 256) s += part[j * SLX_SOLVE_BLOCKS + i];
-        t[j] = block_sum(s, sh);
-    }
-    if (threadIdx.x == 0) {
-        sc[out0] = t[0];
-        if (nsum > 1) sc[out1] = t[1];
-        if (mode == 1) {
-            sc[SC_BETA] = sc[SC_RZ] != 0.0 ? sc[SC_RZN] / sc[SC_RZ] : 0.0;
-            sc[SC_RZ] = sc[SC_RZN];
-        }
-    }
+    const double t = all_sum(part, n, sh);
+    if (threadIdx.x == 0) sc[out] = t;
 }
 
 // inner start: r32 = r, z = r / diag, p = z, d = 0; partials of r.z and r.r
 __global__ void __launch_bounds__(256) pcg_start(int64_t n, const double* __restrict__ r, const float* __restrict__ dinv,
                                                  float* __restrict__ r32, float* __restrict__ z, float* __restrict__ p,
-                                                 float* __restrict__ d, double* __restrict__ part) {
+                                                 float* __restrict__ d, double* __restrict__ prz, double* __restrict__ prr) {
     __shared__ double sh[4];
     double rz = 0.0, rr = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
@@ -240,17 +340,20 @@ __global__ void __launch_bounds__(256) pcg_start(int64_t n, const double* __rest
     const double a = block_sum(rz, sh);
     const double b = block_sum(rr, sh);
     if (threadIdx.x == 0) {
-        part[blockIdx.x] = a;
-        part[SLX_SOLVE_BLOCKS + blockIdx.x] = b;
+        prz[blockIdx.x] = a;
+        prr[blockIdx.x] = b;
     }
 }
 
-// d += a p ; r -= a q ; z = r / diag   (a = rz / pq); partials of r.z and r.r
-__global__ void __launch_bounds__(256) pcg_update(int64_t n, const double* __restrict__ sc, float* __restrict__ d, float* __restrict__ r,
-                                                  const float* __restrict__ p, const float* __restrict__ q, const float* __restrict__ dinv,
-                                                  float* __restrict__ z, double* __restrict__ part) {
+// d += a p ; r -= a q ; z = r / diag   (a = rz / pq, summed from their
+// partials); partials of the new r.z and r.r
+__global__ void __launch_bounds__(256) pcg_update(int64_t n, const double* __restrict__ ppq, int npq, const double* __restrict__ prz,
+                                                  int nrz, float* __restrict__ d, float* __restrict__ r, const float* __restrict__ p,
+                                                  const float* __restrict__ q, const float* __restrict__ dinv, float* __restrict__ z,
+                                                  double* __restrict__ prz_new, double* __restrict__ prr) {
     __shared__ double sh[4];
-    const float alpha = sc[SC_PQ] != 0.0 ? (float)(sc[SC_RZ] / sc[SC_PQ]) : 0.f;
+    const double pq = all_sum(ppq, npq, sh), rz0 = all_sum(prz, nrz, sh);
+    const float alpha = pq != 0.0 ? (float)(rz0 / pq) : 0.f;
     double rz = 0.0, rr = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
         d[i] += alpha * p[i];
@@ -264,15 +367,17 @@ __global__ void __launch_bounds__(256) pcg_update(int64_t n, const double* __res
     const double a = block_sum(rz, sh);
     const double b = block_sum(rr, sh);
     if (threadIdx.x == 0) {
-        part[blockIdx.x] = a;
-        part[SLX_SOLVE_BLOCKS + blockIdx.x] = b;
+        prz_new[blockIdx.x] = a;
+        prr[blockIdx.x] = b;
     }
 }
 
-// p = z + beta p
-__global__ void __launch_bounds__(256) pcg_direction(int64_t n, const double* __restrict__ sc, const float* __restrict__ z,
-                                                     float* __restrict__ p) {
-    const float beta = (float)sc[SC_BETA];
+// p = z + beta p   (beta = rz' / rz)
+__global__ void __launch_bounds__(256) pcg_direction(int64_t n, const double* __restrict__ prz_new, const double* __restrict__ prz, int nrz,
+                                                     const float* __restrict__ z, float* __restrict__ p) {
+    __shared__ double sh[4];
+    const double rzn = all_sum(prz_new, nrz, sh), rz = all_sum(prz, nrz, sh);
+    const float beta = rz != 0.0 ? (float)(rzn / rz) : 0.f;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) p[i] = z[i] + beta * p[i];
 }
 
@@ -290,47 +395,139 @@ static unsigned blocks(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 // ---- GMRES (FP32 vectors, FP64 sums) ----
 
-// z = dinv .* v
-__global__ void precond_kernel(int64_t n, const float* __restrict__ dinv, const float* __restrict__ v, float* __restrict__ z) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) z[i] = dinv[i] * v[i];
-}
+// One iteration is six kernels and no host work: q = A (dinv v_j), twice the
+// dots with the basis and the subtraction, then the norm, v_{j+1} and the
+// Givens rotations.  The host reads the residual history every
+// SLX_GMRES_CHECK iterations and drops the ones past convergence (columns of
+// H up to there do not depend on later ones).  Before, each iteration waited
+// for the host three times and the dots ran a 2048-block grid over one basis
+// vector after the other: 225 us an iteration at 4e3 rows, 30 us now.
 
-// dst = alpha * src
-__global__ void scale_kernel(int64_t n, float alpha, const float* __restrict__ src, float* __restrict__ dst) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = alpha * src[i];
-}
-
-// partials of V_i . w for i < nv (basis rows of length n)
-__global__ void __launch_bounds__(256) multi_dot_partial(int64_t n, const float* __restrict__ V, int nv, const float* __restrict__ w,
-                                                         double* __restrict__ part) {
+// partials of V_i . w: block (c, g) takes chunk c of the rows for the four
+// vectors 4 g .. 4 g + 3; part[i * gridDim.x + c]
+__global__ void __launch_bounds__(256) basis_dots(int64_t n, int64_t chunk, const float* __restrict__ V, int nv, const float* __restrict__ w,
+                                                  double* __restrict__ part) {
     __shared__ double sh[4];
-    for (int i = 0; i < nv; i++) {
-        const float* v = V + (size_t)i * n;
-        double s = 0.0;
-        for (int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x; k < n; k += (int64_t)gridDim.x * 256) s += (double)v[k] * (double)w[k];
-        const double t = block_sum(s, sh);
-        if (threadIdx.x == 0) part[(size_t)i * SLX_SOLVE_BLOCKS + blockIdx.x] = t;
+    const int i0 = 4 * blockIdx.y;
+    const int64_t k0 = blockIdx.x * chunk, k1 = min(n, k0 + chunk);
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+    const float* v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) v[u] = V + (size_t)min(i0 + u, nv - 1) * n;
+    for (int64_t k = k0 + threadIdx.x; k < k1; k += 256) {
+        const double wk = (double)w[k];
+#pragma unroll
+        for (int u = 0; u < 4; u++) s[u] += (double)v[u][k] * wk;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const double t = block_sum(s[u], sh);
+        if (threadIdx.x == 0 && i0 + u < nv) part[(size_t)(i0 + u) * gridDim.x + blockIdx.x] = t;
     }
 }
 
 // out[i] = ordered sum of partial row i (one block per row)
-__global__ void __launch_bounds__(256) sum_rows(const double* __restrict__ part, double* __restrict__ out) {
+__global__ void __launch_bounds__(256) sum_rows(const double* __restrict__ part, int n, double* __restrict__ out) {
     __shared__ double sh[4];
-    double s = 0.0;
-    for (int i = threadIdx.x; i < SLX_SOLVE_BLOCKS; i += 256) s += part[(size_t)blockIdx.x * SLX_SOLVE_BLOCKS + i];
-    const double t = block_sum(s, sh);
+    const double t = all_sum(part + (size_t)blockIdx.x * n, n, sh);
     if (threadIdx.x == 0) out[blockIdx.x] = t;
 }
 
-// w -= sum_i h_i V_i
-__global__ void basis_update(int64_t n, const float* __restrict__ V, int nv, const double* __restrict__ h, float* __restrict__ w) {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    float acc = w[k];
-    for (int i = 0; i < nv; i++) acc -= (float)h[i] * V[(size_t)i * n + k];
-    w[k] = acc;
+// w -= sum_i h_i V_i, h_i the ordered sum of its np partials; 64 rows per block
+// step, four groups of the vectors side by side.  Block 0 keeps h in hcol
+// (add: on top of the first pass's); partials of w.w
+__global__ void __launch_bounds__(256) basis_update(int64_t n, const float* __restrict__ V, int nv, const double* __restrict__ part, int np,
+                                                    int add, double* __restrict__ hcol, float* __restrict__ w, double* __restrict__ pnorm) {
+    __shared__ float h[SLX_GMRES_MAX + 4];
+    __shared__ float red[4][64];
+    __shared__ double sh[4];
+    const int t = threadIdx.x;
+    for (int i = t; i < nv; i += 256) {
+        double s = 0.0;
+        for (int c = 0; c < np; c++) s += part[(size_t)i * np + c];
+        h[i] = (float)s;
+        if (blockIdx.x == 0) hcol[i] = add ? hcol[i] + s : s;
+    }
+    __syncthreads();
+    const int l = t & 63, g = t >> 6, i0 = nv * g / 4, i1 = nv * (g + 1) / 4;
+    double nn = 0.0;
+    for (int64_t b = blockIdx.x; b * 64 < n; b += gridDim.x) {
+        const int64_t k = b * 64 + l;
+        float acc = 0.f;
+        if (k < n) {
+            int i = i0;
+            for (; i + 8 <= i1; i += 8) {
+                float v[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++) v[u] = V[(size_t)(i + u) * n + k];
+#pragma unroll
+                for (int u = 0; u < 8; u++) acc += h[i + u] * v[u];
+            }
+            for (; i < i1; i++) acc += h[i] * V[(size_t)i * n + k];
+        }
+        red[g][l] = acc;
+        __syncthreads();
+        if (g == 0 && k < n) {
+            const float wk = w[k] - ((red[0][l] + red[1][l]) + (red[2][l] + red[3][l]));
+            w[k] = wk;
+            nn += (double)wk * (double)wk;
+        }
+        __syncthreads();
+    }
+    const double s = block_sum(nn, sh);
+    if (t == 0) pnorm[blockIdx.x] = s;
+}
+
+// v = w / |w| (zero when w is), z = dinv .* v; with j >= 0 block 0 also rotates
+// column j of H (hcol: j + 1 entries, then |w|) and stores |g_{j+1}| and |w|
+__global__ void __launch_bounds__(256) basis_next(int64_t n, const double* __restrict__ pnorm, int np, const float* __restrict__ w,
+                                                  const float* __restrict__ dinv, float* __restrict__ v, float* __restrict__ z, int j,
+                                                  double* __restrict__ hcol, double* __restrict__ cs, double* __restrict__ sn,
+                                                  double* __restrict__ gv, double* __restrict__ hist) {
+    __shared__ double sh[4];
+    __shared__ double hl[SLX_GMRES_MAX + 1], cl[SLX_GMRES_MAX], sl[SLX_GMRES_MAX];
+    const double nrm = sqrt(all_sum(pnorm, np, sh));
+    const float inv = nrm > 0.0 ? (float)(1.0 / nrm) : 0.f;
+    for (int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x; k < n; k += (int64_t)gridDim.x * 256) {
+        const float x = inv * w[k];
+        v[k] = x;
+        z[k] = dinv[k] * x;
+    }
+    if (blockIdx.x != 0) return;
+    if (j < 0) {
+        if (threadIdx.x == 0) {
+            gv[0] = nrm;
+            hist[0] = nrm;
+        }
+        return;
+    }
+    for (int i = threadIdx.x; i <= j; i += 256) {
+        hl[i] = hcol[i];
+        if (i < j) {
+            cl[i] = cs[i];
+            sl[i] = sn[i];
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int i = 0; i < j; i++) {
+            const double a = hl[i], b = hl[i + 1];
+            hl[i] = cl[i] * a + sl[i] * b;
+            hl[i + 1] = -sl[i] * a + cl[i] * b;
+        }
+        const double a = hl[j], b = nrm, rr = hypot(a, b);
+        const double c = rr > 0.0 ? a / rr : 1.0, s = rr > 0.0 ? b / rr : 0.0;
+        hl[j] = rr;
+        cs[j] = c;
+        sn[j] = s;
+        const double g = gv[j];
+        gv[j + 1] = -s * g;
+        gv[j] = c * g;
+        hist[2 * j] = fabs(s * g);
+        hist[2 * j + 1] = nrm;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i <= j; i += 256) hcol[i] = hl[i];
 }
 
 // d = dinv .* sum_i y_i V_i   (right preconditioning)
@@ -375,9 +572,13 @@ __global__ void __launch_bounds__(256) sym_kernel(int64_t n, const int64_t* __re
         if (kt < 0) {
             bad = true;
         } else {
-            const int64_t kc = find_col(rowp, col, c, c);
-            const double dcc = kc >= 0 ? fabs(val[kc]) : 0.0;
-            bad = fabs(val[k] - val[kt]) > 1e-5 * (fabs(val[k]) + fabs(val[kt])) + 1e-6 * (drr + dcc);
+            // the partner's diagonal only where the rest of the bound does not settle it
+            const double diff = fabs(val[k] - val[kt]), lim = 1e-5 * (fabs(val[k]) + fabs(val[kt])) + 1e-6 * drr;
+            if (!(diff <= lim)) {
+                const int64_t kc = find_col(rowp, col, c, c);
+                const double dcc = kc >= 0 ? fabs(val[kc]) : 0.0;
+                bad = diff > 1e-5 * (fabs(val[k]) + fabs(val[kt])) + 1e-6 * (drr + dcc);
+            }
         }
     }
     if (bad) flag[0] = 1;
@@ -399,67 +600,65 @@ static hipError_t read_scalar(const double* dsc, int idx, double* h, hipStream_t
 // inner_tol of its start.  d = 0 when r32 = 0.
 static hipError_t gmres_cycle(const SolveSystem& s, const SolveParams& prm, SolveWork& w, int& iters, hipStream_t st) {
     const int64_t n = s.nfree;
-    const unsigned G = SLX_SOLVE_BLOCKS;
     const int m = std::max(1, std::min(prm.restart, prm.max_inner));
-    double beta2 = 0.0;
-    hipLaunchKernelGGL((dot_partial<float>), dim3(G), dim3(256), 0, st, n, w.r32, w.r32, w.part);
-    hipLaunchKernelGGL(sum_partials, dim3(1), dim3(256), 0, st, w.part, 1, (int)SC_DOT, 0, 0, w.sc);
-    HIPERR(read_scalar(w.sc, SC_DOT, &beta2, st));
-    const double beta = sqrt(beta2);
+    // mpart: the dots' partials, then the column store [m][m + 1], cs, sn, g and the history
+    // (up to eight partials of a dot are summed by the kernel that needs it)
+    const int nchunk = n <= 32768 ? (int)std::min<int64_t>(8, (n + 1023) / 1024) : (int)std::min<int64_t>(SLX_SOLVE_BLOCKS, (n + 4095) / 4096);
+    const int64_t chunk = (n + nchunk - 1) / nchunk;
+    double* part = w.mpart;
+    double* H = part + (size_t)(m + 1) * SLX_SOLVE_BLOCKS;
+    double* cs = w.mpart + (size_t)(m + 1) * 2 * SLX_SOLVE_BLOCKS - 5 * (m + 1);
+    double *sn = cs + m, *gv = sn + m, *hist = gv + m + 1;
+    const unsigned gu = (unsigned)std::min<int64_t>(SLX_SOLVE_BLOCKS, (n + 63) / 64);
+    const unsigned gn = (unsigned)std::min<int64_t>(SLX_SOLVE_BLOCKS, (n + 255) / 256);
+    const unsigned gd = (unsigned)std::min<int64_t>(SLX_SOLVE_BLOCKS, (n + 255) / 256);
+    double beta = 0.0;
+    hipLaunchKernelGGL((dot_partial<float>), dim3(gd), dim3(256), 0, st, n, w.r32, w.r32, w.part);
+    hipLaunchKernelGGL(basis_next, dim3(gn), dim3(256), 0, st, n, w.part, (int)gd, w.r32, w.dinv, w.V, w.z, -1, H, cs, sn, gv, hist);
+    HIPERR(read_scalar(hist, 0, &beta, st));
     if (!(beta > 0.0)) {
         HIPERR(hipMemsetAsync(w.d, 0, n * sizeof(float), st));
         return hipSuccess;
     }
-    hipLaunchKernelGGL(scale_kernel, dim3(blocks(n)), dim3(256), 0, st, n, (float)(1.0 / beta), w.r32, w.V);
-    std::vector<double> H((size_t)(m + 1) * m, 0.0), cs(m, 0.0), sn(m, 0.0), g(m + 1, 0.0), hc(m + 1);
-    g[0] = beta;
+    std::vector<double> hh(2 * (size_t)m);
     int k = 0;
-    for (int j = 0; j < m; j++) {
-        const float* vj = w.V + (size_t)j * n;
-        hipLaunchKernelGGL(precond_kernel, dim3(blocks(n)), dim3(256), 0, st, n, w.dinv, vj, w.z);
-        hipLaunchKernelGGL(spmv_stream_f32, dim3(G), dim3(256), 0, st, s.nblk, s.Ablk, s.Arow, s.Acol, w.val32, s.nnzA, w.z, w.q,
-                           w.part);
+    for (int j = 0; j < m && k == 0; j++) {
+        int npart = 0;
+        HIPERR(inner_product(n, s.nnzA, s.max_row, s.nblk, s.Ablk, s.Arow, s.Acol, w.val32, w.z, w.q, w.part, &npart, st));
+        double* hcol = H + (size_t)j * (m + 1);
         // two passes of classical Gram-Schmidt against v_0 .. v_j
         for (int pass = 0; pass < 2; pass++) {
-            hipLaunchKernelGGL(multi_dot_partial, dim3(G), dim3(256), 0, st, n, w.V, j + 1, w.q, w.mpart);
-            hipLaunchKernelGGL(sum_rows, dim3(j + 1), dim3(256), 0, st, w.mpart, w.hv);
-            hipLaunchKernelGGL(basis_update, dim3(blocks(n)), dim3(256), 0, st, n, w.V, j + 1, w.hv, w.q);
-            HIPERR(hipMemcpyAsync(hc.data(), w.hv, (size_t)(j + 1) * sizeof(double), hipMemcpyDeviceToHost, st));
+            hipLaunchKernelGGL(basis_dots, dim3(nchunk, (j + 4) / 4), dim3(256), 0, st, n, chunk, w.V, j + 1, w.q, part);
+            const double* src = part;
+            int np = nchunk;
+            if (nchunk > 8) {
+                hipLaunchKernelGGL(sum_rows, dim3(j + 1), dim3(256), 0, st, part, nchunk, w.hv);
+                src = w.hv;
+                np = 1;
+            }
+            hipLaunchKernelGGL(basis_update, dim3(gu), dim3(256), 0, st, n, w.V, j + 1, src, np, pass, hcol, w.q, w.part);
+        }
+        hipLaunchKernelGGL(basis_next, dim3(gn), dim3(256), 0, st, n, w.part, (int)gu, w.q, w.dinv, w.V + (size_t)(j + 1) * n, w.z, j, hcol,
+                           cs, sn, gv, hist);
+        if ((j + 1) % SLX_GMRES_CHECK == 0 || j + 1 == m) {
+            HIPERR(hipMemcpyAsync(hh.data(), hist, 2 * (size_t)(j + 1) * sizeof(double), hipMemcpyDeviceToHost, st));
             HIPERR(hipStreamSynchronize(st));
-            for (int i = 0; i <= j; i++) H[(size_t)i * m + j] += hc[i];
+            for (int i = j + 1 - std::min(j + 1, SLX_GMRES_CHECK); i <= j && k == 0; i++)
+                if (hh[2 * i] <= prm.inner_tol * beta || !(hh[2 * i + 1] > 0.0)) k = i + 1;
+            if (j + 1 == m && k == 0) k = m;
         }
-        double hn2 = 0.0;
-        hipLaunchKernelGGL((dot_partial<float>), dim3(G), dim3(256), 0, st, n, w.q, w.q, w.part);
-        hipLaunchKernelGGL(sum_partials, dim3(1), dim3(256), 0, st, w.part, 1, (int)SC_DOT, 0, 0, w.sc);
-        HIPERR(read_scalar(w.sc, SC_DOT, &hn2, st));
-        const double hn = sqrt(hn2);
-        H[(size_t)(j + 1) * m + j] = hn;
-        if (hn > 0.0 && j + 1 <= m)
-            hipLaunchKernelGGL(scale_kernel, dim3(blocks(n)), dim3(256), 0, st, n, (float)(1.0 / hn), w.q, w.V + (size_t)(j + 1) * n);
-        // Givens rotations of column j
-        for (int i = 0; i < j; i++) {
-            const double a = H[(size_t)i * m + j], b = H[(size_t)(i + 1) * m + j];
-            H[(size_t)i * m + j] = cs[i] * a + sn[i] * b;
-            H[(size_t)(i + 1) * m + j] = -sn[i] * a + cs[i] * b;
-        }
-        const double a = H[(size_t)j * m + j], b = H[(size_t)(j + 1) * m + j];
-        const double rr = std::hypot(a, b);
-        cs[j] = rr > 0.0 ? a / rr : 1.0;
-        sn[j] = rr > 0.0 ? b / rr : 0.0;
-        H[(size_t)j * m + j] = rr;
-        H[(size_t)(j + 1) * m + j] = 0.0;
-        g[j + 1] = -sn[j] * g[j];
-        g[j] = cs[j] * g[j];
-        k = j + 1;
-        iters++;
-        if (fabs(g[j + 1]) <= prm.inner_tol * beta || !(hn > 0.0)) break;
     }
+    iters += k;
     // y = H(0:k, 0:k)^-1 g(0:k)
-    std::vector<double> y(k, 0.0);
+    std::vector<double> R((size_t)k * (m + 1)), g(k), y(k, 0.0);
+    HIPERR(hipMemcpyAsync(R.data(), H, R.size() * sizeof(double), hipMemcpyDeviceToHost, st));
+    HIPERR(hipMemcpyAsync(g.data(), gv, (size_t)k * sizeof(double), hipMemcpyDeviceToHost, st));
+    HIPERR(hipStreamSynchronize(st));
     for (int i = k - 1; i >= 0; i--) {
         double t = g[i];
-        for (int c = i + 1; c < k; c++) t -= H[(size_t)i * m + c] * y[c];
-        y[i] = H[(size_t)i * m + i] != 0.0 ? t / H[(size_t)i * m + i] : 0.0;
+        for (int c = i + 1; c < k; c++) t -= R[(size_t)c * (m + 1) + i] * y[c];
+        const double d = R[(size_t)i * (m + 1) + i];
+        y[i] = d != 0.0 ? t / d : 0.0;
     }
     HIPERR(hipMemcpyAsync(w.hv, y.data(), (size_t)k * sizeof(double), hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(basis_combine, dim3(blocks(n)), dim3(256), 0, st, n, w.V, k, w.hv, w.dinv, w.d);
@@ -496,10 +695,11 @@ hipError_t matvec_system(const SolveSystem& s, const double* x, double* y, doubl
     return hipGetLastError();
 }
 
-hipError_t spmv_stream_probe(int64_t nrows, const int64_t* rowp, const int32_t* col, const float* val, int64_t nnz, const int64_t* blk,
-                             int64_t nblk, const float* x, float* y, double* part, double* sc, hipStream_t st) {
-    hipLaunchKernelGGL(spmv_stream_f32, dim3(SLX_SOLVE_BLOCKS), dim3(256), 0, st, nblk, blk, rowp, col, val, nnz, x, y, part);
-    hipLaunchKernelGGL(sum_partials, dim3(1), dim3(256), 0, st, part, 1, (int)SC_PQ, 0, 0, sc);
+hipError_t spmv_stream_probe(int64_t nrows, const int64_t* rowp, const int32_t* col, const float* val, int64_t nnz, int max_row,
+                             const int64_t* blk, int64_t nblk, const float* x, float* y, double* part, double* sc, hipStream_t st) {
+    int npart = 0;
+    HIPERR(inner_product(nrows, nnz, max_row, nblk, blk, rowp, col, val, x, y, part, &npart, st));
+    hipLaunchKernelGGL(sum_partials, dim3(1), dim3(256), 0, st, part, npart, (int)SC_PQ, sc);
     return hipGetLastError();
 }
 
@@ -507,18 +707,20 @@ hipError_t solve_system(const SolveSystem& s, const SolveParams& prm, SolveWork&
     const int64_t n = s.nfree;
     out = SolveStats{};
     if (n == 0) return hipSuccess;
-    const unsigned G = SLX_SOLVE_BLOCKS;
+    // at most SLX_SOLVE_BLOCKS blocks (every block of the next kernel sums their partials)
+    const unsigned G = (unsigned)std::min<int64_t>(SLX_SOLVE_BLOCKS, (n + 255) / 256);
+    double *ppq = w.part, *prz = ppq + SLX_SOLVE_BLOCKS, *prz_new = prz + SLX_SOLVE_BLOCKS, *prr = prz_new + SLX_SOLVE_BLOCKS;
     // f = b_A - D x_D ; x_D = Dirichlet values from the rhs
     hipLaunchKernelGGL(gather_kernel, dim3(blocks(n)), dim3(256), 0, st, n, s.free_dofs, s.rhs, w.f);
     if (s.ncons > 0) {
         hipLaunchKernelGGL(gather_kernel, dim3(blocks(s.ncons)), dim3(256), 0, st, s.ncons, s.cons_dofs, s.rhs, w.xd);
         spmv<double, double, double>(n, s.nnzD, s.Drow, s.Dcol, s.Dval, w.xd, w.f, 1.0, 1.0, w.f, nullptr, st);
     }
-    hipLaunchKernelGGL(prep_kernel, dim3(blocks(n)), dim3(256), 0, st, n, s.Arow, s.Acol, s.Aval, w.val32, w.dinv);
+    hipLaunchKernelGGL(prep_kernel, dim3(blocks(16 * n)), dim3(256), 0, st, n, s.Arow, s.Acol, s.Aval, w.val32, w.dinv);
     HIPERR(hipMemsetAsync(w.x, 0, n * sizeof(double), st));
     double h = 0.0;
     hipLaunchKernelGGL((dot_partial<double>), dim3(G), dim3(256), 0, st, n, w.f, w.f, w.part);
-    hipLaunchKernelGGL(sum_partials, dim3(1), dim3(256), 0, st, w.part, 1, (int)SC_DOT, 0, 0, w.sc);
+    hipLaunchKernelGGL(sum_partials, dim3(1), dim3(256), 0, st, w.part, (int)G, (int)SC_DOT, w.sc);
     HIPERR(read_scalar(w.sc, SC_DOT, &h, st));
     const double fnorm = sqrt(h);
     // r = f (x = 0)
@@ -532,29 +734,29 @@ hipError_t solve_system(const SolveSystem& s, const SolveParams& prm, SolveWork&
             HIPERR(gmres_cycle(s, prm, w, out.inner, st));
         } else {
         // inner FP32 PCG on A d = r
-        hipLaunchKernelGGL(pcg_start, dim3(G), dim3(256), 0, st, n, w.r, w.dinv, w.r32, w.z, w.p, w.d, w.part);
-        hipLaunchKernelGGL(sum_partials, dim3(1), dim3(256), 0, st, w.part, 2, (int)SC_RZ, (int)SC_RR, 0, w.sc);
+        hipLaunchKernelGGL(pcg_start, dim3(G), dim3(256), 0, st, n, w.r, w.dinv, w.r32, w.z, w.p, w.d, prz, prr);
+        hipLaunchKernelGGL(sum_partials, dim3(1), dim3(256), 0, st, prr, (int)G, (int)SC_RR, w.sc);
         HIPERR(read_scalar(w.sc, SC_RR, &h, st));
         const double r0 = sqrt(h);
         for (int k = 0; k < prm.max_inner; k++) {
-            hipLaunchKernelGGL(spmv_stream_f32, dim3(G), dim3(256), 0, st, s.nblk, s.Ablk, s.Arow, s.Acol, w.val32, s.nnzA, w.p, w.q,
-                               w.part);
-            hipLaunchKernelGGL(sum_partials, dim3(1), dim3(256), 0, st, w.part, 1, (int)SC_PQ, 0, 0, w.sc);
-            hipLaunchKernelGGL(pcg_update, dim3(G), dim3(256), 0, st, n, w.sc, w.d, w.r32, w.p, w.q, w.dinv, w.z, w.part);
-            hipLaunchKernelGGL(sum_partials, dim3(1), dim3(256), 0, st, w.part, 2, (int)SC_RZN, (int)SC_RR, 1, w.sc);
+            int npq = 0;
+            HIPERR(inner_product(n, s.nnzA, s.max_row, s.nblk, s.Ablk, s.Arow, s.Acol, w.val32, w.p, w.q, ppq, &npq, st));
+            hipLaunchKernelGGL(pcg_update, dim3(G), dim3(256), 0, st, n, ppq, npq, prz, (int)G, w.d, w.r32, w.p, w.q, w.dinv, w.z, prz_new, prr);
             out.inner++;
             if ((k + 1) % 8 == 0 || k + 1 == prm.max_inner) {
+                hipLaunchKernelGGL(sum_partials, dim3(1), dim3(256), 0, st, prr, (int)G, (int)SC_RR, w.sc);
                 HIPERR(read_scalar(w.sc, SC_RR, &h, st));
                 if (sqrt(h) <= prm.inner_tol * r0) break;
             }
-            hipLaunchKernelGGL(pcg_direction, dim3(G), dim3(256), 0, st, n, w.sc, w.z, w.p);
+            hipLaunchKernelGGL(pcg_direction, dim3(G), dim3(256), 0, st, n, prz_new, prz, (int)G, w.z, w.p);
+            std::swap(prz, prz_new);
         }
         }
         hipLaunchKernelGGL(add_f32_to_f64, dim3(blocks(n)), dim3(256), 0, st, n, w.d, w.x);
         // FP64 residual r = f - A x
         spmv<double, double, double>(n, s.nnzA, s.Arow, s.Acol, s.Aval, w.x, w.f, 1.0, 1.0, w.r, nullptr, st);
         hipLaunchKernelGGL((dot_partial<double>), dim3(G), dim3(256), 0, st, n, w.r, w.r, w.part);
-        hipLaunchKernelGGL(sum_partials, dim3(1), dim3(256), 0, st, w.part, 1, (int)SC_DOT, 0, 0, w.sc);
+        hipLaunchKernelGGL(sum_partials, dim3(1), dim3(256), 0, st, w.part, (int)G, (int)SC_DOT, w.sc);
         HIPERR(read_scalar(w.sc, SC_DOT, &h, st));
         rnorm = sqrt(h);
     }

@@ -185,6 +185,11 @@ struct slx_plan_s {
     double symbolic_seconds = 0.0;
     bool signed_slots = false;     // folded orientations: signed segment entries
 
+    // the solve's workspace, kept between calls up to SLX_SOLVE_KEEP bytes (a call
+    // that finds it in use, or needs more, allocates its own)
+    DBuf solve_ws;
+    std::mutex solve_mu;
+
     hipGraphExec_t graph_exec = nullptr;  // captured numeric phase (slx_plan_graph_capture)
     // right-hand-side-only buckets run, with the rhs reduction, on a side
     // stream forked from and joined back into the caller's stream; they keep
@@ -2482,7 +2487,7 @@ SolveSystem solve_view(slx_plan p) {
     return SolveSystem{p->n_dofs, p->nfree, p->ncons, p->nnzA, p->nnzD, p->d_Arow.as<int64_t>(), p->d_Drow.as<int64_t>(),
                        p->d_Acol.as<int32_t>(), p->d_Dcol.as<int32_t>(), p->d_Aval.as<double>(), p->d_Dval.as<double>(),
                        p->d_rhs.as<double>(), p->d_free.as<int64_t>(), p->d_cons.as<int64_t>(), p->d_ablk.as<int64_t>(),
-                       p->n_ablk};
+                       p->n_ablk, p->rd.max_row_len};
 }
 
 void check_assembled(slx_plan p) {
@@ -2535,6 +2540,7 @@ slx_status slx_plan_matvec(slx_plan p, const double* x, double* y) {
 namespace {
 // Device workspace of one solve, in bytes: a 256-byte header (the symmetry
 // check's flag), then the doubles, then the floats (16-byte aligned).
+#define SLX_SOLVE_KEEP ((size_t)256 << 20)
 struct SolveLayout {
     int64_t nD, nF, nV;
     size_t bytes;
@@ -2542,8 +2548,8 @@ struct SolveLayout {
 SolveLayout solve_layout(slx_plan p, bool gm, int restart) {
     const int64_t nf = p->nfree, nc = p->ncons, nd = p->n_dofs;
     SolveLayout L;
-    const int64_t nDg = gm ? (int64_t)(restart + 1) * (SLX_SOLVE_BLOCKS + 1) : 0;
-    L.nD = 3 * nf + nc + nd + 2 * SLX_SOLVE_BLOCKS + 8 + nDg;
+    const int64_t nDg = gm ? (int64_t)(restart + 1) * (SLX_SOLVE_PART + 1) : 0;
+    L.nD = 3 * nf + nc + nd + 2 * SLX_SOLVE_PART + 8 + nDg;
     L.nF = 6 * nf + p->nnzA + 4;
     L.nV = gm ? (int64_t)(restart + 1) * nf : 0;
     L.bytes = 256 + (size_t)L.nD * sizeof(double) + (size_t)(L.nF + L.nV) * sizeof(float) + 64;
@@ -2579,17 +2585,22 @@ void solve_on(slx_plan p, int32_t method, double rel_tol, int32_t max_outer, int
     }
     const SolveSystem sys = solve_view(p);
     DBuf own;
+    std::unique_lock<std::mutex> keep(p->solve_mu, std::defer_lock);
+    if (!ws) (void)keep.try_lock();
+    auto workspace = [&](size_t bytes) {
+        DBuf& b = keep.owns_lock() && bytes <= SLX_SOLVE_KEEP ? p->solve_ws : own;
+        if (b.n < bytes) b.alloc(bytes);
+        return b.as<unsigned char>();
+    };
     const int restart = std::min<int>(max_inner, SLX_GMRES_MAX);
     if (method == SLX_SOLVE_AUTO) {
-        // the check's flag: the first word of the workspace (or of a small
-        // allocation of its own when the solve allocates)
+        // the check's flag: the first word of the workspace
         int* flag = nullptr;
         if (ws) {
             SLX_CHECK(ws_bytes >= 256, "solve: workspace smaller than its header");
             flag = static_cast<int*>(ws);
         } else {
-            own.alloc(256);
-            flag = own.as<int>();
+            flag = (int*)workspace(solve_layout(p, false, restart).bytes);
         }
         int nonsym = 0;
         HIPCHECK(check_symmetric(sys, flag, &nonsym, p->stream));
@@ -2603,8 +2614,7 @@ void solve_on(slx_plan p, int32_t method, double rel_tol, int32_t max_outer, int
                                           << p->nnzA << " nonzeros" << (gm ? ", GMRES basis" : "") << ") exceeds the "
                                           << ws_bytes << " bytes available");
     } else {
-        own.alloc(L.bytes);
-        base = own.as<unsigned char>();
+        base = workspace(L.bytes);
     }
     SolveWork w;
     double* dp = reinterpret_cast<double*>(base + 256);
@@ -2613,9 +2623,9 @@ void solve_on(slx_plan p, int32_t method, double rel_tol, int32_t max_outer, int
     w.x = dp; dp += nf;
     w.xd = dp; dp += p->ncons;
     w.xfull = dp; dp += nd;
-    w.part = dp; dp += 2 * SLX_SOLVE_BLOCKS;
+    w.part = dp; dp += 2 * SLX_SOLVE_PART;
     w.sc = dp; dp += 8;
-    w.mpart = gm ? dp : nullptr; dp += gm ? (int64_t)(restart + 1) * SLX_SOLVE_BLOCKS : 0;
+    w.mpart = gm ? dp : nullptr; dp += gm ? (int64_t)(restart + 1) * SLX_SOLVE_PART : 0;
     w.hv = gm ? dp : nullptr; dp += gm ? restart + 1 : 0;
     float* fp = (float*)dp;
     w.r32 = fp; fp += nf;
@@ -2911,7 +2921,10 @@ slx_status slx_selftest_spmv_stream(slx_ctx ctx, int64_t nrows, const int64_t* r
         upload(dx, x32.data(), nrows, ctx->stream);
         dy.alloc(nrows * sizeof(float));
         dpart.alloc((SLX_SOLVE_BLOCKS + 8) * sizeof(double));
-        HIPCHECK(spmv_stream_probe(nrows, drow.as<int64_t>(), dcol.as<int32_t>(), dval.as<float>(), nnz, dblk.as<int64_t>(),
+        int64_t max_row = 0;
+        for (int64_t r = 0; r < nrows; r++) max_row = std::max(max_row, rowp[r + 1] - rowp[r]);
+        HIPCHECK(spmv_stream_probe(nrows, drow.as<int64_t>(), dcol.as<int32_t>(), dval.as<float>(), nnz,
+                                   (int)std::min<int64_t>(max_row, INT32_MAX), dblk.as<int64_t>(),
                                    (int64_t)blk.size() - 1, dx.as<float>(), dy.as<float>(), dpart.as<double>(),
                                    dpart.as<double>() + SLX_SOLVE_BLOCKS, ctx->stream));
         HIPCHECK(hipStreamSynchronize(ctx->stream));
