@@ -31,7 +31,7 @@ std::map<std::string, hipFunction_t> g_cache;  // key: device id + source
 }  // namespace
 
 std::string coef_kernel_source(const slx_instr* prog, int n, bool fp64, bool runs, const std::vector<int>& field_nff,
-                               const CoefPack& pack) {
+                               const CoefPack& pack, bool several) {
     std::ostringstream o;
     // fields whose values a thread gathers once per element (runs of Gauss
     // points, at most SLX_JIT_GATHER_NFF form functions)
@@ -52,7 +52,12 @@ std::string coef_kernel_source(const slx_instr* prog, int n, bool fp64, bool run
     // consecutive elements at the same points, each thread loads its element's
     // nodes once and walks its qc points.  Without runs (one point per element
     // or per thread): the (element, Gauss point) of the thread, qc unused.
-    o << "extern \"C\" __global__ void __launch_bounds__(256) slx_coef(DevBucket b, DevInputs in, int nq, int qfast, int qc, T* __restrict__ ctab) {\n";
+    // several: blockIdx.y names the bucket; a single one comes by value
+    o << "extern \"C\" __global__ void __launch_bounds__(256) slx_coef(" << (several ? "const DevJob* __restrict__ jobs" : "DevJob job")
+      << ", DevInputs in, int nq, int qfast, int qc, unsigned char* __restrict__ cbase) {\n"
+      << (several ? "    const DevJob& job = jobs[blockIdx.y];\n" : "")
+      << "    const DevBucket& b = job.b;\n"
+         "    T* ctab = (T*)(cbase + job.coff);\n";
     if (runs)
         o << "    const int nch = qfast ? nq : (nq + qc - 1) / qc;\n"
              "    const int64_t total = (int64_t)b.n_elem * nch;\n"
@@ -109,7 +114,7 @@ std::string coef_kernel_source(const slx_instr* prog, int n, bool fp64, bool run
         switch (x.op) {
             case SLX_OP_CONST: rhs = "(T)in.consts[" + std::to_string(x.imm) + "]"; break;
             case SLX_OP_PARAM:
-                rhs = "(T)in.params[(size_t)" + std::to_string(x.imm) + " * in.param_len + b.elem_ids[e]]";
+                rhs = "(T)in.params[(size_t)" + std::to_string(x.imm) + " * in.param_len + ((const SLX_GLOBAL int*)b.elem_ids)[e]]";
                 break;
             case SLX_OP_JAC: rhs = "(T)g.J[" + std::to_string(3 * x.a + x.b) + "]"; break;
             case SLX_OP_INVJAC: rhs = "(T)g.inv[" + std::to_string(3 * x.a + x.b) + "]"; break;
@@ -117,8 +122,8 @@ std::string coef_kernel_source(const slx_instr* prog, int n, bool fp64, bool run
             case SLX_OP_COORD:
                 o << "        T " << v << ";\n        {\n            double s = 0.0;\n"
                   << "            for (int k = 0; k < b.n_geo; k++) {\n"
-                  << "                const int node = b.geo_nodes[(size_t)e * b.n_geo + k];\n"
-                  << "                s += in.xyz[3 * (size_t)node + " << x.a << "] * b.geo_tab[(size_t)k * b.n_gp + q];\n"
+                  << "                const int node = ((const SLX_GLOBAL int*)b.geo_nodes)[(size_t)e * b.n_geo + k];\n"
+                  << "                s += in.xyz[3 * (size_t)node + " << x.a << "] * ((const SLX_CONST double*)b.geo_tab)[(size_t)k * b.n_gp + q];\n"
                   << "            }\n            " << v << " = (T)s;\n        }\n";
                 cur[x.dst] = v;
                 continue;
@@ -149,14 +154,14 @@ std::string coef_kernel_source(const slx_instr* prog, int n, bool fp64, bool run
 }
 
 bool coef_compile(const slx_instr* prog, int n_instr, bool fp64, bool runs, const std::vector<int>& field_nff, hipFunction_t* fn,
-                  std::string* err, const CoefPack& pack) {
+                  std::string* err, const CoefPack& pack, bool several) {
     *fn = nullptr;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) {
         if (err) *err = "no current device";
         return false;
     }
-    const std::string src = coef_kernel_source(prog, n_instr, fp64, runs, field_nff, pack);
+    const std::string src = coef_kernel_source(prog, n_instr, fp64, runs, field_nff, pack, several);
     const std::string key = std::to_string(dev) + "\n" + src;
     {
         std::lock_guard<std::mutex> lk(g_mu);
@@ -212,21 +217,22 @@ bool coef_compile(const slx_instr* prog, int n_instr, bool fp64, bool runs, cons
     return true;
 }
 
-hipError_t coef_launch(hipFunction_t fn, const DevBucket& b, const DevInputs& in, int nq, int qfast, void* ctab, hipStream_t st) {
-    const int64_t pairs = (int64_t)b.n_elem * nq;
+hipError_t coef_launch(hipFunction_t fn, const DevBucket& b, int64_t coff, const DevJob* jobs, int n_jobs, int max_elem, const DevInputs& in, int nq,
+                       int qfast, void* cbase, hipStream_t st) {
+    const int64_t pairs = (int64_t)max_elem * nq;
     if (pairs == 0 || b.n_coefs == 0) return hipSuccess;
     // element-fastest layout: runs of qc points per thread, as long as about
     // 256K threads remain to fill the GPU
     // (a kernel compiled without runs has nq = 1 here, so qc = 1 and the grid
     // is one thread per element)
     int qc = 1;
-    if (!qfast) qc = (int)std::max<int64_t>(1, std::min<int64_t>(nq, pairs / (256 * 1024)));
+    if (!qfast) qc = (int)std::max<int64_t>(1, std::min<int64_t>(nq, pairs * n_jobs / (256 * 1024)));
     const int64_t nch = qfast ? nq : (nq + qc - 1) / qc;
-    const int64_t total = (int64_t)b.n_elem * nch;
-    DevBucket bb = b;
+    const int64_t total = (int64_t)max_elem * nch;
     DevInputs ii = in;
-    void* args[] = {&bb, &ii, &nq, &qfast, &qc, &ctab};
-    return hipModuleLaunchKernel(fn, (unsigned)((total + 255) / 256), 1, 1, 256, 1, 1, 0, st, args, nullptr);
+    DevJob job{b, coff};
+    void* args[] = {n_jobs > 1 ? (void*)&jobs : (void*)&job, &ii, &nq, &qfast, &qc, &cbase};
+    return hipModuleLaunchKernel(fn, (unsigned)((total + 255) / 256), (unsigned)n_jobs, 1, 256, 1, 1, 0, st, args, nullptr);
 }
 
 }  // namespace slx

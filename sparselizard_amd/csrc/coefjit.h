@@ -27,14 +27,16 @@ struct CoefPack {
 // SLX_JIT_GATHER_NFF form functions (field_nff[f] in this bucket) once for
 // the run; otherwise one thread per (element, Gauss point).  With a pack
 // (coefficients constant over the Gauss points) the kernel writes records.
+// several: the kernel of a launch over several buckets.
 std::string coef_kernel_source(const slx_instr* prog, int n_instr, bool fp64, bool runs, const std::vector<int>& field_nff,
-                               const CoefPack& pack = CoefPack());
+                               const CoefPack& pack = CoefPack(), bool several = false);
 // Compiles (or finds in the process-wide cache) the kernel of one program for
 // the current device; fp64 selects FP64 coefficients.  On failure returns
 // false with the compiler log in *err.
 bool coef_compile(const slx_instr* prog, int n_instr, bool fp64, bool runs, const std::vector<int>& field_nff, hipFunction_t* fn,
-                  std::string* err, const CoefPack& pack = CoefPack());
+                  std::string* err, const CoefPack& pack = CoefPack(), bool several = false);
 // Same launch contract as the interpreter's coefficient kernel.
-hipError_t coef_launch(hipFunction_t fn, const DevBucket& b, const DevInputs& in, int nq, int qfast, void* ctab, hipStream_t st);
+hipError_t coef_launch(hipFunction_t fn, const DevBucket& b, int64_t coff, const DevJob* jobs, int n_jobs, int max_elem, const DevInputs& in, int nq,
+                       int qfast, void* cbase, hipStream_t st);
 
 }  // namespace slx

@@ -56,7 +56,7 @@ __device__ void run_program(const DevBucket& b, const DevInputs& in, const int (
             }
             case SLX_OP_PARAM:
 #pragma unroll
-                for (int v = 0; v < V; v++) r[v] = (T)in.params[(size_t)ins.imm * in.param_len + b.elem_ids[e[v]]];
+                for (int v = 0; v < V; v++) r[v] = (T)in.params[(size_t)ins.imm * in.param_len + ((const SLX_GLOBAL int*)b.elem_ids)[e[v]]];
                 break;
             case SLX_OP_JAC:
 #pragma unroll
@@ -75,8 +75,8 @@ __device__ void run_program(const DevBucket& b, const DevInputs& in, const int (
                 for (int v = 0; v < V; v++) {
                     double s = 0.0;
                     for (int k = 0; k < b.n_geo; k++) {
-                        const int node = b.geo_nodes[(size_t)e[v] * b.n_geo + k];
-                        s += in.xyz[3 * (size_t)node + ins.a] * b.geo_tab[(size_t)k * b.n_gp + q[v]];
+                        const int node = ((const SLX_GLOBAL int*)b.geo_nodes)[(size_t)e[v] * b.n_geo + k];
+                        s += in.xyz[3 * (size_t)node + ins.a] * ((const SLX_CONST double*)b.geo_tab)[(size_t)k * b.n_gp + q[v]];
                     }
                     r[v] = (T)s;
                 }
@@ -125,7 +125,10 @@ __device__ void run_program(const DevBucket& b, const DevInputs& in, const int (
 // over the Gauss points); each thread takes V consecutive (element, Gauss
 // point) pairs, element fastest.
 template <typename T, int V>
-__global__ void __launch_bounds__(256) coef_kernel(DevBucket b, DevInputs in, int nq, int qfast, DevPack pk, T* __restrict__ ctab) {
+__global__ void __launch_bounds__(256) coef_kernel(const DevJob* __restrict__ jobs, DevInputs in, int nq, int qfast, DevPack pk,
+                                                   unsigned char* __restrict__ cbase) {
+    const DevBucket& b = jobs[blockIdx.y].b;
+    T* ctab = reinterpret_cast<T*>(cbase + jobs[blockIdx.y].coff);
     const int64_t total = (int64_t)b.n_elem * nq;
     const int64_t idx0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * V;
     if (idx0 >= total) return;
@@ -161,8 +164,11 @@ __global__ void __launch_bounds__(256) coef_kernel(DevBucket b, DevInputs in, in
 //   Ke[i][j] += sum_r tf_r[i][q] h_r        (TI rows per pass)
 // which is the reference's sum over terms and Gauss points regrouped.
 template <typename CT, int TI, bool QV, bool COOP>
-__global__ void __launch_bounds__(256) elem_cols(DevBucket b, const CT* __restrict__ ctab, uint32_t slice_mask, int jc, int qfast,
-                                                 CT* __restrict__ ke) {
+__global__ void __launch_bounds__(256) elem_cols(const DevJob* __restrict__ jobs, const unsigned char* __restrict__ cbase, uint32_t slice_mask,
+                                                 int jc, int qfast, CT* __restrict__ ke) {
+    const DevBucket& b = jobs[blockIdx.y].b;
+    const CT* ctab = reinterpret_cast<const CT*>(cbase + jobs[blockIdx.y].coff);
+    const int n_elem = b.n_elem, n_slices = b.n_slices;
     // QV with COOP: the block's coefficients of the current slice, staged once
     // in LDS ([element][term][q]) and read from there by the element's lanes
     // (dynamic shared memory sized by the launcher)
@@ -171,14 +177,14 @@ __global__ void __launch_bounds__(256) elem_cols(DevBucket b, const CT* __restri
     const int epb = blockDim.x / jc;
     const int el = threadIdx.x / jc, jl = threadIdx.x - (threadIdx.x / jc) * jc;
     const int e = blockIdx.x * epb + el;
-    const bool live = el < epb && e < b.n_elem;
+    const bool live = el < epb && e < n_elem;
     const int ec = live ? e : 0;
     const int nq = b.q_inv ? 1 : b.n_gp;
     const int ngp = b.n_gp;
-    const size_t cstride = (size_t)b.n_elem;
+    const size_t cstride = (size_t)n_elem;
     const SLX_CONST double* gw = (const SLX_CONST double*)b.gp_w;
     const SLX_CONST DevSlice* dsl = (const SLX_CONST DevSlice*)b.dslices;
-    for (int s = 0; s < b.n_slices; s++) {
+    for (int s = 0; s < n_slices; s++) {
         if (!((slice_mask >> s) & 1u)) continue;
         const int n_tf = dsl[s].n_tf, n_dof = dsl[s].n_dof, is_rhs = dsl[s].is_rhs, n_terms = dsl[s].n_terms;
         const int tf_pad = dsl[s].tf_pad, dof_pad = dsl[s].dof_pad;
@@ -193,7 +199,7 @@ __global__ void __launch_bounds__(256) elem_cols(DevBucket b, const CT* __restri
             for (int x = threadIdx.x; x < epb * per; x += blockDim.x) {
                 const int ee = x / per, rem = x - ee * per, t = rem / nq, qq = rem - t * nq;
                 const int eg = blockIdx.x * epb + ee;
-                const int eu = eg < b.n_elem ? eg : 0;
+                const int eu = eg < n_elem ? eg : 0;
                 const int cs = terms[t].coef;
                 cl[x] = qfast ? ctab[((size_t)cs * cstride + eu) * nq + qq] : ctab[((size_t)cs * nq + qq) * cstride + eu];
             }
@@ -577,26 +583,31 @@ __global__ void reduce_rhs(DevReduce rd, const KT* __restrict__ ke, double* __re
 
 // ---------------------------------------------------------------- launchers --
 
-hipError_t launch_coef(const DevBucket& b, const DevInputs& in, bool fp64, void* ctab, hipStream_t st, int qfast, const DevPack& pk) {
-    if (b.n_elem == 0 || b.n_coefs == 0) return hipSuccess;
+// b: one of the launch's buckets (they agree but for their elements), max_elem
+// the largest's elements.
+hipError_t launch_coef(const DevBucket& b, const DevJob* jobs, int n_jobs, int max_elem, const DevInputs& in, bool fp64, void* cbase,
+                       hipStream_t st, int qfast, const DevPack& pk) {
+    if (max_elem == 0 || b.n_coefs == 0) return hipSuccess;
     const int nq = b.q_inv ? 1 : b.n_gp;
-    const int64_t n = (int64_t)b.n_elem * nq;
+    const int64_t n = (int64_t)max_elem * nq;
     if (fp64) {
         const unsigned grid = (unsigned)((n + 2 * 256 - 1) / (2 * 256));
-        hipLaunchKernelGGL((coef_kernel<double, 2>), dim3(grid), dim3(256), 0, st, b, in, nq, qfast, pk, (double*)ctab);
+        hipLaunchKernelGGL((coef_kernel<double, 2>), dim3(grid, n_jobs), dim3(256), 0, st, jobs, in, nq, qfast, pk, (unsigned char*)cbase);
     } else {
         const unsigned grid = (unsigned)((n + 4 * 256 - 1) / (4 * 256));
-        hipLaunchKernelGGL((coef_kernel<float, 4>), dim3(grid), dim3(256), 0, st, b, in, nq, qfast, pk, (float*)ctab);
+        hipLaunchKernelGGL((coef_kernel<float, 4>), dim3(grid, n_jobs), dim3(256), 0, st, jobs, in, nq, qfast, pk, (unsigned char*)cbase);
     }
     return hipGetLastError();
 }
 
 template <typename CT, int TI>
-static void launch_cols(const DevBucket& b, const void* ctab, uint32_t mask, int jc, int qfast, void* ke, hipStream_t st) {
+static void launch_cols(const DevBucket& b, const DevJob* jobs, int n_jobs, int max_elem, const void* cbase, uint32_t mask, int jc, int qfast,
+                        void* ke, hipStream_t st) {
+    const unsigned char* cb = (const unsigned char*)cbase;
     const int epb = 256 / jc;
-    const unsigned grid = (unsigned)((b.n_elem + epb - 1) / epb);
+    const dim3 grid((unsigned)((max_elem + epb - 1) / epb), n_jobs);
     if (b.q_inv) {
-        hipLaunchKernelGGL((elem_cols<CT, TI, false, false>), dim3(grid), dim3(256), 0, st, b, (const CT*)ctab, mask, jc, qfast, (CT*)ke);
+        hipLaunchKernelGGL((elem_cols<CT, TI, false, false>), grid, dim3(256), 0, st, jobs, cb, mask, jc, qfast, (CT*)ke);
     } else {
         // stage the block's coefficients in LDS when they fit under the limit
         // (SLX_TUNE_ELEM_LDS_MAX bytes): a larger stage lowers the blocks a CU
@@ -608,14 +619,15 @@ static void launch_cols(const DevBucket& b, const void* ctab, uint32_t mask, int
         size_t lim = 48 * 1024;
         if (const char* t = std::getenv("SLX_TUNE_ELEM_LDS_MAX")) lim = (size_t)std::min(48L * 1024, std::max(0L, std::atol(t)));
         if (bytes <= lim)
-            hipLaunchKernelGGL((elem_cols<CT, TI, true, true>), dim3(grid), dim3(256), bytes, st, b, (const CT*)ctab, mask, jc, qfast, (CT*)ke);
+            hipLaunchKernelGGL((elem_cols<CT, TI, true, true>), grid, dim3(256), bytes, st, jobs, cb, mask, jc, qfast, (CT*)ke);
         else
-            hipLaunchKernelGGL((elem_cols<CT, TI, true, false>), dim3(grid), dim3(256), 0, st, b, (const CT*)ctab, mask, jc, qfast, (CT*)ke);
+            hipLaunchKernelGGL((elem_cols<CT, TI, true, false>), grid, dim3(256), 0, st, jobs, cb, mask, jc, qfast, (CT*)ke);
     }
 }
 
 template <typename CT>
-static void launch_cols_any(const DevBucket& b, const void* ctab, uint32_t mask, int qfast, void* ke, hipStream_t st) {
+static void launch_cols_any(const DevBucket& b, const DevJob* jobs, int n_jobs, int max_elem, const void* cbase, uint32_t mask, int qfast, void* ke,
+                            hipStream_t st) {
     int ntf = 1, ndof = 1;
     for (int s = 0; s < b.n_slices; s++)
         if ((mask >> s) & 1u) {
@@ -623,10 +635,10 @@ static void launch_cols_any(const DevBucket& b, const void* ctab, uint32_t mask,
             ndof = max(ndof, b.slices[s].n_dof);
         }
     const int jc = min(ndof, 64);
-    if (ntf <= 4) launch_cols<CT, 4>(b, ctab, mask, jc, qfast, ke, st);
-    else if (ntf <= 8) launch_cols<CT, 8>(b, ctab, mask, jc, qfast, ke, st);
-    else if (ntf <= 10) launch_cols<CT, 10>(b, ctab, mask, jc, qfast, ke, st);
-    else launch_cols<CT, 16>(b, ctab, mask, jc, qfast, ke, st);
+    if (ntf <= 4) launch_cols<CT, 4>(b, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, st);
+    else if (ntf <= 8) launch_cols<CT, 8>(b, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, st);
+    else if (ntf <= 10) launch_cols<CT, 10>(b, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, st);
+    else launch_cols<CT, 16>(b, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, st);
 }
 
 // Right-hand-side slices with many tf functions, as a blocked product over
@@ -640,7 +652,10 @@ template <typename CT>
 struct RhsVec4 { typedef CT type __attribute__((ext_vector_type(4))); };
 
 template <typename CT>
-__global__ void __launch_bounds__(256) rhs_tiles(DevBucket b, const CT* __restrict__ ctab, int s, int qfast, CT* __restrict__ ke) {
+__global__ void __launch_bounds__(256) rhs_tiles(const DevJob* __restrict__ jobs, const unsigned char* __restrict__ cbase, int s, int qfast,
+                                                 CT* __restrict__ ke) {
+    const DevBucket& b = jobs[blockIdx.z].b;
+    const CT* ctab = reinterpret_cast<const CT*>(cbase + jobs[blockIdx.z].coff);
     constexpr int RB = 64, EB = 64, RQ = 16;
     typedef typename RhsVec4<CT>::type CT4;
     __shared__ __attribute__((aligned(32))) CT Ts[RQ][RB];  // table values of the chunk, [Gauss point][row]
@@ -714,8 +729,9 @@ __global__ void __launch_bounds__(256) rhs_tiles(DevBucket b, const CT* __restri
     }
 }
 
-hipError_t launch_elem(const DevBucket& b, const void* ctab, int precision, void* ke, hipStream_t st, uint32_t slice_mask, int qfast) {
-    if (b.n_elem == 0 || slice_mask == 0) return hipSuccess;
+hipError_t launch_elem(const DevBucket& b, const DevJob* jobs, int n_jobs, int max_elem, const void* cbase, int precision, void* ke,
+                       hipStream_t st, uint32_t slice_mask, int qfast) {
+    if (max_elem == 0 || slice_mask == 0) return hipSuccess;
     // right-hand sides with more tf functions than one column pass of elem_cols
     // covers go to the tiled kernel
     uint32_t rhs_mask = 0;
@@ -724,17 +740,17 @@ hipError_t launch_elem(const DevBucket& b, const void* ctab, int precision, void
     const uint32_t mat_mask = slice_mask & ~rhs_mask;
     if (mat_mask) {
         if (precision == SLX_PREC_FP64)
-            launch_cols_any<double>(b, ctab, mat_mask, qfast, ke, st);
+            launch_cols_any<double>(b, jobs, n_jobs, max_elem, cbase, mat_mask, qfast, ke, st);
         else
-            launch_cols_any<float>(b, ctab, mat_mask, qfast, ke, st);
+            launch_cols_any<float>(b, jobs, n_jobs, max_elem, cbase, mat_mask, qfast, ke, st);
     }
     for (int s = 0; s < b.n_slices; s++) {
         if (!((rhs_mask >> s) & 1u)) continue;
-        const dim3 grid((unsigned)((b.n_elem + 63) / 64), (unsigned)((b.slices[s].n_tf + 63) / 64));
+        const dim3 grid((unsigned)((max_elem + 63) / 64), (unsigned)((b.slices[s].n_tf + 63) / 64), n_jobs);
         if (precision == SLX_PREC_FP64)
-            hipLaunchKernelGGL((rhs_tiles<double>), grid, dim3(256), 0, st, b, (const double*)ctab, s, qfast, (double*)ke);
+            hipLaunchKernelGGL((rhs_tiles<double>), grid, dim3(256), 0, st, jobs, (const unsigned char*)cbase, s, qfast, (double*)ke);
         else
-            hipLaunchKernelGGL((rhs_tiles<float>), grid, dim3(256), 0, st, b, (const float*)ctab, s, qfast, (float*)ke);
+            hipLaunchKernelGGL((rhs_tiles<float>), grid, dim3(256), 0, st, jobs, (const unsigned char*)cbase, s, qfast, (float*)ke);
     }
     return hipGetLastError();
 }

@@ -50,7 +50,7 @@ __device__ inline void geo_load(const DevBucket& b, const double* xyz, int e, Ge
 #pragma unroll
     for (int k = 0; k < SLX_MAX_GEO; k++) {
         if (k < b.n_geo) {
-            const int node = b.geo_nodes[(size_t)e * b.n_geo + k];
+            const int node = ((const SLX_GLOBAL int*)b.geo_nodes)[(size_t)e * b.n_geo + k];
             gx.x[k][0] = xyz[3 * (size_t)node];
             gx.x[k][1] = xyz[3 * (size_t)node + 1];
             gx.x[k][2] = xyz[3 * (size_t)node + 2];
@@ -73,7 +73,7 @@ __device__ inline void geo_eval(const DevBucket& b, const GeoX& gx, int q, Geo& 
             const double xc[3] = {gx.xyz[3 * (size_t)node], gx.xyz[3 * (size_t)node + 1], gx.xyz[3 * (size_t)node + 2]};
 #pragma unroll
             for (int r = 0; r < 3; r++) {
-                const double dn = r < b.elemdim ? b.geo_tab[((size_t)(1 + r) * b.n_geo + k) * b.n_gp + q] : 0.0;
+                const double dn = r < b.elemdim ? ((const SLX_CONST double*)b.geo_tab)[((size_t)(1 + r) * b.n_geo + k) * b.n_gp + q] : 0.0;
 #pragma unroll
                 for (int c = 0; c < 3; c++)
                     if (c < b.meshdim) g.J[3 * r + c] += xc[c] * dn;
@@ -85,7 +85,7 @@ __device__ inline void geo_eval(const DevBucket& b, const GeoX& gx, int q, Geo& 
             double dn[SLX_MAX_GEO];
 #pragma unroll
             for (int k = 0; k < SLX_MAX_GEO; k++)
-                dn[k] = (r < b.elemdim && k < b.n_geo) ? b.geo_tab[((size_t)(1 + r) * b.n_geo + k) * b.n_gp + q] : 0.0;
+                dn[k] = (r < b.elemdim && k < b.n_geo) ? ((const SLX_CONST double*)b.geo_tab)[((size_t)(1 + r) * b.n_geo + k) * b.n_gp + q] : 0.0;
 #pragma unroll
             for (int c = 0; c < 3; c++) {
                 double s = 0.0;
@@ -144,7 +144,7 @@ __device__ inline double field_value(const DevBucket& b, const DevInputs& in, in
         int a[FB];
         double c[FB];
 #pragma unroll
-        for (int u = 0; u < FB; u++) a[u] = k0 + u < fl.nff ? fl.addr[(size_t)(k0 + u) * b.n_elem + e] : -1;
+        for (int u = 0; u < FB; u++) a[u] = k0 + u < fl.nff ? ((const SLX_GLOBAL int*)fl.addr)[(size_t)(k0 + u) * b.n_elem + e] : -1;
 #pragma unroll
         for (int u = 0; u < FB; u++) c[u] = a[u] >= 0 ? data[a[u]] : 0.0;
 #pragma unroll
@@ -152,7 +152,7 @@ __device__ inline double field_value(const DevBucket& b, const DevInputs& in, in
             if (a[u] < 0) continue;
 #pragma unroll
             for (int d = 0; d < 4; d++)
-                if (d < nd) v[d] += c[u] * fl.tab[((size_t)d * fl.nff + k0 + u) * b.n_gp + q];
+                if (d < nd) v[d] += c[u] * ((const SLX_CONST double*)fl.tab)[((size_t)d * fl.nff + k0 + u) * b.n_gp + q];
         }
     }
     if (sd == 0) return v[0];
@@ -172,7 +172,7 @@ __device__ inline void field_gather(const DevBucket& b, const DevInputs& in, int
     const double* data = in.field_data[f];
     int a[NFF];
 #pragma unroll
-    for (int k = 0; k < NFF; k++) a[k] = fl.addr[(size_t)k * b.n_elem + e];
+    for (int k = 0; k < NFF; k++) a[k] = ((const SLX_GLOBAL int*)fl.addr)[(size_t)k * b.n_elem + e];
 #pragma unroll
     for (int k = 0; k < NFF; k++) {
         ok[k] = a[k] >= 0;
@@ -192,7 +192,7 @@ __device__ inline double field_value_pre(const DevBucket& b, int f, const double
         if (!ok[k]) continue;
 #pragma unroll
         for (int d = 0; d < 4; d++)
-            if (d < nd) v[d] += c[k] * fl.tab[((size_t)d * NFF + k) * b.n_gp + q];
+            if (d < nd) v[d] += c[k] * ((const SLX_CONST double*)fl.tab)[((size_t)d * NFF + k) * b.n_gp + q];
     }
     if (sd == 0) return v[0];
     double s = 0.0;

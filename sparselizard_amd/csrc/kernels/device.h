@@ -43,6 +43,14 @@ struct DevBucket {
     DevField fields[SLX_MAX_FIELDS];
 };
 
+// One bucket of a launch (blockIdx.y names it) and where its coefficients lie.
+// Buckets that differ only in their elements, addresses and table values (the
+// orientations of one element type) share their launches.
+struct DevJob {
+    DevBucket b;
+    int64_t coff;               // bytes from the coefficient tables' base
+};
+
 struct DevInputs {
     const double* xyz;          // [n_nodes][3]
     const double* params;       // [n_params][param_len]
@@ -78,5 +86,8 @@ struct DevReduce {
 
 // Constant-address-space views: uniform loads through them become scalar loads.
 #define SLX_CONST __attribute__((address_space(4)))
+// Pointers read from memory are taken as flat ones otherwise, whose loads also
+// occupy the LDS counter.
+#define SLX_GLOBAL __attribute__((address_space(1)))
 
 }  // namespace slx

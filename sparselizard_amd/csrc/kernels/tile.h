@@ -38,7 +38,7 @@ struct TileSlice {
     const int32_t* tinfo;
     float a_unscale;                // 1 / power-of-two scale of P
     float tqmax;                    // max |tq|
-    const uint32_t* afrag;          // set per launch: afrag_x[arith]
+    const uint32_t* afrag;          // of the launch's arithmetic: afrag_x[arith]
     const uint32_t* afrag_x[3];     // [nkc][mtt][planes][64 lanes][4 words]: lane l of chunk c and row tile mt holds its entries
                                     // v = 0..7, the scaled P^T[16 mt + l % 16][k(c, l / 16, v)], as f16 hi, lo (2 planes),
                                     // bf16 hi, mid, lo (3 planes) or floats (2 words: v = 0..3, 4..7)
@@ -46,11 +46,18 @@ struct TileSlice {
     int64_t ke_base, ke_ld;
 };
 
+// One bucket's slice of a launch (blockIdx.y names it).
+struct TileJob {
+    TileSlice t;
+    int64_t n_elem, coff;           // elements; bytes of the coefficients from the tables' base
+};
+
 size_t tile_lds_bytes(const TileSlice& t, int planes);
-// Element matrices of one slice (coefficient table [slot][element][point]
-// when qfast, else [slot][point][element]).
+// Element matrices of one slice of n_jobs buckets that agree in its shape
+// (one: the first of them, max_elem: the largest's elements; coefficient tables
+// [slot][element][point] when qfast, else [slot][point][element]).
 // arith: 0 FP16 split, 1 BF16 split, 2 FP32.
-hipError_t launch_tile(const DevBucket& b, const TileSlice& t, int arith, const float* ctab, int qfast, float* ke, int n_cu,
-                       hipStream_t st);
+hipError_t launch_tile(const TileJob& one, const TileJob* jobs, int n_jobs, int max_elem, int arith, const void* cbase, int qfast, float* ke,
+                       int n_cu, hipStream_t st);
 
 }  // namespace slx

@@ -30,8 +30,10 @@
 #include <dlfcn.h>
 
 namespace slx {
-hipError_t launch_coef(const DevBucket& b, const DevInputs& in, bool fp64, void* ctab, hipStream_t st, int qfast, const DevPack& pk);
-hipError_t launch_elem(const DevBucket& b, const void* ctab, int precision, void* ke, hipStream_t st, uint32_t slice_mask, int qfast);
+hipError_t launch_coef(const DevBucket& b, const DevJob* jobs, int n_jobs, int max_elem, const DevInputs& in, bool fp64, void* cbase,
+                       hipStream_t st, int qfast, const DevPack& pk);
+hipError_t launch_elem(const DevBucket& b, const DevJob* jobs, int n_jobs, int max_elem, const void* cbase, int precision, void* ke,
+                       hipStream_t st, uint32_t slice_mask, int qfast);
 hipError_t scratch_init(int device);
 hipError_t launch_reduce(const DevReduce& rd, int max_erow_len, bool ke_fp64, const void* ke, double* Aval, double* Dval,
                          double* rhs, bool has_matrix, bool has_rhs, hipStream_t st, const int64_t* class_begin,
@@ -192,8 +194,7 @@ struct slx_plan_s {
 
     hipGraphExec_t graph_exec = nullptr;  // captured numeric phase (slx_plan_graph_capture)
     // right-hand-side-only buckets run, with the rhs reduction, on a side
-    // stream forked from and joined back into the caller's stream; they keep
-    // their coefficients in their own table
+    // stream forked from and joined back into the caller's stream
     std::vector<uint8_t> rhs_only;     // per bucket: every slice is a rhs slice
     bool side_ok = false;              // every rhs slice lives in a rhs-only bucket
     // compiled coefficient programs per bucket ([0] FP32, [1] FP64; null: interpreter)
@@ -202,7 +203,17 @@ struct slx_plan_s {
     std::string coef_jit_error;        // last compiler message (diagnostics)
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-    DBuf d_ctab_side;
+    // coefficient tables: every bucket its own region of d_ctab
+    std::vector<size_t> ctab_off;      // byte offset per bucket
+    size_t ctab_bytes = 0;
+    // launches shared by buckets that agree but for their elements
+    struct Family {
+        std::vector<int> buckets;
+        int max_elem = 0;
+        const DevJob* jobs = nullptr;  // device
+        std::vector<std::pair<int, std::array<const TileJob*, 3>>> tile;  // (slice, jobs per arithmetic)
+    };
+    std::vector<Family> families;      // in the order of their first buckets
     std::vector<MfmaBucket> mfma;      // per bucket; M == 0 when not eligible
     std::vector<uint32_t> mfma_mask;   // matrix slices handled by the MFMA kernel
     std::vector<std::vector<std::pair<int, FactorSlice>>> factor;  // per bucket: (slice, factorized MFMA data)
@@ -212,13 +223,11 @@ struct slx_plan_s {
     int last_qfast = 0;                // coefficient table layout of the last bucket assembled
     bool factor64 = true;              // FP64 mode: factorized slices on v_mfma_f64 (SLX_TUNE_FP64_FACTOR=0: VALU)
     // fused launch: the factorized slices of every bucket in one persistent
-    // launch (per arithmetic: F16, BF16, F32, and 3 = FP64); each fused bucket
-    // keeps its coefficients in its own region of d_ctab_fused
+    // launch (per arithmetic: F16, BF16, F32, and 3 = FP64)
     bool fused = false;
     uint32_t fused_arith = 0;              // bit a: arithmetic a (3 = FP64) uses the fused launch
     std::vector<uint8_t> fuse_bucket;      // per bucket: its factorized slices run in the fused launch
-    std::vector<size_t> fuse_off;          // per bucket: byte offset of its coefficient region
-    DBuf d_ctab_fused, d_fused_counter;
+    DBuf d_fused_counter;
     DBuf d_fused[4];
     int n_fused[4] = {0, 0, 0, 0};
     int64_t fused_total[4] = {0, 0, 0, 0};
@@ -1527,22 +1536,13 @@ void build_fused(slx_plan_s& P, const slx_plan_desc& d) {
     if (const char* t = std::getenv("SLX_TUNE_FUSED")) mode = std::atoi(t);
     P.fused_arith = mode == 1 ? 0xFu : ((1u << AR_F16) | (1u << AR_BF16));
     P.fuse_bucket.assign(d.n_buckets, 0);
-    P.fuse_off.assign(d.n_buckets, 0);
     int nb = 0;
     for (int b = 0; b < d.n_buckets; b++)
         if (!P.factor[b].empty() && !P.rhs_only[b]) nb++;
     P.fused = mode != 0 && (nb >= 2 || (mode == 1 && nb >= 1));
     if (!P.fused) return;
-    size_t bytes = 0;
-    for (int b = 0; b < d.n_buckets; b++) {
-        if (P.factor[b].empty() || P.rhs_only[b]) continue;
-        const slx_bucket_desc& bd = d.buckets[b];
-        P.fuse_bucket[b] = 1;
-        P.fuse_off[b] = bytes;
-        const size_t words = (size_t)std::max(bd.n_coefs, 1) * (bd.q_invariant ? 1 : bd.n_gp) * std::max(bd.n_elem, 1);
-        bytes += (words * sizeof(double) + 255) / 256 * 256;
-    }
-    P.d_ctab_fused.alloc(std::max<size_t>(bytes, 256));
+    for (int b = 0; b < d.n_buckets; b++)
+        if (!P.factor[b].empty() && !P.rhs_only[b]) P.fuse_bucket[b] = 1;
     P.d_fused_counter.alloc(sizeof(unsigned long long));
     for (int a = 0; a < 4; a++) {
         struct Entry {
@@ -1563,7 +1563,7 @@ void build_fused(slx_plan_s& P, const slx_plan_desc& d) {
                     en.fs.f.arith = a;
                     en.fs.f.afrag = f0.afrag_x[a];
                 }
-                en.fs.ctab = (const char*)P.d_ctab_fused.p + P.fuse_off[b];
+                en.fs.ctab = (const char*)P.d_ctab.p + P.ctab_off[b];
                 en.fs.n_elem = d.buckets[b].n_elem;
                 en.fs.variant = factor_variant_index(f0.bm, f0.bn);
                 SLX_CHECK(en.fs.variant >= 0, "internal: factorized slice without a kernel variant");
@@ -1780,6 +1780,76 @@ void choose_direct(slx_plan_s& P, const slx_plan_desc& d, const KeLayout& L) {
     P.dpack.erec = pack.erec;
 }
 
+// Buckets that may share their launches: the same element type, program, slice
+// shapes and kernels; only elements, addresses and table values differ.
+bool same_family(const slx_plan_s& P, const slx_plan_desc& d, int x, int y) {
+    const slx_bucket_desc &a = d.buckets[x], &b = d.buckets[y];
+    if (P.direct && (x == P.direct_bucket || y == P.direct_bucket || x == P.direct_rhs_bucket || y == P.direct_rhs_bucket)) return false;
+    if (P.mfma[x].M > 0 || P.mfma[y].M > 0 || P.factor[x].size() != P.factor[y].size()) return false;
+    for (size_t k = 0; k < P.factor[x].size(); k++) {
+        const FactorSlice &u = P.factor[x][k].second, &v = P.factor[y][k].second;
+        if (P.factor[x][k].first != P.factor[y][k].first || u.arith_ok != v.arith_ok || u.f64_ok != v.f64_ok) return false;
+    }
+    if (a.n_elem == 0 || b.n_elem == 0 || a.elem_type != b.elem_type || a.n_geo != b.n_geo || a.n_gp != b.n_gp || a.n_slices != b.n_slices ||
+        a.n_instr != b.n_instr || a.n_regs != b.n_regs || a.n_coefs != b.n_coefs || a.q_invariant != b.q_invariant)
+        return false;
+    if (a.n_instr > 0 && std::memcmp(a.prog, b.prog, (size_t)a.n_instr * sizeof(slx_instr)) != 0) return false;
+    for (int f = 0; f < d.n_fields; f++)
+        if (d.field_nff[(size_t)f * d.n_buckets + x] != d.field_nff[(size_t)f * d.n_buckets + y]) return false;
+    for (int s = 0; s < a.n_slices; s++) {
+        const slx_slice_desc &u = a.slices[s], &v = b.slices[s];
+        if (u.n_tf != v.n_tf || (u.is_rhs != 0) != (v.is_rhs != 0) || (!u.is_rhs && u.n_dof != v.n_dof) || u.n_terms != v.n_terms) return false;
+        if (u.n_terms > 0 && std::memcmp(u.terms, v.terms, (size_t)u.n_terms * sizeof(slx_term)) != 0) return false;
+    }
+    if (P.tile[x].size() != P.tile[y].size() || P.tile_mask[x] != P.tile_mask[y]) return false;
+    for (size_t k = 0; k < P.tile[x].size(); k++) {
+        const TileSlice &u = P.tile[x][k].second, &v = P.tile[y][k].second;
+        if (P.tile[x][k].first != P.tile[y][k].first || u.na != v.na || u.nkc != v.nkc || u.ngpp != v.ngpp || u.mtt != v.mtt || u.ntt != v.ntt)
+            return false;
+    }
+    return true;
+}
+
+// Families and their launch descriptions.  24 orientation buckets of 2000
+// order-2 tetrahedra each (H(curl) Maxwell, 20^3 x 6) took five launches of at
+// most 48 workgroups apiece, 2.1 ms per assembly; four launches for all of them
+// and the compiled program take 0.47 ms.
+void build_families(slx_plan_s& P, const slx_plan_desc& d) {
+    P.families.clear();
+    for (int b = 0; b < d.n_buckets; b++) {
+        slx_plan_s::Family* f = nullptr;
+        for (auto& x : P.families)
+            if (x.buckets.size() < 65535 && same_family(P, d, x.buckets[0], b)) {
+                f = &x;
+                break;
+            }
+        if (!f) {
+            P.families.emplace_back();
+            f = &P.families.back();
+        }
+        f->buckets.push_back(b);
+        f->max_elem = std::max(f->max_elem, d.buckets[b].n_elem);
+    }
+    for (auto& f : P.families) {
+        std::vector<DevJob> jobs;
+        for (int b : f.buckets) jobs.push_back(DevJob{P.dbuckets[b], (int64_t)P.ctab_off[b]});
+        f.jobs = P.dev(jobs.data(), jobs.size());
+        for (size_t k = 0; k < P.tile[f.buckets[0]].size(); k++) {
+            std::array<const TileJob*, 3> per{};
+            for (int ar = 0; ar < 3; ar++) {
+                std::vector<TileJob> tj;
+                for (int b : f.buckets) {
+                    TileJob j{P.tile[b][k].second, d.buckets[b].n_elem, (int64_t)P.ctab_off[b]};
+                    j.t.afrag = j.t.afrag_x[ar];
+                    tj.push_back(j);
+                }
+                per[ar] = P.dev(tj.data(), tj.size());
+            }
+            f.tile.push_back({P.tile[f.buckets[0]][k].first, per});
+        }
+    }
+}
+
 // The row-wise maps, once the pattern is known; a pattern it cannot take
 // (32-bit slots, rows beyond the LDS accumulators) returns the bucket to the
 // element kernels.
@@ -1792,6 +1862,7 @@ void build_direct(slx_plan_s& P, const slx_plan_desc& d, const KeLayout& L) {
         build_mfma(P, bd, P.direct_bucket, L);
         build_tile(P, bd, P.direct_bucket, L);
         build_factor(P, bd, P.direct_bucket, L);
+        build_families(P, d);
         if (!P.needs_ke) P.d_ke.alloc(P.ke_capacity_bytes);
         P.needs_ke = true;
         return;
@@ -1845,7 +1916,6 @@ void upload_buckets(slx_plan_s& P, const slx_plan_desc& d, const KeLayout& L) {
         hipDeviceProp_t prop;
         if (hipGetDeviceProperties(&prop, P.ctx->device) == hipSuccess && prop.multiProcessorCount > 0) P.n_cu = prop.multiProcessorCount;
     }
-    size_t ctab_words = 1, ctab_side_words = 1;
     P.rhs_only.assign(d.n_buckets, 0);
     bool rhs_in_mixed = false, any_rhs_only = false;
     for (int b = 0; b < d.n_buckets; b++) {
@@ -1897,9 +1967,6 @@ void upload_buckets(slx_plan_s& P, const slx_plan_desc& d, const KeLayout& L) {
             std::vector<float> tq32(tq.begin(), tq.end());
             dtabs32[t] = P.dev(tq32.data(), tq32.size());
         }
-        const size_t words = (size_t)std::max(bd.n_coefs, 1) * (bd.q_invariant ? 1 : bd.n_gp) * std::max(bd.n_elem, 1);
-        if (P.rhs_only[b]) ctab_side_words = std::max(ctab_side_words, words);
-        else ctab_words = std::max(ctab_words, words);
         for (int s = 0; s < bd.n_slices; s++) {
             const slx_slice_desc& sd = bd.slices[s];
             DevSlice& ds = db.slices[s];
@@ -1962,9 +2029,16 @@ void upload_buckets(slx_plan_s& P, const slx_plan_desc& d, const KeLayout& L) {
         build_factor(P, d.buckets[b], b, L);
     }
     upload(P.consts, d.consts, (size_t)std::max(d.n_consts, 1), P.stream);
-    if (P.direct) ctab_words = std::max(ctab_words, (size_t)P.pack.erec * std::max(d.buckets[P.direct_bucket].n_elem, 1));
-    P.d_ctab.alloc(ctab_words * sizeof(double));
-    P.d_ctab_side.alloc(ctab_side_words * sizeof(double));
+    P.ctab_off.assign(d.n_buckets, 0);
+    for (int b = 0; b < d.n_buckets; b++) {
+        const slx_bucket_desc& bd = d.buckets[b];
+        size_t per = (size_t)std::max(bd.n_coefs, 1) * (bd.q_invariant ? 1 : bd.n_gp);
+        if (P.direct && b == P.direct_bucket) per = std::max(per, (size_t)P.pack.erec);
+        P.ctab_off[b] = P.ctab_bytes;
+        P.ctab_bytes += (per * std::max(bd.n_elem, 1) * sizeof(double) + 255) / 256 * 256;
+    }
+    P.d_ctab.alloc(std::max<size_t>(P.ctab_bytes, 256));
+    build_families(P, d);
     build_fused(P, d);
     P.side_ok = d.has_matrix && d.has_rhs && any_rhs_only && !rhs_in_mixed;
     if (P.side_ok) {
@@ -1974,17 +2048,26 @@ void upload_buckets(slx_plan_s& P, const slx_plan_desc& d, const KeLayout& L) {
     }
 }
 
-// Compiled coefficient programs for the buckets the mode selects (auto: buckets
-// of at least SLX_COEF_JIT_MIN elements); unique programs compiled in parallel.
+// Compiled coefficient programs for the buckets the mode selects (auto: programs
+// that at least SLX_COEF_JIT_MIN elements run, over all buckets: the
+// interpreter's scratch registers cost the same per element whatever its
+// bucket); unique programs compiled in parallel.
 #define SLX_COEF_JIT_MIN 4096
 void compile_coef_programs(slx_plan_s& P, const slx_plan_desc& d) {
     P.coef_fn.assign(d.n_buckets, {nullptr, nullptr});
     if (P.coef_mode == 1) return;
     std::vector<std::pair<int, int>> todo;  // (bucket, fp64)
+    std::vector<int64_t> runs(d.n_buckets, 0);  // elements that run the bucket's program
+    for (int b = 0; b < d.n_buckets; b++)
+        for (int c = 0; c < d.n_buckets; c++)
+            if (d.buckets[b].n_instr == d.buckets[c].n_instr &&
+                (d.buckets[b].n_instr == 0 ||
+                 std::memcmp(d.buckets[b].prog, d.buckets[c].prog, (size_t)d.buckets[b].n_instr * sizeof(slx_instr)) == 0))
+                runs[b] += d.buckets[c].n_elem;
     for (int b = 0; b < d.n_buckets; b++) {
         if (d.buckets[b].n_coefs == 0 || d.buckets[b].n_elem == 0) continue;
         // programs beyond the interpreter's register file are always compiled
-        if (P.coef_mode == 0 && d.buckets[b].n_elem < SLX_COEF_JIT_MIN && d.buckets[b].n_regs <= SLX_MAX_REGS) continue;
+        if (P.coef_mode == 0 && runs[b] < SLX_COEF_JIT_MIN && d.buckets[b].n_regs <= SLX_MAX_REGS) continue;
         todo.push_back({b, 0});
         todo.push_back({b, 1});
     }
@@ -2002,8 +2085,11 @@ void compile_coef_programs(slx_plan_s& P, const slx_plan_desc& d) {
                 hipFunction_t fn = nullptr;
                 std::string err;
                 const bool records = P.direct && todo[i].first == P.direct_bucket;
+                bool several = false;
+                for (const auto& f : P.families)
+                    several = several || (f.buckets.size() > 1 && std::find(f.buckets.begin(), f.buckets.end(), todo[i].first) != f.buckets.end());
                 if (coef_compile(bd.prog, bd.n_instr, todo[i].second != 0, bd.q_invariant == 0, fnff, &fn, &err,
-                                 records ? P.pack : CoefPack())) {
+                                 records ? P.pack : CoefPack(), several)) {
                     P.coef_fn[todo[i].first][todo[i].second] = fn;
                 } else {
                     std::lock_guard<std::mutex> lk(mu);
@@ -2093,52 +2179,49 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
     const int fa = arith >= 0 ? arith : ((ke64 && P.factor64) ? 3 : -1);
     const bool fused = P.fused && fa >= 0 && ((P.fused_arith >> fa) & 1u) && P.n_fused[fa] > 0;
     P.last_fused = fused;
-    if (fused) {
-        for (size_t bi = 0; bi < P.dbuckets.size(); bi++) {
-            if (!P.fuse_bucket[bi] || factor_mask(bi) == 0) continue;
-            const DevBucket& b = P.dbuckets[bi];
-            void* ctab = (char*)P.d_ctab_fused.p + P.fuse_off[bi];
-            if (tm) tm->begin(T_COEF);
-            const hipFunction_t cfn = bi < P.coef_fn.size() ? P.coef_fn[bi][ke64 ? 1 : 0] : nullptr;
-            if (cfn) HIPCHECK(coef_launch(cfn, b, in, b.q_inv ? 1 : b.n_gp, 1, ctab, st));
-            else {
-                SLX_CHECK(b.n_regs <= SLX_MAX_REGS, "coefficient program of " << b.n_regs << " registers has no compiled kernel and the interpreter holds "
-                                                   << SLX_MAX_REGS << " (" << P.coef_jit_error << ")");
-                HIPCHECK(launch_coef(b, in, ke64, ctab, st, 1, P.dpack));
-            }
-            if (tm) tm->end();
+    // coefficients of a family into its buckets' regions
+    auto coefficients = [&](const slx_plan_s::Family& f, int qfast, hipStream_t s) {
+        const int b0 = f.buckets[0];
+        const DevBucket& b = P.dbuckets[b0];
+        if (tm) tm->begin(T_COEF);
+        const hipFunction_t cfn = b0 < (int)P.coef_fn.size() ? P.coef_fn[b0][ke64 ? 1 : 0] : nullptr;
+        if (cfn) {
+            HIPCHECK(coef_launch(cfn, b, (int64_t)P.ctab_off[b0], f.jobs, (int)f.buckets.size(), f.max_elem, in, b.q_inv ? 1 : b.n_gp, qfast, P.d_ctab.p, s));
+        } else {
+            SLX_CHECK(b.n_regs <= SLX_MAX_REGS, "coefficient program of " << b.n_regs << " registers has no compiled kernel and the interpreter holds "
+                                               << SLX_MAX_REGS << " (" << P.coef_jit_error << ")");
+            HIPCHECK(launch_coef(b, f.jobs, (int)f.buckets.size(), f.max_elem, in, ke64, P.d_ctab.p, s, qfast, P.dpack));
         }
+        if (tm) tm->end();
+    };
+    if (fused) {
+        for (const auto& f : P.families)
+            if (P.fuse_bucket[f.buckets[0]] && factor_mask(f.buckets[0]) != 0) coefficients(f, 1, st);
         if (tm) tm->begin(T_MFMA);
         HIPCHECK(launch_factor_fused(P.d_fused[fa].as<FusedSlice>(), P.n_fused[fa], P.fused_total[fa],
                                      P.d_fused_counter.as<unsigned long long>(), fa, P.fused_lds[fa], P.d_ke.p, P.n_cu, st));
         if (tm) tm->end();
     }
-    for (size_t bi = 0; bi < P.dbuckets.size(); bi++) {
+    for (const auto& f : P.families) {
+        const size_t bi = (size_t)f.buckets[0];
+        const int nj = (int)f.buckets.size();
         const DevBucket& b = P.dbuckets[bi];
         const hipStream_t bst = (overlap && P.rhs_only[bi]) ? P.side : st;
-        const uint32_t fmask = factor_mask(bi);  // slices on the factorized kernel
+        const uint32_t fmask = factor_mask(bi);  // slices on the factorized kernel (a launch per bucket, or the fused one)
         const uint32_t tmask = arith >= 0 ? P.tile_mask[bi] & ~fmask : 0u;  // slices on the one-tile kernel
         const bool in_fused = fused && P.fuse_bucket[bi] && fmask != 0;
-        void* ctab = in_fused ? (void*)((char*)P.d_ctab_fused.p + P.fuse_off[bi]) : (P.rhs_only[bi] ? P.d_ctab_side.p : P.d_ctab.p);
+        const void* ctab = (const char*)P.d_ctab.p + P.ctab_off[bi];
         uint32_t all = (b.n_slices >= 32) ? 0xffffffffu : ((1u << b.n_slices) - 1u);
         uint32_t done = 0;
         // the factorized kernel reads the coefficients of one element contiguously,
         // the row-wise kernel reads records
         const bool records = P.direct && (int)bi == P.direct_bucket;
         const int qfast = records ? 2 : fmask != 0 ? 1 : 0;
-        P.last_qfast = qfast;
-        P.last_ctab = ctab;
-        if (!in_fused) {
-            if (tm) tm->begin(T_COEF);
-            const hipFunction_t cfn = bi < P.coef_fn.size() ? P.coef_fn[bi][ke64 ? 1 : 0] : nullptr;
-            if (cfn) HIPCHECK(coef_launch(cfn, b, in, b.q_inv ? 1 : b.n_gp, qfast, ctab, bst));
-            else {
-                SLX_CHECK(b.n_regs <= SLX_MAX_REGS, "coefficient program of " << b.n_regs << " registers has no compiled kernel and the interpreter holds "
-                                                   << SLX_MAX_REGS << " (" << P.coef_jit_error << ")");
-                HIPCHECK(launch_coef(b, in, ke64, ctab, bst, qfast, P.dpack));
-            }
-            if (tm) tm->end();
+        if (f.buckets.back() + 1 == (int)P.dbuckets.size()) {
+            P.last_qfast = qfast;
+            P.last_ctab = (const char*)P.d_ctab.p + P.ctab_off.back();
         }
+        if (!in_fused) coefficients(f, qfast, bst);
         if (records || (P.direct && (int)bi == P.direct_rhs_bucket)) continue;  // the row-wise launch does the rest
         if (arith >= 0 && P.mfma[bi].M > 0 && ((P.mfma[bi].arith_ok >> arith) & 1u)) {
             if (tm) tm->begin(T_MFMA);
@@ -2150,26 +2233,33 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
             done |= fmask;  // computed by the fused launch
         } else if (fmask != 0) {
             if (tm) tm->begin(T_MFMA);
-            for (auto& fs : P.factor[bi])
-                if ((fmask >> fs.first) & 1u) {
-                    if (ke64) HIPCHECK(launch_factor64(b, fs.second, (const double*)ctab, P.d_ke.as<double>(), P.n_cu, bst));
-                    else HIPCHECK(launch_factor(b, fs.second, arith, (const float*)ctab, P.d_ke.as<float>(), P.n_cu, bst));
-                }
+            for (int fb : f.buckets) {
+                const void* ct = (const char*)P.d_ctab.p + P.ctab_off[fb];
+                for (auto& fs : P.factor[fb])
+                    if ((fmask >> fs.first) & 1u) {
+                        if (ke64) HIPCHECK(launch_factor64(P.dbuckets[fb], fs.second, (const double*)ct, P.d_ke.as<double>(), P.n_cu, bst));
+                        else HIPCHECK(launch_factor(P.dbuckets[fb], fs.second, arith, (const float*)ct, P.d_ke.as<float>(), P.n_cu, bst));
+                    }
+            }
             if (tm) tm->end();
             done |= fmask;
         }
         if (tmask != 0) {
             if (tm) tm->begin(T_MFMA);
-            for (auto& ts : P.tile[bi])
-                if ((tmask >> ts.first) & 1u) HIPCHECK(launch_tile(b, ts.second, arith == AR_BF16 ? 1 : arith == AR_F32 ? 2 : 0, (const float*)ctab, qfast, P.d_ke.as<float>(),
-                                                                P.n_cu, bst));
+            const int ar = arith == AR_BF16 ? 1 : arith == AR_F32 ? 2 : 0;
+            for (size_t k = 0; k < f.tile.size(); k++)
+                if ((tmask >> f.tile[k].first) & 1u) {
+                    TileJob one{P.tile[bi][k].second, b.n_elem, (int64_t)P.ctab_off[bi]};
+                    one.t.afrag = one.t.afrag_x[ar];
+                    HIPCHECK(launch_tile(one, f.tile[k].second[ar], nj, f.max_elem, ar, P.d_ctab.p, qfast, P.d_ke.as<float>(), P.n_cu, bst));
+                }
             if (tm) tm->end();
             done |= tmask;
         }
         int p = (precision == SLX_PREC_FP64) ? SLX_PREC_FP64 : SLX_PREC_FP32;
         if ((all & ~done) != 0) {
             if (tm) tm->begin(T_VALU);
-            HIPCHECK(launch_elem(b, ctab, p, P.d_ke.p, bst, all & ~done, qfast));
+            HIPCHECK(launch_elem(b, f.jobs, nj, f.max_elem, P.d_ctab.p, p, P.d_ke.p, bst, all & ~done, qfast));
             if (tm) tm->end();
         }
     }
@@ -2183,7 +2273,8 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
             cl.push_back(c.max_len);
         }
         if (P.direct)
-            HIPCHECK(launch_direct(P.dd, ke64, P.d_ctab.p, P.direct_rhs_bucket == P.direct_bucket ? P.d_ctab.p : P.d_ctab_side.p,
+            HIPCHECK(launch_direct(P.dd, ke64, (char*)P.d_ctab.p + P.ctab_off[P.direct_bucket],
+                                   (char*)P.d_ctab.p + P.ctab_off[std::max(P.direct_rhs_bucket, 0)],
                                    P.d_Aval.as<double>(), P.d_Dval.as<double>(), P.d_rhs.as<double>(), st, cb.data(), ce.data(), cl.data(),
                                    (int)cl.size()));
         else
@@ -2821,8 +2912,9 @@ slx_status slx_plan_element_matrices(slx_plan p, double* out, int64_t cap) {
         if (p->direct) {
             // row-wise plans keep no element matrices: from the last assembly's coefficients
             if (!p->d_ke.p) p->d_ke.alloc(p->ke_capacity_bytes);
-            HIPCHECK(launch_direct_ke(p->dd, p->dbuild, p->last_precision == SLX_PREC_FP64, p->d_ctab.p,
-                                      p->direct_rhs_bucket == p->direct_bucket ? p->d_ctab.p : p->d_ctab_side.p, p->d_ke.p, p->stream));
+            HIPCHECK(launch_direct_ke(p->dd, p->dbuild, p->last_precision == SLX_PREC_FP64,
+                                      (char*)p->d_ctab.p + p->ctab_off[p->direct_bucket],
+                                      (char*)p->d_ctab.p + p->ctab_off[std::max(p->direct_rhs_bucket, 0)], p->d_ke.p, p->stream));
             HIPCHECK(hipStreamSynchronize(p->stream));
         }
         if (p->last_precision == SLX_PREC_FP64) {

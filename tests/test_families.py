@@ -1,0 +1,26 @@
+"""Launches shared by the orientation buckets of one element type (24 tetrahedra
+orientations at most) against the oracle: interpreted and compiled programs
+(4096 elements and more over all buckets), every kernel of the family (one-tile,
+VALU element kernel, FP64, right-hand sides)."""
+import numpy as np
+import pytest
+
+import sparselizard_amd as sa
+from oracle import py_oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("f16split", 1e-6), ("bf16split", 1e-6), ("fp32", 1e-6)])
+@pytest.mark.parametrize("spec,tile", [("elem=tet;term=maxwell;n=3;order=2", "1"), ("elem=tet;term=maxwell;n=9;order=2", "1"),
+                                       ("elem=tet;term=maxwell;n=3;order=2", "0"), ("elem=tet;term=maxwell;n=5;order=1", "1")])
+def test_orientation_buckets(ctx, spec, tile, precision, tol, monkeypatch):
+    print("case families", spec, tile, precision, flush=True)
+    monkeypatch.setenv("SLX_TUNE_TILE", tile)
+    prob = sa.Problem(ctx, "hcurlprojection", spec)
+    info = prob.info()
+    got = prob.generate(precision).csr(info["ndofs"])
+    ref = py_oracle.assemble(prob.desc_ptr(), prob.numeric(), info["ndofs"], info["nfree"], nthreads=8)
+    assert np.array_equal(got.Arow, ref.Arow) and np.array_equal(got.Acol, ref.Acol)
+    for a, b in ((got.Aval, ref.Aval), (got.rhs, ref.rhs)):
+        assert np.linalg.norm(a - b) <= tol * np.linalg.norm(b)
