@@ -21,6 +21,20 @@ struct CoefPack {
     std::vector<int> pos, pads;
 };
 
+// Shape of an element kernel: the slices of a bucket whose element matrices one
+// thread can hold.
+struct ElemShape {
+    struct Slice {
+        int n_tf, n_dof;              // n_dof 0: right-hand side
+        bool vec4;                    // rows start 16-byte aligned (FP32)
+        std::vector<slx_term> terms;
+    };
+    std::vector<Slice> slices;        // every slice of the bucket
+    bool affine = false, q_inv = false;
+    bool store = false;               // also writes the coefficient table [slot][point][element]
+};
+#define SLX_ELEM_MAX 72               // element-matrix entries of one thread
+
 // Full source of the kernel of one program (prelude included).  runs: each
 // thread walks a run of Gauss points of one element (Gauss-point-varying
 // buckets), and gathers the values of every field of at most
@@ -29,12 +43,22 @@ struct CoefPack {
 // (coefficients constant over the Gauss points) the kernel writes records.
 // several: the kernel of a launch over several buckets.
 std::string coef_kernel_source(const slx_instr* prog, int n_instr, bool fp64, bool runs, const std::vector<int>& field_nff,
-                               const CoefPack& pack = CoefPack(), bool several = false);
+                               const CoefPack& pack = CoefPack(), bool several = false, bool affine = false);
+// Source of the element kernel slx_elem of one program: one thread per element
+// evaluates the geometry, the program and the contraction of every slice, point
+// by point, so that no coefficient goes through memory.
+std::string elem_kernel_source(const slx_instr* prog, int n_instr, bool fp64, const std::vector<int>& field_nff, const ElemShape& shape,
+                               bool several);
 // Compiles (or finds in the process-wide cache) the kernel of one program for
 // the current device; fp64 selects FP64 coefficients.  On failure returns
 // false with the compiler log in *err.
 bool coef_compile(const slx_instr* prog, int n_instr, bool fp64, bool runs, const std::vector<int>& field_nff, hipFunction_t* fn,
-                  std::string* err, const CoefPack& pack = CoefPack(), bool several = false);
+                  std::string* err, const CoefPack& pack = CoefPack(), bool several = false,
+                  bool affine = false);
+bool elem_compile(const slx_instr* prog, int n_instr, bool fp64, const std::vector<int>& field_nff, const ElemShape& shape, bool several,
+                  hipFunction_t* fn, std::string* err);
+hipError_t elem_launch(hipFunction_t fn, const DevBucket& b, int64_t coff, const DevJob* jobs, int n_jobs, int max_elem, const DevInputs& in,
+                       void* cbase, void* ke, hipStream_t st);
 // Same launch contract as the interpreter's coefficient kernel.
 hipError_t coef_launch(hipFunction_t fn, const DevBucket& b, int64_t coff, const DevJob* jobs, int n_jobs, int max_elem, const DevInputs& in, int nq,
                        int qfast, void* cbase, hipStream_t st);

@@ -199,6 +199,7 @@ struct slx_plan_s {
     bool side_ok = false;              // every rhs slice lives in a rhs-only bucket
     // compiled coefficient programs per bucket ([0] FP32, [1] FP64; null: interpreter)
     std::vector<std::array<hipFunction_t, 2>> coef_fn;
+    std::vector<std::array<hipFunction_t, 2>> elem_fn;  // element kernels per bucket (program and contraction in one)
     int coef_mode = 0;                 // 0 auto, 1 interpreter only, 2 compiled everywhere
     std::string coef_jit_error;        // last compiler message (diagnostics)
     hipStream_t side = nullptr;
@@ -2053,8 +2054,46 @@ void upload_buckets(slx_plan_s& P, const slx_plan_desc& d, const KeLayout& L) {
 // interpreter's scratch registers cost the same per element whatever its
 // bucket); unique programs compiled in parallel.
 #define SLX_COEF_JIT_MIN 4096
+//
+// Element kernels: a bucket whose slices all run on the VALU element kernel in
+// every mode and fit one thread's registers (SLX_ELEM_MAX entries: P2
+// triangles, order-1 hexahedra and prisms, small right-hand sides) is computed
+// by one compiled kernel.  The last bucket also stores its coefficient table
+// there, which slx_plan_coefficients reads.  Measured against the program and
+// element kernels at 5e5 P2 triangles (whole assembly): 0.20 vs 0.51 ms.
+// SLX_TUNE_ELEM_FUSED=0 keeps the two kernels apart.
+// Constant Jacobian: lines, triangles and tetrahedra of order-1 geometry.
+bool elem_affine(const slx_bucket_desc& bd) {
+    return (bd.elem_type == 1 && bd.n_geo == 2) || (bd.elem_type == 2 && bd.n_geo == 3) || (bd.elem_type == 4 && bd.n_geo == 4);
+}
+
+bool elem_shape(const slx_plan_s& P, const slx_plan_desc& d, int b, ElemShape& shape) {
+    const slx_bucket_desc& bd = d.buckets[b];
+    if (const char* t = std::getenv("SLX_TUNE_ELEM_FUSED"))
+        if (std::atoi(t) == 0) return false;
+    if (P.direct && (b == P.direct_bucket || b == P.direct_rhs_bucket)) return false;
+    if (bd.n_slices == 0 || bd.n_coefs == 0 || bd.n_geo > SLX_MAX_GEO || P.mfma[b].M > 0 || !P.factor[b].empty() || !P.tile[b].empty()) return false;
+    shape = ElemShape();
+    int entries = 0;
+    for (int s = 0; s < bd.n_slices; s++) {
+        const slx_slice_desc& sd = bd.slices[s];
+        ElemShape::Slice sl;
+        sl.n_tf = sd.n_tf;
+        sl.n_dof = sd.is_rhs ? 0 : sd.n_dof;
+        sl.vec4 = !sd.is_rhs && P.dbuckets[b].slices[s].ke_base % 4 == 0 && P.dbuckets[b].slices[s].ke_ld % 4 == 0;
+        sl.terms.assign(sd.terms, sd.terms + sd.n_terms);
+        entries += sd.n_tf * std::max(sl.n_dof, 1);
+        shape.slices.push_back(sl);
+    }
+    shape.affine = elem_affine(bd);
+    shape.q_inv = bd.q_invariant != 0;
+    shape.store = b == d.n_buckets - 1;
+    return entries <= SLX_ELEM_MAX;
+}
+
 void compile_coef_programs(slx_plan_s& P, const slx_plan_desc& d) {
     P.coef_fn.assign(d.n_buckets, {nullptr, nullptr});
+    P.elem_fn.assign(d.n_buckets, {nullptr, nullptr});
     if (P.coef_mode == 1) return;
     std::vector<std::pair<int, int>> todo;  // (bucket, fp64)
     std::vector<int64_t> runs(d.n_buckets, 0);  // elements that run the bucket's program
@@ -2088,8 +2127,21 @@ void compile_coef_programs(slx_plan_s& P, const slx_plan_desc& d) {
                 bool several = false;
                 for (const auto& f : P.families)
                     several = several || (f.buckets.size() > 1 && std::find(f.buckets.begin(), f.buckets.end(), todo[i].first) != f.buckets.end());
+                ElemShape shape;
+                if (elem_shape(P, d, todo[i].first, shape)) {
+                    // one kernel per family: its last bucket's store is everyone's
+                    for (const auto& f : P.families)
+                        if (std::find(f.buckets.begin(), f.buckets.end(), todo[i].first) != f.buckets.end())
+                            shape.store = f.buckets.back() == d.n_buckets - 1;
+                    std::string eerr;
+                    hipFunction_t efn = nullptr;
+                    if (elem_compile(bd.prog, bd.n_instr, todo[i].second != 0, fnff, shape, several, &efn, &eerr))
+                        P.elem_fn[todo[i].first][todo[i].second] = efn;
+                }
+                const bool affine = elem_affine(bd);
+                if (P.elem_fn[todo[i].first][todo[i].second]) continue;
                 if (coef_compile(bd.prog, bd.n_instr, todo[i].second != 0, bd.q_invariant == 0, fnff, &fn, &err,
-                                 records ? P.pack : CoefPack(), several)) {
+                                        records ? P.pack : CoefPack(), several, affine)) {
                     P.coef_fn[todo[i].first][todo[i].second] = fn;
                 } else {
                     std::lock_guard<std::mutex> lk(mu);
@@ -2220,6 +2272,13 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
         if (f.buckets.back() + 1 == (int)P.dbuckets.size()) {
             P.last_qfast = qfast;
             P.last_ctab = (const char*)P.d_ctab.p + P.ctab_off.back();
+        }
+        const hipFunction_t efn = bi < P.elem_fn.size() ? P.elem_fn[bi][ke64 ? 1 : 0] : nullptr;
+        if (efn) {
+            if (tm) tm->begin(T_VALU);
+            HIPCHECK(elem_launch(efn, b, (int64_t)P.ctab_off[bi], f.jobs, nj, f.max_elem, in, P.d_ctab.p, P.d_ke.p, bst));
+            if (tm) tm->end();
+            continue;
         }
         if (!in_fused) coefficients(f, qfast, bst);
         if (records || (P.direct && (int)bi == P.direct_rhs_bucket)) continue;  // the row-wise launch does the rest
@@ -2942,7 +3001,8 @@ slx_status slx_plan_coef_mode(slx_plan p, int32_t mode, int32_t* n_compiled) {
             compile_coef_programs(*p, *p->src);
         }
         int n = 0;
-        for (auto& f : p->coef_fn) n += (f[0] ? 1 : 0) + (f[1] ? 1 : 0);
+        for (size_t b = 0; b < p->coef_fn.size(); b++)
+            for (int k = 0; k < 2; k++) n += p->coef_fn[b][k] || p->elem_fn[b][k] ? 1 : 0;
         if (n_compiled) *n_compiled = n;
         if (mode == 2) {
             int want = 0;
