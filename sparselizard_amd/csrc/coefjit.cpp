@@ -381,4 +381,88 @@ hipError_t coef_launch(hipFunction_t fn, const DevBucket& b, int64_t coff, const
     return hipModuleLaunchKernel(fn, (unsigned)((total + 255) / 256), (unsigned)n_jobs, 1, 256, 1, 1, 0, st, args, nullptr);
 }
 
+// Where the tables are kept and how many waves share them.  Registers: both
+// tables in at most 72 (1 x 1 tiles of up to 4 chunks), or the dof table in at most
+// 40 with P in LDS: more would leave fewer than three waves a SIMD.  The
+// registers that are held across the chunk loop then say how many waves a SIMD
+// takes (the compiler adds about 20 to 40; measured without scratch on 16 x 16 to
+// 64 x 64 slices).  LDS: as many workgroups of 4 or 8 waves as 144 KB hold (three
+// 53 KB groups of a CU don't start together), or one with the whole 160 KB.
+std::string tile_kernel_source(const TileSpec& s, TileKernel& k) {
+    const int nt = (int)s.term_a.size();
+    std::vector<int> bl, pa, pb, tp;
+    for (int b = 0; b < 4; b++)
+        if (std::find(s.term_b.begin(), s.term_b.end(), b) != s.term_b.end()) bl.push_back(b);
+    for (int t = 0; t < nt; t++) {
+        const int bi = (int)(std::find(bl.begin(), bl.end(), s.term_b[t]) - bl.begin());
+        int x = 0;
+        while (x < (int)pa.size() && (pa[x] != s.term_a[t] || pb[x] != bi)) x++;
+        if (x == (int)pa.size()) {
+            pa.push_back(s.term_a[t]);
+            pb.push_back(bi);
+        }
+        tp.push_back(x);
+    }
+    const int nb = (int)bl.size(), np = (int)pa.size(), qh = 8 / s.na, ngpp = s.nkc * 4 * qh, npl = s.arith == 1 ? 3 : 2;
+    const int hregs = s.nkc * s.ntt * qh * nb, pregs = s.nkc * s.mtt * npl * 4;
+    const bool preg = hregs + pregs <= 72, hreg = preg || hregs <= 40;
+    // four elements' coefficients at a time where they fit the registers and their
+    // rows the LDS beside eight waves' tables
+    const int cregs = (ngpp + 63) / 64 * nt;
+    const size_t tables = (size_t)(hreg ? 0 : hregs * 256) + (size_t)(preg ? 0 : pregs * 256), row = (size_t)np * ngpp * 4;
+    k.batch = cregs <= 9 && tables + 32 * row <= 72 * 1024 ? 4 : 1;
+    const int held = (preg ? pregs : s.mtt * npl * 4) + (hreg ? hregs : qh * nb) + s.mtt * s.ntt * 4 + npl * 4 + np * qh;
+    const int occ = held <= 110 ? 4 : held <= 124 ? 3 : 2;
+    const size_t wave = k.batch * row;
+    k.waves = 0;
+    for (int w : {4, 8}) {
+        const size_t need = tables + w * wave;
+        const int g = std::min<int>(4 * occ / w, (int)(144 * 1024 / need));
+        if (g >= 1 && w * g > k.waves * k.groups) {
+            k.waves = w;
+            k.groups = g;
+        }
+    }
+    if (k.waves * k.groups < 8 && tables + 8 * wave <= 160 * 1024) {
+        k.waves = 8;
+        k.groups = 1;
+    }
+    if (k.waves == 0) return std::string();
+    std::ostringstream o;
+    auto list = [&](const char* name, const std::vector<int>& v) {
+        o << "constexpr int " << name << "[] = {";
+        for (size_t i = 0; i < v.size(); i++) o << (i ? ", " : "") << v[i];
+        o << "};\n";
+    };
+    o << "#define TJ_ARG " << (s.several ? "const TileJob* __restrict__ jobs" : "TileJob job") << "\n#define TJ_JOB "
+      << (s.several ? "const TileJob& job = jobs[blockIdx.y]" : "") << "\nnamespace slx { namespace tj {\nconstexpr int AR = " << s.arith
+      << ", NA = " << s.na << ", NB = " << nb << ", NT = " << nt << ", NP = " << np << ", NKC = " << s.nkc << ", NGP = " << s.ngp << ", MTT = " << s.mtt
+      << ", NTT = " << s.ntt << ", N_TF = " << s.n_tf << ", N_DOF = " << s.n_dof << ", EB = " << k.batch << ", WAVES = " << k.waves
+      << ", OCC = " << occ << ";\nconstexpr bool H_REG = " << (hreg ? "true" : "false") << ", P_REG = " << (preg ? "true" : "false") << ";\n";
+    list("B_OF", bl);
+    list("PAIR_A", pa);
+    list("PAIR_B", pb);
+    list("TERM_PAIR", tp);
+    list("TERM_SLOT", s.term_slot);
+    o << "} }\n";
+    return std::string(kTilePrelude) + o.str() + kTileKernel;
+}
+
+bool tile_compile(const TileSpec& s, TileKernel* k, std::string* err) {
+    const std::string src = tile_kernel_source(s, *k);
+    k->fn = nullptr;
+    if (src.empty()) return false;  // the tables exceed the LDS
+    return compile_source(src, "slx_tile", &k->fn, err);
+}
+
+hipError_t tile_launch(const TileKernel& k, const TileJob& one, const TileJob* jobs, int n_jobs, int max_elem, const void* cbase, int qfast, float* ke,
+                       int n_cu, hipStream_t st) {
+    if (max_elem == 0 || n_jobs == 0) return hipSuccess;
+    TileJob job = one;
+    void* args[] = {n_jobs > 1 ? (void*)&jobs : (void*)&job, &cbase, &qfast, &ke};
+    const int step = k.waves * k.batch;
+    const int64_t groups = ((int64_t)max_elem + step - 1) / step, fit = ((int64_t)n_cu * k.groups + n_jobs - 1) / n_jobs;
+    return hipModuleLaunchKernel(k.fn, (unsigned)((std::min(groups, fit) + 7) / 8 * 8), (unsigned)n_jobs, 1, 64 * k.waves, 1, 1, 0, st, args, nullptr);
+}
+
 }  // namespace slx

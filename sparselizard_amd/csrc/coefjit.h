@@ -8,6 +8,7 @@
 #include <string>
 #include <vector>
 #include "kernels/device.h"
+#include "kernels/tile.h"
 
 namespace slx {
 
@@ -62,5 +63,23 @@ hipError_t elem_launch(hipFunction_t fn, const DevBucket& b, int64_t coff, const
 // Same launch contract as the interpreter's coefficient kernel.
 hipError_t coef_launch(hipFunction_t fn, const DevBucket& b, int64_t coff, const DevJob* jobs, int n_jobs, int max_elem, const DevInputs& in, int nq,
                        int qfast, void* cbase, hipStream_t st);
+
+// One slice's tile kernel (kernels/tile_jit.h).
+struct TileSpec {
+    int arith;                        // 0 FP16 split, 1 BF16 split, 2 FP32
+    int na, nkc, ngp, mtt, ntt, n_tf, n_dof;
+    std::vector<int> term_a, term_b, term_slot;  // index of the tf derivative, dof derivative, coefficient slot
+    bool several;
+};
+struct TileKernel {
+    hipFunction_t fn = nullptr;
+    int waves = 0, groups = 0;        // waves of a workgroup, workgroups on a CU
+    int batch = 1;                    // elements whose coefficients a wave loads at once
+};
+// Source of the kernel and its launch shape; empty when its tables don't fit.
+std::string tile_kernel_source(const TileSpec& spec, TileKernel& k);
+bool tile_compile(const TileSpec& spec, TileKernel* k, std::string* err);
+hipError_t tile_launch(const TileKernel& k, const TileJob& one, const TileJob* jobs, int n_jobs, int max_elem, const void* cbase, int qfast, float* ke,
+                       int n_cu, hipStream_t st);
 
 }  // namespace slx

@@ -52,6 +52,7 @@ struct TileJob {
     int64_t n_elem, coff;           // elements; bytes of the coefficients from the tables' base
 };
 
+#ifndef SLX_RUNTIME_COMPILED
 size_t tile_lds_bytes(const TileSlice& t, int planes);
 // Element matrices of one slice of n_jobs buckets that agree in its shape
 // (one: the first of them, max_elem: the largest's elements; coefficient tables
@@ -59,5 +60,6 @@ size_t tile_lds_bytes(const TileSlice& t, int planes);
 // arith: 0 FP16 split, 1 BF16 split, 2 FP32.
 hipError_t launch_tile(const TileJob& one, const TileJob* jobs, int n_jobs, int max_elem, int arith, const void* cbase, int qfast, float* ke,
                        int n_cu, hipStream_t st);
+#endif
 
 }  // namespace slx

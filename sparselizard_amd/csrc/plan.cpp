@@ -213,6 +213,7 @@ struct slx_plan_s {
         int max_elem = 0;
         const DevJob* jobs = nullptr;  // device
         std::vector<std::pair<int, std::array<const TileJob*, 3>>> tile;  // (slice, jobs per arithmetic)
+        std::vector<std::array<TileKernel, 3>> tile_fn;                   // kernels compiled for the slice, per arithmetic
     };
     std::vector<Family> families;      // in the order of their first buckets
     std::vector<MfmaBucket> mfma;      // per bucket; M == 0 when not eligible
@@ -1832,6 +1833,7 @@ void build_families(slx_plan_s& P, const slx_plan_desc& d) {
         f->max_elem = std::max(f->max_elem, d.buckets[b].n_elem);
     }
     for (auto& f : P.families) {
+        f.tile_fn.assign(P.tile[f.buckets[0]].size(), {});
         std::vector<DevJob> jobs;
         for (int b : f.buckets) jobs.push_back(DevJob{P.dbuckets[b], (int64_t)P.ctab_off[b]});
         f.jobs = P.dev(jobs.data(), jobs.size());
@@ -2094,6 +2096,7 @@ bool elem_shape(const slx_plan_s& P, const slx_plan_desc& d, int b, ElemShape& s
 void compile_coef_programs(slx_plan_s& P, const slx_plan_desc& d) {
     P.coef_fn.assign(d.n_buckets, {nullptr, nullptr});
     P.elem_fn.assign(d.n_buckets, {nullptr, nullptr});
+    for (auto& f : P.families) f.tile_fn.assign(f.tile.size(), {});
     if (P.coef_mode == 1) return;
     std::vector<std::pair<int, int>> todo;  // (bucket, fp64)
     std::vector<int64_t> runs(d.n_buckets, 0);  // elements that run the bucket's program
@@ -2110,13 +2113,47 @@ void compile_coef_programs(slx_plan_s& P, const slx_plan_desc& d) {
         todo.push_back({b, 0});
         todo.push_back({b, 1});
     }
+    // Tile kernels of the same families, under the same rule.  Slices whose tables
+    // exceed the LDS and smaller launches keep the general kernel (tile.hip).
+    // SLX_TUNE_TILE_JIT=0: all of them.
+    struct TileTodo {
+        slx_plan_s::Family* f;
+        size_t k;
+        int arith;
+    };
+    std::vector<TileTodo> tiles;
+    const char* tj = std::getenv("SLX_TUNE_TILE_JIT");
+    for (auto& f : P.families)
+        for (size_t k = 0; k < f.tile.size(); k++)
+            if ((P.coef_mode != 0 || runs[f.buckets[0]] >= SLX_COEF_JIT_MIN) && !(tj && std::atoi(tj) == 0))
+                for (int ar = 0; ar < 3; ar++) tiles.push_back({&f, k, ar});
     std::mutex mu;
     std::vector<std::thread> th;
     const int device = P.ctx->device;
-    const size_t nth = std::min<size_t>(todo.size(), 8);
+    const size_t nth = std::min<size_t>(todo.size() + tiles.size(), 8);
     for (size_t t = 0; t < nth; t++)
         th.emplace_back([&, t]() {
             (void)hipSetDevice(device);
+            for (size_t i = t; i < tiles.size(); i += nth) {
+                const TileTodo& td = tiles[i];
+                const int b0 = td.f->buckets[0];
+                const TileSlice& ts = P.tile[b0][td.k].second;
+                const slx_slice_desc& sd = d.buckets[b0].slices[td.f->tile[td.k].first];
+                TileSpec spec{td.arith, ts.na, ts.nkc, ts.ngp, ts.mtt, ts.ntt, ts.n_tf, ts.n_dof, {}, {}, {}, td.f->buckets.size() > 1};
+                std::vector<int> al;
+                for (int k = 0; k < sd.n_terms; k++) al.push_back(sd.terms[k].tf_deriv);
+                std::sort(al.begin(), al.end());
+                al.erase(std::unique(al.begin(), al.end()), al.end());
+                for (int k = 0; k < sd.n_terms; k++) {
+                    spec.term_a.push_back((int)(std::find(al.begin(), al.end(), sd.terms[k].tf_deriv) - al.begin()));
+                    spec.term_b.push_back(sd.terms[k].dof_deriv);
+                    spec.term_slot.push_back(sd.terms[k].coef);
+                }
+                std::string err;
+                TileKernel tk;
+                if (tile_compile(spec, &tk, &err)) td.f->tile_fn[td.k][td.arith] = tk;
+                else if (!err.empty()) std::fprintf(stderr, "tile kernel not compiled, the general one runs: %s\n", err.c_str());
+            }
             for (size_t i = t; i < todo.size(); i += nth) {
                 const slx_bucket_desc& bd = d.buckets[todo[i].first];
                 std::vector<int> fnff(d.n_fields);
@@ -2310,7 +2347,11 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
                 if ((tmask >> f.tile[k].first) & 1u) {
                     TileJob one{P.tile[bi][k].second, b.n_elem, (int64_t)P.ctab_off[bi]};
                     one.t.afrag = one.t.afrag_x[ar];
-                    HIPCHECK(launch_tile(one, f.tile[k].second[ar], nj, f.max_elem, ar, P.d_ctab.p, qfast, P.d_ke.as<float>(), P.n_cu, bst));
+                    const TileKernel& tk = f.tile_fn[k][ar];
+                    if (tk.fn)
+                        HIPCHECK(tile_launch(tk, one, f.tile[k].second[ar], nj, f.max_elem, P.d_ctab.p, qfast, P.d_ke.as<float>(), P.n_cu, bst));
+                    else
+                        HIPCHECK(launch_tile(one, f.tile[k].second[ar], nj, f.max_elem, ar, P.d_ctab.p, qfast, P.d_ke.as<float>(), P.n_cu, bst));
                 }
             if (tm) tm->end();
             done |= tmask;
