@@ -437,7 +437,7 @@ std::string tile_kernel_source(const TileSpec& s, TileKernel& k) {
     o << "#define TJ_ARG " << (s.several ? "const TileJob* __restrict__ jobs" : "TileJob job") << "\n#define TJ_JOB "
       << (s.several ? "const TileJob& job = jobs[blockIdx.y]" : "") << "\nnamespace slx { namespace tj {\nconstexpr int AR = " << s.arith
       << ", NA = " << s.na << ", NB = " << nb << ", NT = " << nt << ", NP = " << np << ", NKC = " << s.nkc << ", NGP = " << s.ngp << ", MTT = " << s.mtt
-      << ", NTT = " << s.ntt << ", N_TF = " << s.n_tf << ", N_DOF = " << s.n_dof << ", EB = " << k.batch << ", WAVES = " << k.waves
+      << ", NTT = " << s.ntt << ", N_TF = " << s.n_tf << ", N_STORE = " << s.n_store << ", EB = " << k.batch << ", WAVES = " << k.waves
       << ", OCC = " << occ << ";\nconstexpr bool H_REG = " << (hreg ? "true" : "false") << ", P_REG = " << (preg ? "true" : "false") << ";\n";
     list("B_OF", bl);
     list("PAIR_A", pa);

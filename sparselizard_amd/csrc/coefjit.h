@@ -68,6 +68,7 @@ hipError_t coef_launch(hipFunction_t fn, const DevBucket& b, int64_t coff, const
 struct TileSpec {
     int arith;                        // 0 FP16 split, 1 BF16 split, 2 FP32
     int na, nkc, ngp, mtt, ntt, n_tf, n_dof;
+    int n_store;                      // columns stored: n_dof, or more where the rows' padding may be written
     std::vector<int> term_a, term_b, term_slot;  // index of the tf derivative, dof derivative, coefficient slot
     bool several;
 };

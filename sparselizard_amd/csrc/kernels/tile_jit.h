@@ -13,9 +13,12 @@
 // and products in the same order.  Measured, tile.hip -> here: 5.5e5 order-3
 // quadrangles FP16 split 634 -> 313 us (EB = 1: 430); 1.6e4 order-3 prisms BF16 split,
 // stiffness 222 -> 164 us, mass 158 -> 48 us; 48000 order-2 H(curl) tetrahedra in 24
-// buckets 130 -> 92 us.  Rows of whole lines (16 columns) are stored past the caches
-// (quadrangles 320 us, else 342); others not, since their pieces of a line meet in
-// L2 (mass matrices of prisms 48 us, else 67; H(curl) 97, else 189).
+// buckets 130 -> 82 us.
+// N_STORE: the columns or, where no other slice shares the rows, with the padding
+// up to ld (zeros).  Rows of whole lines are stored past the caches (quadrangles
+// 320 us, else 342; H(curl) 82 us, else 92, and the reduction 165 us, else 205);
+// others not, since their pieces of a line meet in L2 (mass matrices of prisms
+// 48 us, else 67).
 namespace slx {
 
 typedef _Float16 tj_half2 __attribute__((ext_vector_type(2)));
@@ -327,13 +330,13 @@ extern "C" __global__ void __launch_bounds__(64 * tj::WAVES, tj::OCC)
                     const int i = mt * 16 + jl, j = jt * 16 + 4 * g;
                     float* o = out + i * ld + j;
                     if (i < N_TF) {
-                        if (j + 4 <= N_DOF) {
-                            if constexpr (N_DOF % 16 == 0) __builtin_nontemporal_store(v, reinterpret_cast<tj_f4u*>(o));
+                        if (j + 4 <= N_STORE) {
+                            if constexpr (N_STORE % 16 == 0) __builtin_nontemporal_store(v, reinterpret_cast<tj_f4u*>(o));
                             else *reinterpret_cast<tj_f4u*>(o) = v;
                         } else {
 #pragma unroll
                             for (int r = 0; r < 4; r++)
-                                if (j + r < N_DOF) o[r] = v[r];
+                                if (j + r < N_STORE) o[r] = v[r];
                         }
                     }
                 }

@@ -2139,7 +2139,15 @@ void compile_coef_programs(slx_plan_s& P, const slx_plan_desc& d) {
                 const int b0 = td.f->buckets[0];
                 const TileSlice& ts = P.tile[b0][td.k].second;
                 const slx_slice_desc& sd = d.buckets[b0].slices[td.f->tile[td.k].first];
-                TileSpec spec{td.arith, ts.na, ts.nkc, ts.ngp, ts.mtt, ts.ntt, ts.n_tf, ts.n_dof, {}, {}, {}, td.f->buckets.size() > 1};
+                TileSpec spec{td.arith, ts.na, ts.nkc, ts.ngp, ts.mtt, ts.ntt, ts.n_tf, ts.n_dof, ts.n_dof, {}, {}, {}, td.f->buckets.size() > 1};
+                bool alone = true;  // no other slice's columns in the rows, whose padding then may be written
+                for (int b : td.f->buckets) {
+                    const int64_t base = P.tile[b][td.k].second.ke_base, ld = P.tile[b][td.k].second.ke_ld;
+                    alone = alone && ld == ts.ke_ld;
+                    for (int s = 0; s < d.buckets[b].n_slices; s++)
+                        if (s != td.f->tile[td.k].first) alone = alone && std::llabs((long long)(P.dbuckets[b].slices[s].ke_base - base)) >= ld;
+                }
+                if (alone) spec.n_store = (int)std::min<int64_t>(16 * ts.ntt, ts.ke_ld);
                 std::vector<int> al;
                 for (int k = 0; k < sd.n_terms; k++) al.push_back(sd.terms[k].tf_deriv);
                 std::sort(al.begin(), al.end());
