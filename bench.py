@@ -246,9 +246,15 @@ def main():
                     "kernel_ms": round(t_contract, 4), "algorithmic": con_bytes,
                     "mfma_tflops": round(flops / (t_contract * 1e-3) / 1e12, 3)}
     else:
+        # constant coefficients and no contraction launch: the row-wise kernel
+        # assembles straight into the CSR values, without element matrices
+        rowwise = prof_mix["mfma"] == 0 and all(d.buckets[b].q_invariant for b in range(d.n_buckets)
+                                                if any(not d.buckets[b].slices[s_].is_rhs for s_ in range(d.buckets[b].n_slices)))
+        if rowwise:
+            ke_roundtrip = 0
         achieved = red_bytes / (prof_mix["reduce"] * 1e-3) / 1e9
         roof = {"bound": "hbm", "achieved": round(achieved, 2), "peak": PEAKS["hbm_GBps"], "unit": "GB/s",
-                "frac": round(achieved / PEAKS["hbm_GBps"], 5), "traffic": None, "kernel": "reduce_rows",
+                "frac": round(achieved / PEAKS["hbm_GBps"], 5), "traffic": None, "kernel": "direct_rows" if rowwise else "reduce_rows",
                 "kernel_ms": round(prof_mix["reduce"], 4), "algorithmic": red_bytes,
                 "ke_roundtrip_bytes": ke_roundtrip}
     traffic_file = os.path.join(ROOT, "profiles", "traffic.json")

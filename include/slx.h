@@ -47,6 +47,8 @@ typedef int32_t slx_status;
  * accumulation, and everything else on the FP32 VALU element kernel; the
  * CSR reduction is FP64 in every mode.  The FP16 split also takes the batched
  * kernel for Gauss-point-varying coefficients when the table says so. */
+/* Constant-coefficient matrices of simplices are assembled row by row without
+ * element matrices: in FP64 in SLX_PREC_FP64, else in FP32 products summed in FP64. */
 #define SLX_PREC_FP64 0        /* plain FP64 element kernel (FP64 everywhere) */
 #define SLX_PREC_F16_SPLIT 1   /* FP16 hi/lo split MFMA (3 products), FP32 accumulation, FP64 reduction */
 #define SLX_PREC_BF16_SPLIT 2  /* BF16 hi/mid/lo split MFMA (6 products), FP32 accumulation, FP64 reduction */

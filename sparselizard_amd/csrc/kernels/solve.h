@@ -1,5 +1,6 @@
 // Device solve of an assembled system: FP64 iterative refinement around a
-// Jacobi-preconditioned FP32 conjugate-gradient inner solve (SPD systems).
+// Jacobi-preconditioned FP32 inner solve: conjugate gradients (SPD systems) or
+// GMRES.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cstdint>

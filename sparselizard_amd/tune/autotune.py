@@ -125,7 +125,8 @@ def main():
                 with tempfile.NamedTemporaryFile("w", suffix=".txt", delete=False) as f:
                     f.write("%d %d %d %d %s %d %d\n" % (c + (kern, mtw, var)))
                     tab = f.name
-                env = dict(os.environ, SLX_TUNE_TABLE=tab)
+                # the kernels that the table chooses between, without those that take the bucket before it is read
+                env = dict(os.environ, SLX_TUNE_TABLE=tab, SLX_TUNE_DIRECT="0", SLX_TUNE_ELEM_FUSED="0")
                 print("tuning %s %s class %s: %s mtw %d variant %d" % (kind, spec, c, kern, mtw, var), flush=True)
                 r = subprocess.run([sys.executable, __file__, "--child", kind, spec, "--iters", str(args.iters)],
                                    env=env, capture_output=True, text=True, timeout=600)
