@@ -307,7 +307,7 @@ slx_status slx_plan_eliminate(slx_plan plan, const double* b, double* out);
  * x, y: n_dofs entries in DOF numbering, host memory. */
 slx_status slx_plan_matvec(slx_plan plan, const double* x, double* y);
 /* Coefficient programs: 0 (auto, the default) compiles the program of every
- * bucket of at least 4096 elements at plan creation into its own kernel
+ * bucket whose program at least 512 elements run at plan creation into its own kernel
  * (hipRTC; values in registers instead of the interpreter's scratch register
  * file; the same arithmetic, results equal to rounding), 1 uses the
  * interpreter everywhere, 2

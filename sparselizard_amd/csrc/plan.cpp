@@ -2054,8 +2054,11 @@ void upload_buckets(slx_plan_s& P, const slx_plan_desc& d, const KeLayout& L) {
 // Compiled coefficient programs for the buckets the mode selects (auto: programs
 // that at least SLX_COEF_JIT_MIN elements run, over all buckets: the
 // interpreter's scratch registers cost the same per element whatever its
-// bucket); unique programs compiled in parallel.
-#define SLX_COEF_JIT_MIN 4096
+// bucket); unique programs compiled in parallel.  At 4096 hp Poisson 9^3 (729
+// hexahedra, orders 1 to 5) took 565 us a call on the interpreter and the general
+// kernels, at 512 443 us; P2 elasticity on 750 tetrahedra 115 and 22 us.  Below,
+// the calls are launches and the compiler's half second is not earned back.
+#define SLX_COEF_JIT_MIN 512
 //
 // Element kernels: a bucket whose slices all run on the VALU element kernel in
 // every mode and fit one thread's registers (SLX_ELEM_MAX entries: P2

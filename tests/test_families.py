@@ -1,6 +1,6 @@
 """Launches shared by the orientation buckets of one element type (24 tetrahedra
 orientations at most) against the oracle: interpreted and compiled programs
-(4096 elements and more over all buckets), every kernel of the family (one-tile,
+(512 elements and more over all buckets), every kernel of the family (one-tile,
 VALU element kernel, FP64, right-hand sides)."""
 import numpy as np
 import pytest
