@@ -304,7 +304,9 @@ __global__ void __launch_bounds__((256 * direct_waves<KT, NB, P>()), (direct_wav
                         put(a, dd, lane + 64 * h, v[y][h]);
                         if (lane + 64 * h < acc_stride) ar[lane + 64 * h] = 0.0;
                     }
-                    for (int x = lane + 128; x < len; x += 64) {
+                    // and the spare entry behind them, which takes the absent columns
+                    // and may be a column of the next row in this accumulator
+                    for (int x = lane + 128; x <= len; x += 64) {
                         put(a, dd, x, ar[x]);
                         ar[x] = 0.0;
                     }
