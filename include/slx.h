@@ -360,6 +360,9 @@ slx_status slx_selftest_mfma_layout_kind(slx_ctx ctx, int32_t kind, float* out25
  * y = A x and xy = x . y (FP64 sum of the FP32 products). */
 slx_status slx_selftest_spmv_stream(slx_ctx ctx, int64_t nrows, const int64_t* rowp, const int32_t* col,
                                     const double* val, const double* x, double* y, double* xy);
+/* Test hook: a device allocation of more bytes than any device has; *kept = the
+ * size that the buffer claims to hold after the failure (0). */
+slx_status slx_selftest_failed_alloc(int64_t bytes, int64_t* kept);
 
 /* ---- Reference tables ------------------------------------------------------
  * gausspoints(type, order) (src/gausspoint/gausspoints.cpp:4-54): writes up to

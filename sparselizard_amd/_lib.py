@@ -120,6 +120,7 @@ def lib():
         "slx_plan_coef_mode": (i32, [vp, i32, p32]),
         "slx_plan_matvec": (i32, [vp, pd, pd]),
         "slx_selftest_spmv_stream": (i32, [vp, i64, p64, p32, pd, pd, pd, pd]),
+        "slx_selftest_failed_alloc": (i32, [i64, p64]),
         "slx_plan_element_matrices": (i32, [vp, pd, i64]),
         "slx_plan_coefficients": (i32, [vp, pd, i64, p64]),
         "slx_plan_reduction_maps": (i32, [vp, p64, p64, C.POINTER(C.c_uint64), p64, p32, p64, C.POINTER(C.c_uint64), p64, p64]),
@@ -159,7 +160,7 @@ EXPORTED = [
     "slx_problem_generate", "slx_problem_info", "slx_problem_desc", "slx_problem_setdata", "slx_problem_setdata_vec",
     "slx_plan_graph_capture", "slx_plan_graph_launch",
     "slx_gauss_rule", "slx_h1_count", "slx_h1_tables", "slx_geometry_tables", "slx_hcurl_count", "slx_hcurl_tables", "slx_selftest_mfma_layout", "slx_selftest_mfma_layout_kind",
-    "slx_selftest_spmv_stream",
+    "slx_selftest_spmv_stream", "slx_selftest_failed_alloc",
 ]
 
 

@@ -89,8 +89,11 @@ struct DBuf {
     void alloc(size_t bytes) {
         if (p) (void)hipFree(p);
         p = nullptr;
+        n = 0;  // until the allocation has succeeded: buffers are reused by their size
+        void* q = nullptr;
+        if (bytes) HIPCHECK(hipMalloc(&q, bytes));
+        p = q;
         n = bytes;
-        if (bytes) HIPCHECK(hipMalloc(&p, bytes));
     }
     // take over a hipMalloc'd allocation
     void adopt(void* ptr, size_t bytes) {
@@ -3136,6 +3139,21 @@ slx_status slx_selftest_spmv_stream(slx_ctx ctx, int64_t nrows, const int64_t* r
         HIPCHECK(hipMemcpy(y32.data(), dy.p, nrows * sizeof(float), hipMemcpyDeviceToHost));
         HIPCHECK(hipMemcpy(xy, dpart.as<double>() + SLX_SOLVE_BLOCKS + 1, sizeof(double), hipMemcpyDeviceToHost));
         std::copy(y32.begin(), y32.end(), y);
+    });
+}
+
+slx_status slx_selftest_failed_alloc(int64_t bytes, int64_t* kept) {
+    return guarded([&] {
+        SLX_CHECK(kept && bytes > 0, "null argument");
+        DBuf b;
+        bool failed = false;
+        try {
+            b.alloc((size_t)bytes);
+        } catch (const DeviceError&) {
+            failed = true;
+        }
+        SLX_CHECK(failed, "an allocation of " << bytes << " bytes succeeded");
+        *kept = b.p ? -1 : (int64_t)b.n;
     });
 }
 

@@ -53,6 +53,14 @@ def test_error_status_and_message():
         sa.Problem(None, "msh", "file=/nonexistent.msh")
 
 
+def test_failed_allocation_keeps_no_size():
+    # the solve reuses its workspace when it is large enough: a buffer whose allocation
+    # failed must not look like one (2^60 bytes; without a device every allocation fails)
+    kept = C.c_int64(-1)
+    L.check(L.lib().slx_selftest_failed_alloc(1 << 60, C.byref(kept)))
+    assert kept.value == 0
+
+
 def test_negative_integration_order_rejected(tmp_path):
     msh = write_msh(tmp_path / "one.msh", [(0, 0), (1, 0), (0, 1)], [(TRI, 1, (1, 2, 3))])
     with pytest.raises(sa.SlxError, match="negative order"):
