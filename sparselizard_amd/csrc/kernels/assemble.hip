@@ -124,11 +124,12 @@ __device__ void run_program(const DevBucket& b, const DevInputs& in, const int (
 // Coefficient table of one bucket (nq = 1 when the coefficients do not vary
 // over the Gauss points); each thread takes V consecutive (element, Gauss
 // point) pairs, element fastest.
-template <typename T, int V>
-__global__ void __launch_bounds__(256) coef_kernel(const DevJob* __restrict__ jobs, DevInputs in, int nq, int qfast, DevPack pk,
+template <typename T, int V, bool MULTI>
+__global__ void __launch_bounds__(256) coef_kernel(DevJob one, const DevJob* __restrict__ jobs, DevInputs in, int nq, int qfast, DevPack pk,
                                                    unsigned char* __restrict__ cbase) {
-    const DevBucket& b = jobs[blockIdx.y].b;
-    T* ctab = reinterpret_cast<T*>(cbase + jobs[blockIdx.y].coff);
+    const DevJob& job = MULTI ? jobs[blockIdx.y] : one;
+    const DevBucket& b = job.b;
+    T* ctab = reinterpret_cast<T*>(cbase + job.coff);
     const int64_t total = (int64_t)b.n_elem * nq;
     const int64_t idx0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * V;
     if (idx0 >= total) return;
@@ -163,11 +164,12 @@ __global__ void __launch_bounds__(256) coef_kernel(const DevJob* __restrict__ jo
 //   h_r     = w_q sum_s D_rs dof_s[j][q]
 //   Ke[i][j] += sum_r tf_r[i][q] h_r        (TI rows per pass)
 // which is the reference's sum over terms and Gauss points regrouped.
-template <typename CT, int TI, bool QV, bool COOP>
-__global__ void __launch_bounds__(256) elem_cols(const DevJob* __restrict__ jobs, const unsigned char* __restrict__ cbase, uint32_t slice_mask,
-                                                 int jc, int qfast, CT* __restrict__ ke) {
-    const DevBucket& b = jobs[blockIdx.y].b;
-    const CT* ctab = reinterpret_cast<const CT*>(cbase + jobs[blockIdx.y].coff);
+template <typename CT, int TI, bool QV, bool COOP, bool MULTI>
+__global__ void __launch_bounds__(256) elem_cols(DevJob one, const DevJob* __restrict__ jobs, const unsigned char* __restrict__ cbase,
+                                                 uint32_t slice_mask, int jc, int qfast, CT* __restrict__ ke) {
+    const DevJob& job = MULTI ? jobs[blockIdx.y] : one;
+    const DevBucket& b = job.b;
+    const CT* ctab = reinterpret_cast<const CT*>(cbase + job.coff);
     const int n_elem = b.n_elem, n_slices = b.n_slices;
     // QV with COOP: the block's coefficients of the current slice, staged once
     // in LDS ([element][term][q]) and read from there by the element's lanes
@@ -583,31 +585,45 @@ __global__ void reduce_rhs(DevReduce rd, const KT* __restrict__ ke, double* __re
 
 // ---------------------------------------------------------------- launchers --
 
-// b: one of the launch's buckets (they agree but for their elements), max_elem
-// the largest's elements.
-hipError_t launch_coef(const DevBucket& b, const DevJob* jobs, int n_jobs, int max_elem, const DevInputs& in, bool fp64, void* cbase,
+// one: a bucket of the launch (they agree but for their elements), by value
+// where it is the only one: the interpreter reads the description for every
+// instruction, and through memory one launch took 12 to 28 us more (P2
+// elasticity 162 elements 145 vs 170 us, orders 1 to 5 of 64 hexahedra 337 vs
+// 395 us an assembly).  max_elem: the largest bucket's elements.
+hipError_t launch_coef(const DevJob& one, const DevJob* jobs, int n_jobs, int max_elem, const DevInputs& in, bool fp64, void* cbase,
                        hipStream_t st, int qfast, const DevPack& pk) {
+    const DevBucket& b = one.b;
     if (max_elem == 0 || b.n_coefs == 0) return hipSuccess;
     const int nq = b.q_inv ? 1 : b.n_gp;
     const int64_t n = (int64_t)max_elem * nq;
+    unsigned char* cb = (unsigned char*)cbase;
+#define SLX_COEF_GO(T_, V_, M_) \
+    hipLaunchKernelGGL((coef_kernel<T_, V_, M_>), dim3((unsigned)((n + V_ * 256 - 1) / (V_ * 256)), n_jobs), dim3(256), 0, st, one, jobs, in, nq, qfast, pk, cb)
     if (fp64) {
-        const unsigned grid = (unsigned)((n + 2 * 256 - 1) / (2 * 256));
-        hipLaunchKernelGGL((coef_kernel<double, 2>), dim3(grid, n_jobs), dim3(256), 0, st, jobs, in, nq, qfast, pk, (unsigned char*)cbase);
+        if (n_jobs > 1) SLX_COEF_GO(double, 2, true);
+        else SLX_COEF_GO(double, 2, false);
     } else {
-        const unsigned grid = (unsigned)((n + 4 * 256 - 1) / (4 * 256));
-        hipLaunchKernelGGL((coef_kernel<float, 4>), dim3(grid, n_jobs), dim3(256), 0, st, jobs, in, nq, qfast, pk, (unsigned char*)cbase);
+        if (n_jobs > 1) SLX_COEF_GO(float, 4, true);
+        else SLX_COEF_GO(float, 4, false);
     }
+#undef SLX_COEF_GO
     return hipGetLastError();
 }
 
 template <typename CT, int TI>
-static void launch_cols(const DevBucket& b, const DevJob* jobs, int n_jobs, int max_elem, const void* cbase, uint32_t mask, int jc, int qfast,
+static void launch_cols(const DevJob& one, const DevJob* jobs, int n_jobs, int max_elem, const void* cbase, uint32_t mask, int jc, int qfast,
                         void* ke, hipStream_t st) {
+    const DevBucket& b = one.b;
     const unsigned char* cb = (const unsigned char*)cbase;
     const int epb = 256 / jc;
     const dim3 grid((unsigned)((max_elem + epb - 1) / epb), n_jobs);
+#define SLX_COLS_GO(QV_, COOP_, LDS_)                                                                                                       \
+    do {                                                                                                                                    \
+        if (n_jobs > 1) hipLaunchKernelGGL((elem_cols<CT, TI, QV_, COOP_, true>), grid, dim3(256), LDS_, st, one, jobs, cb, mask, jc, qfast, (CT*)ke); \
+        else hipLaunchKernelGGL((elem_cols<CT, TI, QV_, COOP_, false>), grid, dim3(256), LDS_, st, one, jobs, cb, mask, jc, qfast, (CT*)ke); \
+    } while (0)
     if (b.q_inv) {
-        hipLaunchKernelGGL((elem_cols<CT, TI, false, false>), grid, dim3(256), 0, st, jobs, cb, mask, jc, qfast, (CT*)ke);
+        SLX_COLS_GO(false, false, 0);
     } else {
         // stage the block's coefficients in LDS when they fit under the limit
         // (SLX_TUNE_ELEM_LDS_MAX bytes): a larger stage lowers the blocks a CU
@@ -618,16 +634,16 @@ static void launch_cols(const DevBucket& b, const DevJob* jobs, int n_jobs, int 
         const size_t bytes = (size_t)epb * maxt * b.n_gp * sizeof(CT);
         size_t lim = 48 * 1024;
         if (const char* t = std::getenv("SLX_TUNE_ELEM_LDS_MAX")) lim = (size_t)std::min(48L * 1024, std::max(0L, std::atol(t)));
-        if (bytes <= lim)
-            hipLaunchKernelGGL((elem_cols<CT, TI, true, true>), grid, dim3(256), bytes, st, jobs, cb, mask, jc, qfast, (CT*)ke);
-        else
-            hipLaunchKernelGGL((elem_cols<CT, TI, true, false>), grid, dim3(256), 0, st, jobs, cb, mask, jc, qfast, (CT*)ke);
+        if (bytes <= lim) SLX_COLS_GO(true, true, bytes);
+        else SLX_COLS_GO(true, false, 0);
     }
+#undef SLX_COLS_GO
 }
 
 template <typename CT>
-static void launch_cols_any(const DevBucket& b, const DevJob* jobs, int n_jobs, int max_elem, const void* cbase, uint32_t mask, int qfast, void* ke,
+static void launch_cols_any(const DevJob& one, const DevJob* jobs, int n_jobs, int max_elem, const void* cbase, uint32_t mask, int qfast, void* ke,
                             hipStream_t st) {
+    const DevBucket& b = one.b;
     int ntf = 1, ndof = 1;
     for (int s = 0; s < b.n_slices; s++)
         if ((mask >> s) & 1u) {
@@ -635,10 +651,10 @@ static void launch_cols_any(const DevBucket& b, const DevJob* jobs, int n_jobs, 
             ndof = max(ndof, b.slices[s].n_dof);
         }
     const int jc = min(ndof, 64);
-    if (ntf <= 4) launch_cols<CT, 4>(b, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, st);
-    else if (ntf <= 8) launch_cols<CT, 8>(b, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, st);
-    else if (ntf <= 10) launch_cols<CT, 10>(b, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, st);
-    else launch_cols<CT, 16>(b, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, st);
+    if (ntf <= 4) launch_cols<CT, 4>(one, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, st);
+    else if (ntf <= 8) launch_cols<CT, 8>(one, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, st);
+    else if (ntf <= 10) launch_cols<CT, 10>(one, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, st);
+    else launch_cols<CT, 16>(one, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, st);
 }
 
 // Right-hand-side slices with many tf functions, as a blocked product over
@@ -651,11 +667,12 @@ static void launch_cols_any(const DevBucket& b, const DevJob* jobs, int n_jobs, 
 template <typename CT>
 struct RhsVec4 { typedef CT type __attribute__((ext_vector_type(4))); };
 
-template <typename CT>
-__global__ void __launch_bounds__(256) rhs_tiles(const DevJob* __restrict__ jobs, const unsigned char* __restrict__ cbase, int s, int qfast,
-                                                 CT* __restrict__ ke) {
-    const DevBucket& b = jobs[blockIdx.z].b;
-    const CT* ctab = reinterpret_cast<const CT*>(cbase + jobs[blockIdx.z].coff);
+template <typename CT, bool MULTI>
+__global__ void __launch_bounds__(256) rhs_tiles(DevJob one, const DevJob* __restrict__ jobs, const unsigned char* __restrict__ cbase, int s,
+                                                 int qfast, CT* __restrict__ ke) {
+    const DevJob& job = MULTI ? jobs[blockIdx.z] : one;
+    const DevBucket& b = job.b;
+    const CT* ctab = reinterpret_cast<const CT*>(cbase + job.coff);
     constexpr int RB = 64, EB = 64, RQ = 16;
     typedef typename RhsVec4<CT>::type CT4;
     __shared__ __attribute__((aligned(32))) CT Ts[RQ][RB];  // table values of the chunk, [Gauss point][row]
@@ -729,8 +746,9 @@ __global__ void __launch_bounds__(256) rhs_tiles(const DevJob* __restrict__ jobs
     }
 }
 
-hipError_t launch_elem(const DevBucket& b, const DevJob* jobs, int n_jobs, int max_elem, const void* cbase, int precision, void* ke,
+hipError_t launch_elem(const DevJob& one, const DevJob* jobs, int n_jobs, int max_elem, const void* cbase, int precision, void* ke,
                        hipStream_t st, uint32_t slice_mask, int qfast) {
+    const DevBucket& b = one.b;
     if (max_elem == 0 || slice_mask == 0) return hipSuccess;
     // right-hand sides with more tf functions than one column pass of elem_cols
     // covers go to the tiled kernel
@@ -740,17 +758,23 @@ hipError_t launch_elem(const DevBucket& b, const DevJob* jobs, int n_jobs, int m
     const uint32_t mat_mask = slice_mask & ~rhs_mask;
     if (mat_mask) {
         if (precision == SLX_PREC_FP64)
-            launch_cols_any<double>(b, jobs, n_jobs, max_elem, cbase, mat_mask, qfast, ke, st);
+            launch_cols_any<double>(one, jobs, n_jobs, max_elem, cbase, mat_mask, qfast, ke, st);
         else
-            launch_cols_any<float>(b, jobs, n_jobs, max_elem, cbase, mat_mask, qfast, ke, st);
+            launch_cols_any<float>(one, jobs, n_jobs, max_elem, cbase, mat_mask, qfast, ke, st);
     }
     for (int s = 0; s < b.n_slices; s++) {
         if (!((rhs_mask >> s) & 1u)) continue;
         const dim3 grid((unsigned)((max_elem + 63) / 64), (unsigned)((b.slices[s].n_tf + 63) / 64), n_jobs);
-        if (precision == SLX_PREC_FP64)
-            hipLaunchKernelGGL((rhs_tiles<double>), grid, dim3(256), 0, st, jobs, (const unsigned char*)cbase, s, qfast, (double*)ke);
-        else
-            hipLaunchKernelGGL((rhs_tiles<float>), grid, dim3(256), 0, st, jobs, (const unsigned char*)cbase, s, qfast, (float*)ke);
+        const unsigned char* cb = (const unsigned char*)cbase;
+#define SLX_RHS_GO(T_, M_) hipLaunchKernelGGL((rhs_tiles<T_, M_>), grid, dim3(256), 0, st, one, jobs, cb, s, qfast, (T_*)ke)
+        if (precision == SLX_PREC_FP64) {
+            if (n_jobs > 1) SLX_RHS_GO(double, true);
+            else SLX_RHS_GO(double, false);
+        } else {
+            if (n_jobs > 1) SLX_RHS_GO(float, true);
+            else SLX_RHS_GO(float, false);
+        }
+#undef SLX_RHS_GO
     }
     return hipGetLastError();
 }

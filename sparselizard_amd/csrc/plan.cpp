@@ -30,9 +30,9 @@
 #include <dlfcn.h>
 
 namespace slx {
-hipError_t launch_coef(const DevBucket& b, const DevJob* jobs, int n_jobs, int max_elem, const DevInputs& in, bool fp64, void* cbase,
+hipError_t launch_coef(const DevJob& one, const DevJob* jobs, int n_jobs, int max_elem, const DevInputs& in, bool fp64, void* cbase,
                        hipStream_t st, int qfast, const DevPack& pk);
-hipError_t launch_elem(const DevBucket& b, const DevJob* jobs, int n_jobs, int max_elem, const void* cbase, int precision, void* ke,
+hipError_t launch_elem(const DevJob& one, const DevJob* jobs, int n_jobs, int max_elem, const void* cbase, int precision, void* ke,
                        hipStream_t st, uint32_t slice_mask, int qfast);
 hipError_t scratch_init(int device);
 hipError_t launch_reduce(const DevReduce& rd, int max_erow_len, bool ke_fp64, const void* ke, double* Aval, double* Dval,
@@ -2293,7 +2293,7 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
         } else {
             SLX_CHECK(b.n_regs <= SLX_MAX_REGS, "coefficient program of " << b.n_regs << " registers has no compiled kernel and the interpreter holds "
                                                << SLX_MAX_REGS << " (" << P.coef_jit_error << ")");
-            HIPCHECK(launch_coef(b, f.jobs, (int)f.buckets.size(), f.max_elem, in, ke64, P.d_ctab.p, s, qfast, P.dpack));
+            HIPCHECK(launch_coef(DevJob{b, (int64_t)P.ctab_off[b0]}, f.jobs, (int)f.buckets.size(), f.max_elem, in, ke64, P.d_ctab.p, s, qfast, P.dpack));
         }
         if (tm) tm->end();
     };
@@ -2373,7 +2373,7 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
         int p = (precision == SLX_PREC_FP64) ? SLX_PREC_FP64 : SLX_PREC_FP32;
         if ((all & ~done) != 0) {
             if (tm) tm->begin(T_VALU);
-            HIPCHECK(launch_elem(b, f.jobs, nj, f.max_elem, P.d_ctab.p, p, P.d_ke.p, bst, all & ~done, qfast));
+            HIPCHECK(launch_elem(DevJob{b, (int64_t)P.ctab_off[bi]}, f.jobs, nj, f.max_elem, P.d_ctab.p, p, P.d_ke.p, bst, all & ~done, qfast));
             if (tm) tm->end();
         }
     }
