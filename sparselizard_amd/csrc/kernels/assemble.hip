@@ -42,9 +42,15 @@ template <typename T, int V>
 __device__ void run_program(const DevBucket& b, const DevInputs& in, const int (&e)[V], const int (&q)[V], const Geo (&g)[V],
                             const bool (&on)[V], int nq, int qfast, const DevPack& pk, T* __restrict__ ctab) {
     T reg[SLX_MAX_REGS][V];
-    const int64_t stride = (int64_t)nq * b.n_elem;
+    // outputs at imm * stride + at[v]: the slot, or the record position (qfast 2)
+    const int64_t stride = qfast == 2 ? 1 : (int64_t)nq * b.n_elem;
+    const slx_instr* prog = qfast == 2 ? pk.prog : b.prog;
+    int64_t at[V];
+#pragma unroll
+    for (int v = 0; v < V; v++)
+        at[v] = qfast == 2 ? (int64_t)e[v] * pk.erec : qfast ? (int64_t)e[v] * nq + q[v] : (int64_t)q[v] * b.n_elem + e[v];
     for (int pc = 0; pc < b.n_instr; pc++) {
-        const slx_instr ins = b.prog[pc];
+        const slx_instr ins = prog[pc];
         const int ia = ins.a < SLX_MAX_REGS ? ins.a : 0, ib = ins.b < SLX_MAX_REGS ? ins.b : 0;
         T r[V];
         switch (ins.op) {
@@ -98,18 +104,10 @@ __device__ void run_program(const DevBucket& b, const DevInputs& in, const int (
                 for (int v = 0; v < V; v++) r[v] = pow(reg[ia][v], reg[ib][v]);
                 break;
             case SLX_OP_OUT:
-                if (qfast == 2) {
-                    const int at = pk.pos[ins.imm];
-#pragma unroll
-                    for (int v = 0; v < V; v++)
-                        if (on[v] && at >= 0) ctab[(size_t)e[v] * pk.erec + at] = reg[ia][v] * (T)fabs(g[v].det);
-                    continue;
-                }
+                if (ins.imm < 0) continue;
 #pragma unroll
                 for (int v = 0; v < V; v++)
-                    if (on[v])
-                        ctab[(size_t)ins.imm * stride + (qfast ? (size_t)e[v] * nq + q[v] : (size_t)q[v] * b.n_elem + e[v])] =
-                            reg[ia][v] * (T)fabs(g[v].det);
+                    if (on[v]) ctab[ins.imm * stride + at[v]] = reg[ia][v] * (T)fabs(g[v].det);
                 continue;
             default:
 #pragma unroll

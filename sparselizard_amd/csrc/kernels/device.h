@@ -59,10 +59,11 @@ struct DevInputs {
     const double* field_data[SLX_MAX_FIELDS];
 };
 
-// Record layout of a bucket's coefficients: slot s of element e at
-// e * erec + pos[s] (pos < 0: not stored), zeros at the pads.
+// Record layout of a bucket's coefficients, as the interpreter writes it: the
+// program with each output's record position in place of its slot (< 0: not
+// stored), zeros at the pads of the erec values per element.
 struct DevPack {
-    const int32_t* pos;
+    const slx_instr* prog;
     const int32_t* pads;
     int32_t n_pads, erec;
 };

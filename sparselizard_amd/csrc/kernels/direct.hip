@@ -172,10 +172,18 @@ int direct_max_row(const DirectDev& d) {
 hipError_t launch_direct(const DirectDev& d, bool fp64, const void* ctab, const void* rtab, double* Aval, double* Dval, double* rhs,
                          hipStream_t st, const int64_t* cb, const int64_t* ce, const int* cl, int nc) {
     if (d.nrows == 0) return hipSuccess;
+    const size_t phi = direct_phi_bytes(d, fp64);
     for (int c = 0; c < nc;) {
-        // classes whose longest row keeps eight workgroups on a CU run together
+        // classes whose longest row keeps eight workgroups on a CU run together;
+        // so do all the rows that the waves in flight hold at once with the
+        // longest one's accumulators: no wave takes a second batch then, and one
+        // launch ends with its longest rows, where several add theirs up (P2
+        // elasticity, us an assembly in the FP16 split, one launch against one per
+        // class: 3^3 x 6 213 and 236, 8^3 x 6 42 and 65)
         int last = c;
-        if ((size_t)4 * (64 / d.G) * direct_stride(cl[c]) * 8 + direct_phi_bytes(d, fp64) <= 20 * 1024) last = nc - 1;
+        const size_t wave = (size_t)(64 / d.G) * direct_stride(cl[c]) * 8;
+        const int64_t waves = (int64_t)std::min<size_t>(8, (SLX_DIRECT_CU_LDS - phi) / wave) * d.n_cu;
+        if (4 * wave + phi <= 20 * 1024 || ce[nc - 1] - cb[c] <= waves * (64 / d.G)) last = nc - 1;
         DirectLaunch q{ctab, rtab, Aval, Dval, rhs, cb[c], ce[last], cl[c], d.has_rhs && last == nc - 1, st};
         const hipError_t e = fp64 ? launch_direct_f64(d, q) : launch_direct_f32(d, q);
         if (e != hipSuccess) return e;

@@ -1778,8 +1778,11 @@ void choose_direct(slx_plan_s& P, const slx_plan_desc& d, const KeLayout& L) {
         P.dd.rphi32 = P.dev(rphi32.data(), rphi32.size());
         P.dd.rbase = P.dev(rbase.data(), rbase.size());
     }
-    std::vector<int32_t> pos(pack.pos.begin(), pack.pos.end()), pads(pack.pads.begin(), pack.pads.end());
-    P.dpack.pos = P.dev(pos.data(), pos.size());
+    std::vector<int32_t> pads(pack.pads.begin(), pack.pads.end());
+    std::vector<slx_instr> prog(bd.prog, bd.prog + bd.n_instr);
+    for (slx_instr& x : prog)
+        if (x.op == SLX_OP_OUT) x.imm = pack.pos[x.imm];
+    P.dpack.prog = P.dev(prog.data(), prog.size());
     P.dpack.pads = pads.empty() ? nullptr : P.dev(pads.data(), pads.size());
     P.dpack.n_pads = (int)pads.size();
     P.dpack.erec = pack.erec;

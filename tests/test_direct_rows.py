@@ -24,7 +24,8 @@ CASES = [
     ("convdiff2d", "n=6;order=2"),
     ("elasticity3d", "n=2;order=1"),    # 4 x 4, three fields, 9 pairs
     ("elasticity3d", "n=3"),            # 10 x 10, five lanes per row
-    ("elasticity3d", "n=10"),           # compiled records, three row classes
+    ("elasticity3d", "n=10"),           # compiled records, three row classes in one launch
+    ("elasticity3d", "n=11"),           # the longest rows by themselves, the others in one launch
     ("elasticity3d", "n=2;clamp=0"),    # no constrained column
 ]
 
