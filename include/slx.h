@@ -251,6 +251,12 @@ slx_status slx_plan_kernel_counts(slx_plan plan, int32_t precision, int32_t* n_b
  * coefficients; the FP16 split, BF16 split and FP32-MFMA modes, 0 for the FP32
  * VALU and FP64 modes). */
 slx_status slx_plan_tile_count(slx_plan plan, int32_t precision, int32_t* n_tile);
+/* What else a mode's assemblies run: *row_wise 1 when the matrix is assembled
+ * row by row, without element matrices; *n_elem_fused buckets whose coefficient
+ * program and contraction are one compiled kernel; *n_tile_compiled slices of
+ * slx_plan_tile_count whose kernel is compiled for the slice. */
+slx_status slx_plan_routes(slx_plan plan, int32_t precision, int32_t* row_wise, int32_t* n_elem_fused,
+                           int32_t* n_tile_compiled);
 /* The fused launch of a precision mode: factorized slices of every bucket in
  * one persistent launch (contribution.cpp:61-133 loops over the element
  * groups one after the other; here their elements share one work queue,

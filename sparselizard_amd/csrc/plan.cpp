@@ -2189,8 +2189,13 @@ void compile_coef_programs(slx_plan_s& P, const slx_plan_desc& d) {
                             shape.store = f.buckets.back() == d.n_buckets - 1;
                     std::string eerr;
                     hipFunction_t efn = nullptr;
-                    if (elem_compile(bd.prog, bd.n_instr, todo[i].second != 0, fnff, shape, several, &efn, &eerr))
+                    if (elem_compile(bd.prog, bd.n_instr, todo[i].second != 0, fnff, shape, several, &efn, &eerr)) {
                         P.elem_fn[todo[i].first][todo[i].second] = efn;
+                    } else {
+                        std::fprintf(stderr, "element kernel not compiled, program and contraction run apart: %s\n", eerr.c_str());
+                        std::lock_guard<std::mutex> lk(mu);
+                        P.coef_jit_error = eerr;
+                    }
                 }
                 const bool affine = elem_affine(bd);
                 if (P.elem_fn[todo[i].first][todo[i].second]) continue;
@@ -2919,6 +2924,22 @@ slx_status slx_plan_tile_count(slx_plan p, int32_t precision, int32_t* n_tile) {
         if (precision == SLX_PREC_F16_SPLIT || precision == SLX_PREC_BF16_SPLIT || precision == SLX_PREC_FP32_MFMA)
             for (auto& v : p->tile) n += (int)v.size();
         *n_tile = n;
+    });
+}
+
+slx_status slx_plan_routes(slx_plan p, int32_t precision, int32_t* row_wise, int32_t* n_elem_fused, int32_t* n_tile_compiled) {
+    return guarded([&] {
+        SLX_CHECK(p && row_wise && n_elem_fused && n_tile_compiled, "null argument");
+        SLX_CHECK(precision >= 0 && precision <= 4, "unknown precision " << precision);
+        const int ar = precision == SLX_PREC_F16_SPLIT ? 0 : precision == SLX_PREC_BF16_SPLIT ? 1 : precision == SLX_PREC_FP32_MFMA ? 2 : -1;
+        *row_wise = p->direct ? 1 : 0;
+        *n_elem_fused = *n_tile_compiled = 0;
+        for (const auto& f : p->families) {
+            const int n = (int)f.buckets.size();
+            if (p->elem_fn[f.buckets[0]][precision == SLX_PREC_FP64 ? 1 : 0]) *n_elem_fused += n;
+            for (size_t k = 0; ar >= 0 && k < f.tile_fn.size(); k++)
+                if (f.tile_fn[k][ar].fn) *n_tile_compiled += n;
+        }
     });
 }
 

@@ -51,7 +51,7 @@ def test_rows_match_oracle(ctx, kind, spec, precision, tol):
     print("case direct", kind, spec, precision, flush=True)
     prob = sa.Problem(ctx, kind, spec)
     plan = prob.generate(precision)
-    assert plan.kernel_counts("f16split") == dict(batched=0, factorized=0)
+    assert plan.routes(precision)["row_wise"]
     a = check(prob, plan, tol)
     b = prob.generate(precision).csr(prob.info()["ndofs"])
     assert np.array_equal(a.Aval, b.Aval) and np.array_equal(a.Dval, b.Dval) and np.array_equal(a.rhs, b.rhs)
@@ -76,6 +76,7 @@ def test_element_kernels_agree(ctx, kind, spec, precision, tol, monkeypatch):
     monkeypatch.setenv("SLX_TUNE_DIRECT", "0")
     prob2 = sa.Problem(ctx, kind, spec)
     plan2 = prob2.generate(precision)
+    assert plan.routes(precision)["row_wise"] and not plan2.routes(precision)["row_wise"]
     kb, kl = plan2.ke_layout()
     d, sel, k = prob2.desc(), [], 0
     for b in range(d.n_buckets):
@@ -116,6 +117,7 @@ def test_absent_columns(ctx, kind, spec, precision, tol):
     prob = sa.Problem(ctx, kind, spec)
     drop_columns(prob, 7)
     plan = sa.Plan.create(ctx, prob)
+    assert plan.routes(precision)["row_wise"]
     plan.assemble(prob.numeric(), precision)
     plan.sync()
     info = prob.info()

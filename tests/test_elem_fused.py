@@ -22,9 +22,10 @@ def relerr(a, b):
 
 
 @pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("f16split", 1e-6), ("fp32", 1e-6)])
-@pytest.mark.parametrize("kind,spec", [("newton2d", "n=2"), ("newton2d", "n=12"), ("newton2d", "n=46"), ("hppoisson3d", "n=3;pmin=1;pmax=1"),
-                                       ("hppoisson3d", "n=3;pmin=1;pmax=2"), ("prism3d", "n=4"), ("quadbatch", "instances=2;nmin=3;nmax=5;order=1")])
-def test_matches_oracle_and_separate_kernels(ctx, kind, spec, precision, tol, monkeypatch):
+@pytest.mark.parametrize("kind,spec,n_fused", [("newton2d", "n=2", 2), ("newton2d", "n=12", 2), ("newton2d", "n=46", 2),
+                                               ("hppoisson3d", "n=3;pmin=1;pmax=1", 2), ("hppoisson3d", "n=3;pmin=1;pmax=2", 3),
+                                               ("prism3d", "n=4", 3), ("quadbatch", "instances=2;nmin=3;nmax=5;order=1", 1)])
+def test_matches_oracle_and_separate_kernels(ctx, kind, spec, n_fused, precision, tol, monkeypatch):
     print("case elem fused", kind, spec, precision, flush=True)
     got = {}
     for fused in ("1", "0"):
@@ -36,6 +37,7 @@ def test_matches_oracle_and_separate_kernels(ctx, kind, spec, precision, tol, mo
             prob.setdata_vec(0.1 * x)
         plan = prob.plan()
         assert plan.coef_mode("compiled") > 0
+        assert plan.routes(precision)["elem_fused"] == (n_fused if fused == "1" else 0)
         plan = prob.generate(precision)
         got[fused] = plan.csr(info["ndofs"]), plan.coefficients()
     ref = py_oracle.assemble(prob.desc_ptr(), prob.numeric(), info["ndofs"], info["nfree"])

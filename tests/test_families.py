@@ -12,14 +12,19 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("f16split", 1e-6), ("bf16split", 1e-6), ("fp32", 1e-6)])
-@pytest.mark.parametrize("spec,tile", [("elem=tet;term=maxwell;n=3;order=2", "1"), ("elem=tet;term=maxwell;n=9;order=2", "1"),
-                                       ("elem=tet;term=maxwell;n=3;order=2", "0"), ("elem=tet;term=maxwell;n=5;order=1", "1")])
-def test_orientation_buckets(ctx, spec, tile, precision, tol, monkeypatch):
+@pytest.mark.parametrize("spec,tile,compiled", [("elem=tet;term=maxwell;n=3;order=2", "1", False), ("elem=tet;term=maxwell;n=9;order=2", "1", True),
+                                                ("elem=tet;term=maxwell;n=3;order=2", "0", False), ("elem=tet;term=maxwell;n=5;order=1", "1", True)])
+def test_orientation_buckets(ctx, spec, tile, compiled, precision, tol, monkeypatch):
     print("case families", spec, tile, precision, flush=True)
     monkeypatch.setenv("SLX_TUNE_TILE", tile)
     prob = sa.Problem(ctx, "hcurlprojection", spec)
     info = prob.info()
-    got = prob.generate(precision).csr(info["ndofs"])
+    plan = prob.generate(precision)
+    split = precision in ("f16split", "bf16split")
+    assert plan.tile_count(precision) == (2 * sum(prob.desc().buckets[b].n_elem > 0 for b in range(prob.desc().n_buckets))
+                                          if split and tile == "1" else 0)
+    assert plan.routes(precision)["tile_compiled"] == (plan.tile_count(precision) if compiled else 0)
+    got = plan.csr(info["ndofs"])
     ref = py_oracle.assemble(prob.desc_ptr(), prob.numeric(), info["ndofs"], info["nfree"], nthreads=8)
     assert np.array_equal(got.Arow, ref.Arow) and np.array_equal(got.Acol, ref.Acol)
     for a, b in ((got.Aval, ref.Aval), (got.rhs, ref.rhs)):

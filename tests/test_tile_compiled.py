@@ -41,7 +41,11 @@ def test_matches_oracle_and_general_kernel(ctx, kind, spec, precision, tol, monk
         info = prob.info()
         plan = prob.plan()
         plan.coef_mode("compiled")
-        assert plan.tile_count(precision) >= 1
+        n_tile = plan.tile_count(precision)
+        assert n_tile >= 1
+        # order-3 hexahedra in the BF16 split: the tables exceed the LDS, the general kernel runs
+        fits = (spec, precision) != ("n=2;pmin=3;pmax=3", "bf16split")
+        assert plan.routes(precision)["tile_compiled"] == (n_tile if compiled == "1" and fits else 0)
         plan = prob.generate(precision)
         got[compiled] = plan.csr(info["ndofs"])
     assert "not compiled" not in capfd.readouterr().err
