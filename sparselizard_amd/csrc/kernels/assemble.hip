@@ -752,7 +752,7 @@ hipError_t launch_elem(const DevJob& one, const DevJob* jobs, int n_jobs, int ma
     // covers go to the tiled kernel
     uint32_t rhs_mask = 0;
     for (int s = 0; s < b.n_slices; s++)
-        if (((slice_mask >> s) & 1u) && b.slices[s].is_rhs && b.slices[s].n_tf > 16) rhs_mask |= 1u << s;
+        if (((slice_mask >> s) & 1u) && b.slices[s].is_rhs && b.slices[s].n_tf > SLX_RHS_COLS) rhs_mask |= 1u << s;
     const uint32_t mat_mask = slice_mask & ~rhs_mask;
     if (mat_mask) {
         if (precision == SLX_PREC_FP64)

@@ -2071,7 +2071,12 @@ void upload_buckets(slx_plan_s& P, const slx_plan_desc& d, const KeLayout& L) {
 // triangles, order-1 hexahedra and prisms, small right-hand sides) is computed
 // by one compiled kernel.  The last bucket also stores its coefficient table
 // there, which slx_plan_coefficients reads.  Measured against the program and
-// element kernels at 5e5 P2 triangles (whole assembly): 0.20 vs 0.51 ms.
+// element kernels, in us: whole assemblies of P2 Newton on 5e5 triangles 200 and
+// 510, on 512 triangles 53 and 66; order-1 prisms, 1024 of them 105 and 127.
+// Right-hand sides of more than SLX_RHS_COLS functions keep the tiled kernel: one
+// thread would walk all Gauss points of an element with so many sums, 77 us for
+// 700 to 1.6e4 order-2 prisms (18 functions, 48 points) where program and tiles
+// take 25 to 41, 112 to 184 us for order-3 ones (40, 80) where they take 30 to 90.
 // SLX_TUNE_ELEM_FUSED=0 keeps the two kernels apart.
 // Constant Jacobian: lines, triangles and tetrahedra of order-1 geometry.
 bool elem_affine(const slx_bucket_desc& bd) {
@@ -2088,6 +2093,7 @@ bool elem_shape(const slx_plan_s& P, const slx_plan_desc& d, int b, ElemShape& s
     int entries = 0;
     for (int s = 0; s < bd.n_slices; s++) {
         const slx_slice_desc& sd = bd.slices[s];
+        if (sd.is_rhs && sd.n_tf > SLX_RHS_COLS) return false;
         ElemShape::Slice sl;
         sl.n_tf = sd.n_tf;
         sl.n_dof = sd.is_rhs ? 0 : sd.n_dof;

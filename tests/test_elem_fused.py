@@ -3,7 +3,8 @@ and against the separate program and element kernels: triangles of order 2 with
 a field in the coefficients (matrix and right-hand side in one bucket), order-1
 hexahedra and prisms (Gauss-point-varying Jacobians, two matrix slices), a
 constant right-hand side, order-1 quadrangles; one element over the workgroup
-size and a few.
+size and a few.  Right-hand sides of more than 16 functions (order-2 hexahedra
+and prisms) keep the tiled kernel.
 
 Gates as for the element kernels: FP64 1e-12; FP32 modes 1e-6 (sums of at most 36
 rounded products per entry).
@@ -23,8 +24,8 @@ def relerr(a, b):
 
 @pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("f16split", 1e-6), ("fp32", 1e-6)])
 @pytest.mark.parametrize("kind,spec,n_fused", [("newton2d", "n=2", 2), ("newton2d", "n=12", 2), ("newton2d", "n=46", 2),
-                                               ("hppoisson3d", "n=3;pmin=1;pmax=1", 2), ("hppoisson3d", "n=3;pmin=1;pmax=2", 3),
-                                               ("prism3d", "n=4", 3), ("quadbatch", "instances=2;nmin=3;nmax=5;order=1", 1)])
+                                               ("hppoisson3d", "n=3;pmin=1;pmax=1", 2), ("hppoisson3d", "n=3;pmin=1;pmax=2", 2),
+                                               ("prism3d", "n=4", 3), ("prism3d", "n=3;order=2", 0), ("quadbatch", "instances=2;nmin=3;nmax=5;order=1", 1)])
 def test_matches_oracle_and_separate_kernels(ctx, kind, spec, n_fused, precision, tol, monkeypatch):
     print("case elem fused", kind, spec, precision, flush=True)
     got = {}
