@@ -2189,10 +2189,15 @@ void compile_coef_programs(slx_plan_s& P, const slx_plan_desc& d) {
                     several = several || (f.buckets.size() > 1 && std::find(f.buckets.begin(), f.buckets.end(), todo[i].first) != f.buckets.end());
                 ElemShape shape;
                 if (elem_shape(P, d, todo[i].first, shape)) {
-                    // one kernel per family: its last bucket's store is everyone's
+                    // one kernel per family: its last bucket's store is everyone's, and
+                    // rows start 16-byte aligned only where they do in every bucket
                     for (const auto& f : P.families)
-                        if (std::find(f.buckets.begin(), f.buckets.end(), todo[i].first) != f.buckets.end())
+                        if (std::find(f.buckets.begin(), f.buckets.end(), todo[i].first) != f.buckets.end()) {
                             shape.store = f.buckets.back() == d.n_buckets - 1;
+                            for (int c : f.buckets)
+                                for (size_t k = 0; k < shape.slices.size(); k++)
+                                    shape.slices[k].vec4 = shape.slices[k].vec4 && P.dbuckets[c].slices[k].ke_base % 4 == 0;
+                        }
                     std::string eerr;
                     hipFunction_t efn = nullptr;
                     if (elem_compile(bd.prog, bd.n_instr, todo[i].second != 0, fnff, shape, several, &efn, &eerr)) {

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 import sparselizard_amd as sa
+from _synthetic import Synthetic, addresses
 from oracle import py_oracle
 
 pytestmark = pytest.mark.gpu
@@ -28,4 +29,29 @@ def test_orientation_buckets(ctx, spec, tile, compiled, precision, tol, monkeypa
     ref = py_oracle.assemble(prob.desc_ptr(), prob.numeric(), info["ndofs"], info["nfree"], nthreads=8)
     assert np.array_equal(got.Arow, ref.Arow) and np.array_equal(got.Acol, ref.Acol)
     for a, b in ((got.Aval, ref.Aval), (got.rhs, ref.rhs)):
+        assert np.linalg.norm(a - b) <= tol * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("fp32", 1e-6)])
+def test_buckets_with_other_row_layouts(ctx, precision, tol):
+    """One launch over two buckets: the two slices of the first have rows of their
+    own, those of the second share theirs, so that the second slice's columns
+    start at another alignment there."""
+    print("case family layouts", precision, flush=True)
+    rng = np.random.default_rng(5)
+    pairs = [(1, 1), (2, 2), (3, 0)]
+    cols = [addresses(rng, 3, 300, 0, 90), addresses(rng, 3, 300, 90, 180)]
+    rows = [addresses(rng, 4, 300, 0, 90), addresses(rng, 4, 300, 90, 180)]
+    buckets = [[dict(tf=rows[0], dof=cols[0], pairs=pairs), dict(tf=rows[1], dof=cols[1], pairs=pairs)],
+               [dict(tf=rows[0][:, :90], dof=cols[0][:, :90], pairs=pairs), dict(tf=rows[0][:, :90], dof=cols[1][:, :90], pairs=pairs)]]
+    prob = Synthetic(buckets, 180, rng.random(180) < 0.1, q_invariant=0)
+    plan = sa.Plan.create(ctx, prob)
+    plan.coef_mode("compiled")
+    assert plan.routes(precision)["elem_fused"] == 2
+    plan.assemble(prob.numeric(), precision)
+    plan.sync()
+    got = plan.csr(prob.ndofs)
+    ref = py_oracle.assemble(prob.desc_ptr(), prob.numeric(), prob.ndofs, prob.nfree)
+    assert np.array_equal(got.Arow, ref.Arow) and np.array_equal(got.Acol, ref.Acol)
+    for a, b in ((got.Aval, ref.Aval), (got.Dval, ref.Dval)):
         assert np.linalg.norm(a - b) <= tol * np.linalg.norm(b)
