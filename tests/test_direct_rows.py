@@ -1,7 +1,9 @@
-"""Row-wise assembly (kernels/direct.hip) against the oracle: every shape of
-the kernel (one or three dof fields, 4, 6, 9 and 12 derivative pairs, two or
-three columns per lane), one to many elements, compiled and interpreted
-coefficients, and the element kernels that SLX_TUNE_DIRECT=0 keeps.
+"""Row-wise assembly (kernels/direct.hip) against the oracle: the workloads that
+take it, one to many elements, compiled and interpreted coefficients, the element
+kernels that SLX_TUNE_DIRECT=0 keeps, absent columns, and on synthetic descriptions
+the other shapes of the kernel (two dof fields, 12 derivative pairs, two and five
+columns per lane, rows of 255 columns and more, right-hand sides in the matrix
+bucket) and the plans that fall back.
 
 Gates: FP64 1e-12; the reduced modes run this kernel in FP32, whose entries are
 sums of at most 12 products of rounded factors (below 14 * 6e-8 of the sum of
@@ -11,6 +13,7 @@ import numpy as np
 import pytest
 
 import sparselizard_amd as sa
+from _synthetic import Synthetic, addresses
 from oracle import py_oracle
 
 pytestmark = pytest.mark.gpu
@@ -23,7 +26,7 @@ CASES = [
     ("convdiff2d", "n=8"),              # 6 pairs
     ("convdiff2d", "n=6;order=2"),
     ("elasticity3d", "n=2;order=1"),    # 4 x 4, three fields, 9 pairs
-    ("elasticity3d", "n=3"),            # 10 x 10, five lanes per row
+    ("elasticity3d", "n=3"),            # 10 x 10, four lanes per row
     ("elasticity3d", "n=10"),           # compiled records, three row classes in one launch
     ("elasticity3d", "n=11"),           # the longest rows by themselves, the others in one launch
     ("elasticity3d", "n=2;clamp=0"),    # no constrained column
@@ -133,3 +136,70 @@ def test_absent_columns(ctx, kind, spec, precision, tol):
         a, b = getattr(got, name), getattr(ref, name)
         assert relerr(a, b) <= tol, name
         assert np.abs(a - b).max() <= 100 * tol * np.abs(b).max(), name
+
+
+ALL = [(r, c) for r in range(4) for c in range(4)]
+# fields of rows and columns, derivative pairs, row and column functions, elements, dofs per field, right-hand side
+SHAPES = [
+    (2, 1, 12, 3, 3, 50, 40, "other"),       # one lane a row
+    (1, 1, 11, 5, 5, 60, 40, "same"),        # two lanes, three columns each
+    (2, 2, 3, 4, 4, 70, 60, "other"),        # two lanes, two columns each
+    (3, 2, 9, 10, 10, 40, 50, "same"),       # two dof fields, 9 pairs
+    (1, 2, 7, 6, 6, 65, 50, "none"),
+    (3, 3, 12, 10, 10, 40, 60, "other"),     # 36 coefficients a segment
+    (3, 3, 9, 20, 20, 25, 60, "same"),       # five columns a lane
+    (2, 1, 6, 15, 13, 33, 70, "other"),      # a last lane without columns
+    (1, 1, 4, 4, 10, 64, 80, "other"),       # more columns than rows
+    (3, 3, 9, 10, 10, 700, 300, "other"),    # 16-bit slots
+    (2, 2, 9, 10, 10, 700, 300, "same"),
+    (1, 1, 9, 20, 20, 12000, 2500, "none"),  # rows of 1300 columns: fewer than 16 of them a wave
+    (1, 1, 12, 12, 12, 900, 400, "same"),
+]
+
+
+def synthetic(na, nb, n_pairs, n_tf, n_dof, n_elem, per_field, rhs, seed=3):
+    rng = np.random.default_rng(seed)
+    nf = max(na, nb)
+    tf = [addresses(rng, n_tf, n_elem, a * per_field, (a + 1) * per_field, 0.03) for a in range(na)]
+    dof = [addresses(rng, n_dof, n_elem, b * per_field, (b + 1) * per_field, 0.03) for b in range(nb)]
+    mat = [dict(tf=t, dof=u, pairs=ALL[:n_pairs]) for t in tf for u in dof]
+    rows = [dict(tf=t, pairs=[(a % 4, 0)]) for a, t in enumerate(tf)]
+    buckets = [mat + rows] if rhs == "same" else [mat, rows] if rhs == "other" else [mat]
+    return Synthetic(buckets, nf * per_field, rng.random(nf * per_field) < 0.1, seed)
+
+
+def check_synthetic(ctx, prob, precision, tol, row_wise):
+    ref = py_oracle.assemble(prob.desc_ptr(), prob.numeric(), prob.ndofs, prob.nfree, nthreads=8)
+    plan = sa.Plan.create(ctx, prob)
+    assert plan.routes(precision)["row_wise"] == row_wise
+    for mode in ("interpreter", "compiled"):
+        plan.coef_mode(mode)
+        plan.assemble(prob.numeric(), precision)
+        plan.sync()
+        got = plan.csr(prob.ndofs)
+        for name in ("Arow", "Acol", "Drow", "Dcol"):
+            assert np.array_equal(getattr(got, name), getattr(ref, name)), name
+        for name in ("Aval", "Dval", "rhs"):
+            a, b = getattr(got, name), getattr(ref, name)
+            assert relerr(a, b) <= tol, (name, mode)
+            assert np.abs(a - b).max(initial=0.0) <= 100 * tol * np.abs(b).max(initial=0.0), (name, mode)
+    return ref
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("f16split", 1e-6)])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "-".join(map(str, s)))
+def test_synthetic_shapes(ctx, shape, precision, tol):
+    print("case synthetic", shape, precision, flush=True)
+    ref = check_synthetic(ctx, synthetic(*shape), precision, tol, True)
+    if shape[5] >= 700:
+        assert (np.diff(ref.Arow) + np.diff(ref.Drow)).max() >= (1200 if shape[5] == 12000 else 255)
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("f16split", 1e-6)])
+@pytest.mark.parametrize("shape", [(1, 2, 10, 6, 6, 60, 50, "other"),       # two dof fields with more than 9 pairs
+                                   (1, 3, 4, 6, 6, 2000, 300, "other"),     # two lanes a row: none of more than 254 columns
+                                   (1, 1, 4, 24, 24, 30, 60, "same")],      # more than 20 columns
+                         ids=lambda s: "-".join(map(str, s)))
+def test_element_kernels_take_the_rest(ctx, shape, precision, tol):
+    print("case synthetic", shape, precision, flush=True)
+    check_synthetic(ctx, synthetic(*shape), precision, tol, False)
