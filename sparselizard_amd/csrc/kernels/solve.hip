@@ -52,31 +52,19 @@ __device__ inline double all_sum(const double* __restrict__ part, int n, double*
 
 // y[r] = c0 f[r] - c1 (A x)[r] over one CSR matrix, LPR lanes per row (the
 // lanes of a row group share r, so the width-LPR shuffles stay inside
-// active lanes); with part != null the block also writes its partial sum of
-// x[r] y[r] (square A)
+// active lanes)
 template <int LPR, typename VT, typename XT, typename YT>
 __global__ void __launch_bounds__(256) spmv_kernel(int64_t nrows, const int64_t* __restrict__ rowp, const int32_t* __restrict__ col,
-                                                   const VT* __restrict__ val, const XT* __restrict__ x, const YT* f, YT c0, YT c1,
-                                                   YT* y, double* __restrict__ part) {
-    __shared__ double sh[4];
+                                                   const VT* __restrict__ val, const XT* __restrict__ x, const YT* f, YT c0, YT c1, YT* y) {
     const int l = threadIdx.x % LPR;
     const int64_t rstride = (int64_t)gridDim.x * (256 / LPR);
-    double acc = 0.0;
     for (int64_t r = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR; r < nrows; r += rstride) {
         YT s = 0;
         const int64_t e = rowp[r + 1];
         for (int64_t k = rowp[r] + l; k < e; k += LPR) s += (YT)val[k] * (YT)x[col[k]];
 #pragma unroll
         for (int o = LPR / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, LPR);
-        if (l == 0) {
-            const YT v = (f ? c0 * f[r] : (YT)0) - c1 * s;
-            y[r] = v;
-            if (part) acc += (double)x[r] * (double)v;
-        }
-    }
-    if (part) {
-        const double t = block_sum(acc, sh);
-        if (threadIdx.x == 0) part[blockIdx.x] = t;
+        if (l == 0) y[r] = (f ? c0 * f[r] : (YT)0) - c1 * s;
     }
 }
 
@@ -92,15 +80,13 @@ static int spmv_lpr(int64_t nrows, int64_t nnz) {
 
 template <typename VT, typename XT, typename YT>
 static void spmv(int64_t nrows, int64_t nnz, const int64_t* rowp, const int32_t* col, const VT* val, const XT* x, const YT* f, YT c0,
-                 YT c1, YT* y, double* part, hipStream_t st) {
+                 YT c1, YT* y, hipStream_t st) {
     if (nrows <= 0) return;
     const int lpr = spmv_lpr(nrows, nnz);
-    // the fixed grid when partial sums are wanted, else one row group per thread group
-    const int64_t want = (nrows * lpr + 255) / 256;
-    const unsigned grid = part ? SLX_SOLVE_BLOCKS : (unsigned)std::min<int64_t>(want, 1 << 20);
+    const unsigned grid = (unsigned)std::min<int64_t>((nrows * lpr + 255) / 256, 1 << 20);
 #define SLX_SPMV_CASE(L)                                                                                                          \
     case L:                                                                                                                       \
-        hipLaunchKernelGGL((spmv_kernel<L, VT, XT, YT>), dim3(grid), dim3(256), 0, st, nrows, rowp, col, val, x, f, c0, c1, y, part); \
+        hipLaunchKernelGGL((spmv_kernel<L, VT, XT, YT>), dim3(grid), dim3(256), 0, st, nrows, rowp, col, val, x, f, c0, c1, y);       \
         break;
     switch (lpr) {
         SLX_SPMV_CASE(2)
@@ -676,7 +662,7 @@ hipError_t eliminate_system(const SolveSystem& s, const double* b, double* out, 
     hipLaunchKernelGGL(gather_kernel, dim3(blocks(n)), dim3(256), 0, st, n, s.free_dofs, b, out);
     if (s.ncons > 0) {
         hipLaunchKernelGGL(gather_kernel, dim3(blocks(s.ncons)), dim3(256), 0, st, s.ncons, s.cons_dofs, b, xd);
-        spmv<double, double, double>(n, s.nnzD, s.Drow, s.Dcol, s.Dval, xd, out, 1.0, 1.0, out, nullptr, st);
+        spmv<double, double, double>(n, s.nnzD, s.Drow, s.Dcol, s.Dval, xd, out, 1.0, 1.0, out, st);
     }
     return hipGetLastError();
 }
@@ -686,10 +672,10 @@ hipError_t matvec_system(const SolveSystem& s, const double* x, double* y, doubl
     HIPERR(hipMemcpyAsync(y, x, s.n_dofs * sizeof(double), hipMemcpyDeviceToDevice, st));
     if (n == 0) return hipSuccess;
     hipLaunchKernelGGL(gather_kernel, dim3(blocks(n)), dim3(256), 0, st, n, s.free_dofs, x, xa);
-    spmv<double, double, double>(n, s.nnzA, s.Arow, s.Acol, s.Aval, xa, (const double*)nullptr, 0.0, -1.0, ya, nullptr, st);
+    spmv<double, double, double>(n, s.nnzA, s.Arow, s.Acol, s.Aval, xa, (const double*)nullptr, 0.0, -1.0, ya, st);
     if (s.ncons > 0) {
         hipLaunchKernelGGL(gather_kernel, dim3(blocks(s.ncons)), dim3(256), 0, st, s.ncons, s.cons_dofs, x, xd);
-        spmv<double, double, double>(n, s.nnzD, s.Drow, s.Dcol, s.Dval, xd, ya, 1.0, -1.0, ya, nullptr, st);
+        spmv<double, double, double>(n, s.nnzD, s.Drow, s.Dcol, s.Dval, xd, ya, 1.0, -1.0, ya, st);
     }
     hipLaunchKernelGGL(scatter_kernel, dim3(blocks(n)), dim3(256), 0, st, n, s.free_dofs, ya, y);
     return hipGetLastError();
@@ -714,7 +700,7 @@ hipError_t solve_system(const SolveSystem& s, const SolveParams& prm, SolveWork&
     hipLaunchKernelGGL(gather_kernel, dim3(blocks(n)), dim3(256), 0, st, n, s.free_dofs, s.rhs, w.f);
     if (s.ncons > 0) {
         hipLaunchKernelGGL(gather_kernel, dim3(blocks(s.ncons)), dim3(256), 0, st, s.ncons, s.cons_dofs, s.rhs, w.xd);
-        spmv<double, double, double>(n, s.nnzD, s.Drow, s.Dcol, s.Dval, w.xd, w.f, 1.0, 1.0, w.f, nullptr, st);
+        spmv<double, double, double>(n, s.nnzD, s.Drow, s.Dcol, s.Dval, w.xd, w.f, 1.0, 1.0, w.f, st);
     }
     hipLaunchKernelGGL(prep_kernel, dim3(blocks(16 * n)), dim3(256), 0, st, n, s.Arow, s.Acol, s.Aval, w.val32, w.dinv);
     HIPERR(hipMemsetAsync(w.x, 0, n * sizeof(double), st));
@@ -754,7 +740,7 @@ hipError_t solve_system(const SolveSystem& s, const SolveParams& prm, SolveWork&
         }
         hipLaunchKernelGGL(add_f32_to_f64, dim3(blocks(n)), dim3(256), 0, st, n, w.d, w.x);
         // FP64 residual r = f - A x
-        spmv<double, double, double>(n, s.nnzA, s.Arow, s.Acol, s.Aval, w.x, w.f, 1.0, 1.0, w.r, nullptr, st);
+        spmv<double, double, double>(n, s.nnzA, s.Arow, s.Acol, s.Aval, w.x, w.f, 1.0, 1.0, w.r, st);
         hipLaunchKernelGGL((dot_partial<double>), dim3(G), dim3(256), 0, st, n, w.r, w.r, w.part);
         hipLaunchKernelGGL(sum_partials, dim3(1), dim3(256), 0, st, w.part, (int)G, (int)SC_DOT, w.sc);
         HIPERR(read_scalar(w.sc, SC_DOT, &h, st));
