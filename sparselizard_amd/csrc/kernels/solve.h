@@ -13,8 +13,11 @@
     } while (0)
 
 #define SLX_SOLVE_BLOCKS 1024  // partial sums of one dot product at most
+#define SLX_STREAM_BLOCKS 2048 // blocks and partial sums of the streaming product at most
 #define SLX_SOLVE_PART 2048    // half the doubles of the partial sums in the workspace
 #define SLX_ROWS_MAX 1024      // longest row of the row-wise FP32 product
+#define SLX_ROWS_SMALL 131072  // rows of unequal length on it, and
+#define SLX_ROWS_AREA 40000000 // these rows times the longest
 #define SLX_GMRES_CHECK 8      // GMRES iterations between looks at the residual
 #define SLX_STREAM_NNZ 4096    // nonzeros of one row block of the streaming FP32 product
 #define SLX_GMRES_MAX 100        // Krylov vectors per GMRES cycle at most

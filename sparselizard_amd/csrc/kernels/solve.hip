@@ -212,20 +212,35 @@ __global__ void __launch_bounds__(512) spmv_rows_f32(int64_t nrows, const int64_
     }
 }
 
-// The FP32 product of the inner iterations: rows of at most SLX_ROWS_MAX
-// nonzeros on the row kernel, longer ones (a few lanes would walk them alone)
-// on the streaming kernel.  *npart: partial sums of x.y written.
+// The FP32 product of the inner iterations.  The row kernel takes
+//  - rows of at most SLX_ROWS_MAX nonzeros, or of 64 and 256 where one lane and
+//    two walk a row: a long row is a chain of loads there.  With 1 % of the rows
+//    512 long, 4e5 rows of 5: 91 us, streaming 41; 2e4 rows of 20 (four lanes):
+//    20 us, streaming 36.
+//  - rows of nearly one length (the longest up to 1.5 times the mean) of any
+//    number, others up to SLX_ROWS_SMALL of them and SLX_ROWS_AREA: with short and
+//    long rows in a wave its loads spread over more lines than the caches of many
+//    rows in flight hold, where the streaming kernel reads in one sweep.
+// Whole CG iterations, us, row kernel and streaming: P1 2D Poisson 3.6e5 rows 24.6
+// and 26.7, P2 elasticity 1.2e5 rows 42.8 and 50, 3.5e5 88 and 79, 2.7e6 833 and
+// 668, orders 1 to 5 of hexahedra 2.3e4 rows 32 and 38, 8.5e4 84 and 59, P3 2D Poisson 9.8e5
+// rows 106 and 71.
+// *npart: partial sums of x.y written, at most SLX_STREAM_BLOCKS and at most
+// nrows of them where they are more than SLX_SOLVE_BLOCKS.
 static hipError_t inner_product(int64_t nrows, int64_t nnz, int max_row, int64_t nblk, const int64_t* blk, const int64_t* rowp,
                                 const int32_t* col, const float* val, const float* x, float* y, double* part, int* npart, hipStream_t st) {
-    if (max_row > SLX_ROWS_MAX) {
-        *npart = SLX_SOLVE_BLOCKS;
-        hipLaunchKernelGGL(spmv_stream_f32, dim3(SLX_SOLVE_BLOCKS), dim3(256), 0, st, nblk, blk, rowp, col, val, nnz, x, y, part);
-        return hipGetLastError();
-    }
     // the fewest lanes whose batches of six or eight hold the mean row
     const int64_t avg = nrows ? (nnz + nrows - 1) / nrows : 1;
     int lpr = 1;
     while (lpr < 32 && lpr * 8 < avg) lpr *= 2;
+    if (max_row > std::min(SLX_ROWS_MAX, 64 * lpr * lpr) || (2 * (int64_t)max_row > 3 * avg && (nrows > SLX_ROWS_SMALL || nrows * max_row > SLX_ROWS_AREA))) {
+        // eight blocks on a CU: four took 124 us where eight take 84 (5e5 rows of 60)
+        int64_t grid = std::min<int64_t>(SLX_STREAM_BLOCKS, (nblk + SLX_XCDS - 1) / SLX_XCDS * SLX_XCDS);
+        if (grid > nrows) grid = std::min<int64_t>(grid, SLX_SOLVE_BLOCKS);
+        *npart = (int)grid;
+        hipLaunchKernelGGL(spmv_stream_f32, dim3((unsigned)grid), dim3(256), 0, st, nblk, blk, rowp, col, val, nnz, x, y, part);
+        return hipGetLastError();
+    }
     const bool six = lpr * 6 >= avg;
     const int64_t blocks = (nrows * lpr + 511) / 512;
     const unsigned grid = (unsigned)std::min<int64_t>(SLX_SOLVE_BLOCKS, (blocks + SLX_XCDS - 1) / SLX_XCDS * SLX_XCDS);
@@ -695,7 +710,10 @@ hipError_t solve_system(const SolveSystem& s, const SolveParams& prm, SolveWork&
     if (n == 0) return hipSuccess;
     // at most SLX_SOLVE_BLOCKS blocks (every block of the next kernel sums their partials)
     const unsigned G = (unsigned)std::min<int64_t>(SLX_SOLVE_BLOCKS, (n + 255) / 256);
-    double *ppq = w.part, *prz = ppq + SLX_SOLVE_BLOCKS, *prz_new = prz + SLX_SOLVE_BLOCKS, *prr = prz_new + SLX_SOLVE_BLOCKS;
+    double *prz = w.part + SLX_SOLVE_BLOCKS, *prz_new = prz + SLX_SOLVE_BLOCKS, *prr = prz_new + SLX_SOLVE_BLOCKS;
+    // the product's partials: the streaming kernel's may be more than a quarter of
+    // w.part takes, and the full solution's place is free until the end
+    double* ppq = s.n_dofs > SLX_SOLVE_BLOCKS ? w.xfull : w.part;
     // f = b_A - D x_D ; x_D = Dirichlet values from the rhs
     hipLaunchKernelGGL(gather_kernel, dim3(blocks(n)), dim3(256), 0, st, n, s.free_dofs, s.rhs, w.f);
     if (s.ncons > 0) {

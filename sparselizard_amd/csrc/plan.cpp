@@ -3162,17 +3162,17 @@ slx_status slx_selftest_spmv_stream(slx_ctx ctx, int64_t nrows, const int64_t* r
         upload(dblk, blk.data(), blk.size(), ctx->stream);
         upload(dx, x32.data(), nrows, ctx->stream);
         dy.alloc(nrows * sizeof(float));
-        dpart.alloc((SLX_SOLVE_BLOCKS + 8) * sizeof(double));
+        dpart.alloc((SLX_STREAM_BLOCKS + 8) * sizeof(double));
         int64_t max_row = 0;
         for (int64_t r = 0; r < nrows; r++) max_row = std::max(max_row, rowp[r + 1] - rowp[r]);
         HIPCHECK(spmv_stream_probe(nrows, drow.as<int64_t>(), dcol.as<int32_t>(), dval.as<float>(), nnz,
                                    (int)std::min<int64_t>(max_row, INT32_MAX), dblk.as<int64_t>(),
                                    (int64_t)blk.size() - 1, dx.as<float>(), dy.as<float>(), dpart.as<double>(),
-                                   dpart.as<double>() + SLX_SOLVE_BLOCKS, ctx->stream));
+                                   dpart.as<double>() + SLX_STREAM_BLOCKS, ctx->stream));
         HIPCHECK(hipStreamSynchronize(ctx->stream));
         std::vector<float> y32(nrows);
         HIPCHECK(hipMemcpy(y32.data(), dy.p, nrows * sizeof(float), hipMemcpyDeviceToHost));
-        HIPCHECK(hipMemcpy(xy, dpart.as<double>() + SLX_SOLVE_BLOCKS + 1, sizeof(double), hipMemcpyDeviceToHost));
+        HIPCHECK(hipMemcpy(xy, dpart.as<double>() + SLX_STREAM_BLOCKS + 1, sizeof(double), hipMemcpyDeviceToHost));
         std::copy(y32.begin(), y32.end(), y);
     });
 }

@@ -107,10 +107,13 @@ def _random_csr(rng, lens):
     return rowp, col, val
 
 
-@pytest.mark.parametrize("case", ["short", "mixed_long", "edges"])
+@pytest.mark.parametrize("case", ["short", "mixed_long", "edges", "rows4", "rows7", "rows10", "rows25", "rows50", "rows100", "rows200",
+                                  "skewed", "many_short"])
 def test_spmv_stream_matches_numpy(ctx, case):
-    # the inner-iteration product: row blocks of at most 4096 nonzeros and
-    # 256 rows, 16-byte loads from aligned-down starts, long rows by a whole block
+    # the inner-iteration product.  Streaming: row blocks of at most 4096 nonzeros
+    # and 256 rows, long rows by a whole block, more than 131072 short rows.  By rows:
+    # one to 32 lanes, six and eight nonzeros each, rows much shorter and longer than
+    # the mean, a last workgroup that is not full
     from sparselizard_amd import _lib as L
     print("case spmv_stream", case, flush=True)
     rng = np.random.default_rng(7)
@@ -120,6 +123,16 @@ def test_spmv_stream_matches_numpy(ctx, case):
     elif case == "mixed_long":
         lens = rng.integers(20, 120, n)
         lens[[5, 777, n - 1]] = [4097, 9000, 12001]
+    elif case.startswith("rows"):
+        n, mean = 20003, int(case[4:])
+        lens = rng.integers(0, 2 * mean + 1, n)
+        lens[[0, 1, 9, n - 1]] = [0, min(1024, 4 * mean), 1, 3 * mean]
+    elif case == "skewed":
+        lens = rng.integers(2, 7, n)
+        lens[rng.choice(n, 50, replace=False)] = 700
+    elif case == "many_short":
+        n = 140001
+        lens = rng.integers(3, 9, n)
     else:
         lens = np.zeros(n, np.int64)
         lens[:300] = 1                 # more than 256 rows in one block's nonzero budget
@@ -170,7 +183,8 @@ def test_matvec_and_eliminate(ctx, kind, spec):
 
 
 @pytest.mark.parametrize("spec,precision", [("n=24", "fp64"), ("n=16;order=2", "fp64"), ("n=24", "f16split"),
-                                            ("n=24;bx=200;by=-80", "fp64")])
+                                            ("n=24;bx=200;by=-80", "fp64"),
+                                            ("n=190;bx=4000;by=-2000", "fp64")])  # over 32768 rows: dots in more than eight parts
 def test_gmres_convection_diffusion_matches_direct(ctx, spec, precision):
     # non-symmetric A: the automatic choice is GMRES; the result matches a
     # direct solve of the same assembled system
@@ -199,3 +213,25 @@ def test_solve_method_choice(ctx):
     assert relerr(x_gm, x_cg) <= 1e-9
     with pytest.raises(KeyError):
         plan.solve(info["ndofs"], method="lu")
+
+
+def test_solve_long_rows(ctx):
+    # rows of more than 1024 nonzeros and more than 1024 row blocks: the streaming
+    # product, whose partial sums are more than any other kernel's
+    import scipy.sparse as sp
+    print("case solve long rows", flush=True)
+    p = sa.Problem(ctx, "hppoisson3d", "n=7;pmin=5;pmax=5")
+    info = register_free(p)
+    plan = p.generate("fp64")
+    x, it = plan.solve(info["ndofs"], rel_tol=1e-11)
+    print("solve", it, flush=True)
+    csr, nd, nf = plan.csr(info["ndofs"]), info["ndofs"], info["nfree"]
+    assert np.diff(csr.Arow).max() > 1024 and csr.Arow[-1] > 1024 * 4096
+    free = _FREE[(nd, nf)]
+    cons = np.ones(nd, bool)
+    cons[free] = False
+    b = csr.rhs[free] - sp.csr_matrix((csr.Dval, csr.Dcol, csr.Drow), shape=(nf, nd - nf)) @ csr.rhs[cons]
+    r = b - sp.csr_matrix((csr.Aval, csr.Acol, csr.Arow), shape=(nf, nf)) @ x[free]
+    assert it["method"] == "cg" and it["rel_residual"] <= 1e-11
+    assert np.linalg.norm(r) <= 2e-11 * np.linalg.norm(b)
+    assert np.array_equal(x[cons], csr.rhs[cons])
