@@ -33,7 +33,7 @@ namespace slx {
 hipError_t launch_coef(const DevJob& one, const DevJob* jobs, int n_jobs, int max_elem, const DevInputs& in, bool fp64, void* cbase,
                        hipStream_t st, int qfast, const DevPack& pk);
 hipError_t launch_elem(const DevJob& one, const DevJob* jobs, int n_jobs, int max_elem, const void* cbase, int precision, void* ke,
-                       hipStream_t st, uint32_t slice_mask, int qfast);
+                       int n_cu, hipStream_t st, uint32_t slice_mask, int qfast);
 hipError_t scratch_init(int device);
 hipError_t launch_reduce(const DevReduce& rd, int max_erow_len, bool ke_fp64, const void* ke, double* Aval, double* Dval,
                          double* rhs, bool has_matrix, bool has_rhs, hipStream_t st, const int64_t* class_begin,
@@ -2392,7 +2392,7 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
         int p = (precision == SLX_PREC_FP64) ? SLX_PREC_FP64 : SLX_PREC_FP32;
         if ((all & ~done) != 0) {
             if (tm) tm->begin(T_VALU);
-            HIPCHECK(launch_elem(DevJob{b, (int64_t)P.ctab_off[bi]}, f.jobs, nj, f.max_elem, P.d_ctab.p, p, P.d_ke.p, bst, all & ~done, qfast));
+            HIPCHECK(launch_elem(DevJob{b, (int64_t)P.ctab_off[bi]}, f.jobs, nj, f.max_elem, P.d_ctab.p, p, P.d_ke.p, P.n_cu, bst, all & ~done, qfast));
             if (tm) tm->end();
         }
     }
