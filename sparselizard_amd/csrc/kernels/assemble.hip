@@ -610,7 +610,7 @@ hipError_t launch_coef(const DevJob& one, const DevJob* jobs, int n_jobs, int ma
 
 template <typename CT, int TI>
 static void launch_cols(const DevJob& one, const DevJob* jobs, int n_jobs, int max_elem, const void* cbase, uint32_t mask, int jc, int qfast,
-                        void* ke, int n_cu, hipStream_t st) {
+                        void* ke, hipStream_t st) {
     const DevBucket& b = one.b;
     const unsigned char* cb = (const unsigned char*)cbase;
     const int epb = 256 / jc;
@@ -629,27 +629,18 @@ static void launch_cols(const DevJob& one, const DevJob* jobs, int n_jobs, int m
         int maxt = 0;
         for (int s = 0; s < b.n_slices; s++)
             if ((mask >> s) & 1u) maxt = max(maxt, b.slices[s].n_terms);
-        size_t bytes = (size_t)epb * maxt * b.n_gp * sizeof(CT);
+        const size_t bytes = (size_t)epb * maxt * b.n_gp * sizeof(CT);
         size_t lim = 48 * 1024;
         if (const char* t = std::getenv("SLX_TUNE_ELEM_LDS_MAX")) lim = (size_t)std::min(48L * 1024, std::max(0L, std::atol(t)));
-        if (bytes <= lim) {
-            // few blocks for every CU: room for no more than that on one, which some
-            // CUs would take when the side stream's kernels hold others as this one
-            // starts (order-4 hexahedra FP32, 1728 elements in 432 blocks 5.1 ms,
-            // 3.7 so; 2744 in 686 5.2 and 4.6)
-            const int64_t share = ((int64_t)grid.x * n_jobs + n_cu - 1) / n_cu;
-            if (share <= 6) bytes = std::max<size_t>(bytes, 160 * 1024 / (share + 1) + 512);
-            SLX_COLS_GO(true, true, bytes);
-        } else {
-            SLX_COLS_GO(true, false, 0);
-        }
+        if (bytes <= lim) SLX_COLS_GO(true, true, bytes);
+        else SLX_COLS_GO(true, false, 0);
     }
 #undef SLX_COLS_GO
 }
 
 template <typename CT>
 static void launch_cols_any(const DevJob& one, const DevJob* jobs, int n_jobs, int max_elem, const void* cbase, uint32_t mask, int qfast, void* ke,
-                            int n_cu, hipStream_t st) {
+                            hipStream_t st) {
     const DevBucket& b = one.b;
     int ntf = 1, ndof = 1;
     for (int s = 0; s < b.n_slices; s++)
@@ -658,10 +649,10 @@ static void launch_cols_any(const DevJob& one, const DevJob* jobs, int n_jobs, i
             ndof = max(ndof, b.slices[s].n_dof);
         }
     const int jc = min(ndof, 64);
-    if (ntf <= 4) launch_cols<CT, 4>(one, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, n_cu, st);
-    else if (ntf <= 8) launch_cols<CT, 8>(one, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, n_cu, st);
-    else if (ntf <= 10) launch_cols<CT, 10>(one, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, n_cu, st);
-    else launch_cols<CT, 16>(one, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, n_cu, st);
+    if (ntf <= 4) launch_cols<CT, 4>(one, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, st);
+    else if (ntf <= 8) launch_cols<CT, 8>(one, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, st);
+    else if (ntf <= 10) launch_cols<CT, 10>(one, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, st);
+    else launch_cols<CT, 16>(one, jobs, n_jobs, max_elem, cbase, mask, jc, qfast, ke, st);
 }
 
 // Right-hand-side slices with many tf functions, as a blocked product over
@@ -754,7 +745,7 @@ __global__ void __launch_bounds__(256) rhs_tiles(DevJob one, const DevJob* __res
 }
 
 hipError_t launch_elem(const DevJob& one, const DevJob* jobs, int n_jobs, int max_elem, const void* cbase, int precision, void* ke,
-                       int n_cu, hipStream_t st, uint32_t slice_mask, int qfast) {
+                       hipStream_t st, uint32_t slice_mask, int qfast) {
     const DevBucket& b = one.b;
     if (max_elem == 0 || slice_mask == 0) return hipSuccess;
     // right-hand sides with more tf functions than one column pass of elem_cols
@@ -765,9 +756,9 @@ hipError_t launch_elem(const DevJob& one, const DevJob* jobs, int n_jobs, int ma
     const uint32_t mat_mask = slice_mask & ~rhs_mask;
     if (mat_mask) {
         if (precision == SLX_PREC_FP64)
-            launch_cols_any<double>(one, jobs, n_jobs, max_elem, cbase, mat_mask, qfast, ke, n_cu, st);
+            launch_cols_any<double>(one, jobs, n_jobs, max_elem, cbase, mat_mask, qfast, ke, st);
         else
-            launch_cols_any<float>(one, jobs, n_jobs, max_elem, cbase, mat_mask, qfast, ke, n_cu, st);
+            launch_cols_any<float>(one, jobs, n_jobs, max_elem, cbase, mat_mask, qfast, ke, st);
     }
     for (int s = 0; s < b.n_slices; s++) {
         if (!((rhs_mask >> s) & 1u)) continue;

@@ -536,11 +536,7 @@ __global__ void __launch_bounds__(512) factor64_kernel(int n_elem, FactorSlice f
 
 template <int BM, int BN>
 static hipError_t launch_f64(const DevBucket& b, const FactorSlice& f, const double* ctab, double* ke, int n_cu, hipStream_t st) {
-    // at least 96 KB of LDS, so that no two of the grid's workgroups share a CU:
-    // each walks its share of the elements, and when another stream's kernel held
-    // some CUs as this one started, the pairs ended last (5488 order-3 prisms
-    // beside their right-hand side's program 892 us an assembly, 745 us so)
-    const size_t lds = std::max<size_t>(factor64_lds_bytes(f), 96 * 1024);
+    const size_t lds = factor64_lds_bytes(f);
     if (lds > 160 * 1024) return hipErrorInvalidValue;
     const int64_t grid = std::min<int64_t>(b.n_elem, (int64_t)n_cu);
     hipLaunchKernelGGL((factor64_kernel<BM, BN>), dim3((unsigned)grid), dim3(512), lds, st, b.n_elem, f, ctab, ke);

@@ -33,7 +33,7 @@ namespace slx {
 hipError_t launch_coef(const DevJob& one, const DevJob* jobs, int n_jobs, int max_elem, const DevInputs& in, bool fp64, void* cbase,
                        hipStream_t st, int qfast, const DevPack& pk);
 hipError_t launch_elem(const DevJob& one, const DevJob* jobs, int n_jobs, int max_elem, const void* cbase, int precision, void* ke,
-                       int n_cu, hipStream_t st, uint32_t slice_mask, int qfast);
+                       hipStream_t st, uint32_t slice_mask, int qfast);
 hipError_t scratch_init(int device);
 hipError_t launch_reduce(const DevReduce& rd, int max_erow_len, bool ke_fp64, const void* ke, double* Aval, double* Dval,
                          double* rhs, bool has_matrix, bool has_rhs, hipStream_t st, const int64_t* class_begin,
@@ -2280,10 +2280,6 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
     // (serial when every launch is timed)
     // (a row-wise right-hand side is part of the matrix launch)
     const bool overlap = P.side_ok && !tm && !(P.direct && P.dd.has_rhs);
-    if (overlap) {
-        HIPCHECK(hipEventRecord(P.ev_fork, st));
-        HIPCHECK(hipStreamWaitEvent(P.side, P.ev_fork, 0));
-    }
     // fused launch: coefficients of every fused bucket into its region, then one
     // persistent launch over all their factorized slices
     // slices of bucket bi on the factorized kernel in this arithmetic (or in FP64)
@@ -2298,6 +2294,9 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
         }
         return m;
     };
+    // coefficient layout: the factorized kernel reads the coefficients of one
+    // element contiguously, the row-wise kernel records
+    auto layout = [&](int bi) { return P.direct && bi == P.direct_bucket ? 2 : factor_mask(bi) != 0 ? 1 : 0; };
     const int fa = arith >= 0 ? arith : ((ke64 && P.factor64) ? 3 : -1);
     const bool fused = P.fused && fa >= 0 && ((P.fused_arith >> fa) & 1u) && P.n_fused[fa] > 0;
     P.last_fused = fused;
@@ -2316,6 +2315,25 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
         }
         if (tm) tm->end();
     };
+    // The fork comes after the first matrix program, so that the matrix kernel that
+    // follows is on the CUs before the right-hand side's: programs of both at once
+    // hold some CUs as it starts, and others get more of its workgroups than their
+    // share (5488 order-3 prisms FP64 892 us an assembly, 741 so; 1728 order-4
+    // hexahedra FP32 5.1 ms and 3.8; asking for LDS that keeps the workgroups apart
+    // does the same for one plan, but takes the room of other plans' streams).  The
+    // fused launch holds every CU once it runs: the right-hand sides start ahead of it.
+    const slx_plan_s::Family* ahead = nullptr;
+    if (overlap) {
+        if (!fused)
+            for (const auto& f : P.families) {
+                if (P.rhs_only[f.buckets[0]]) continue;
+                if (!P.elem_fn[f.buckets[0]][ke64 ? 1 : 0]) ahead = &f;
+                break;
+            }
+        if (ahead) coefficients(*ahead, layout(ahead->buckets[0]), st);
+        HIPCHECK(hipEventRecord(P.ev_fork, st));
+        HIPCHECK(hipStreamWaitEvent(P.side, P.ev_fork, 0));
+    }
     if (fused) {
         for (const auto& f : P.families)
             if (P.fuse_bucket[f.buckets[0]] && factor_mask(f.buckets[0]) != 0) coefficients(f, 1, st);
@@ -2324,7 +2342,12 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
                                      P.d_fused_counter.as<unsigned long long>(), fa, P.fused_lds[fa], P.d_ke.p, P.n_cu, st));
         if (tm) tm->end();
     }
-    for (const auto& f : P.families) {
+    std::vector<const slx_plan_s::Family*> order;
+    if (ahead) order.push_back(ahead);
+    for (const auto& f : P.families)
+        if (&f != ahead) order.push_back(&f);
+    for (const auto* fp : order) {
+        const auto& f = *fp;
         const size_t bi = (size_t)f.buckets[0];
         const int nj = (int)f.buckets.size();
         const DevBucket& b = P.dbuckets[bi];
@@ -2335,10 +2358,7 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
         const void* ctab = (const char*)P.d_ctab.p + P.ctab_off[bi];
         uint32_t all = (b.n_slices >= 32) ? 0xffffffffu : ((1u << b.n_slices) - 1u);
         uint32_t done = 0;
-        // the factorized kernel reads the coefficients of one element contiguously,
-        // the row-wise kernel reads records
-        const bool records = P.direct && (int)bi == P.direct_bucket;
-        const int qfast = records ? 2 : fmask != 0 ? 1 : 0;
+        const int qfast = layout((int)bi);
         if (f.buckets.back() + 1 == (int)P.dbuckets.size()) {
             P.last_qfast = qfast;
             P.last_ctab = (const char*)P.d_ctab.p + P.ctab_off.back();
@@ -2350,8 +2370,8 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
             if (tm) tm->end();
             continue;
         }
-        if (!in_fused) coefficients(f, qfast, bst);
-        if (records || (P.direct && (int)bi == P.direct_rhs_bucket)) continue;  // the row-wise launch does the rest
+        if (!in_fused && &f != ahead) coefficients(f, qfast, bst);
+        if (qfast == 2 || (P.direct && (int)bi == P.direct_rhs_bucket)) continue;  // the row-wise launch does the rest
         if (arith >= 0 && P.mfma[bi].M > 0 && ((P.mfma[bi].arith_ok >> arith) & 1u)) {
             if (tm) tm->begin(T_MFMA);
             HIPCHECK(launch_mfma(b, mfma_for(P.mfma[bi], arith), (const float*)ctab, P.d_ke.as<float>(), bst));
@@ -2392,7 +2412,7 @@ void numeric(slx_plan_s& P, const double* xyz, const double* params, int64_t ple
         int p = (precision == SLX_PREC_FP64) ? SLX_PREC_FP64 : SLX_PREC_FP32;
         if ((all & ~done) != 0) {
             if (tm) tm->begin(T_VALU);
-            HIPCHECK(launch_elem(DevJob{b, (int64_t)P.ctab_off[bi]}, f.jobs, nj, f.max_elem, P.d_ctab.p, p, P.d_ke.p, P.n_cu, bst, all & ~done, qfast));
+            HIPCHECK(launch_elem(DevJob{b, (int64_t)P.ctab_off[bi]}, f.jobs, nj, f.max_elem, P.d_ctab.p, p, P.d_ke.p, bst, all & ~done, qfast));
             if (tm) tm->end();
         }
     }

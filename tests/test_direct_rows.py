@@ -154,6 +154,7 @@ SHAPES = [
     (2, 2, 9, 10, 10, 700, 300, "same"),
     (1, 1, 9, 20, 20, 12000, 2500, "none"),  # rows of 1300 columns: fewer than 16 of them a wave
     (1, 1, 12, 12, 12, 900, 400, "same"),
+    (2, 2, 9, 10, 10, 90, 80, "apart"),      # a right-hand side that keeps its kernels, on the side stream
 ]
 
 
@@ -163,8 +164,8 @@ def synthetic(na, nb, n_pairs, n_tf, n_dof, n_elem, per_field, rhs, seed=3):
     tf = [addresses(rng, n_tf, n_elem, a * per_field, (a + 1) * per_field, 0.03) for a in range(na)]
     dof = [addresses(rng, n_dof, n_elem, b * per_field, (b + 1) * per_field, 0.03) for b in range(nb)]
     mat = [dict(tf=t, dof=u, pairs=ALL[:n_pairs]) for t in tf for u in dof]
-    rows = [dict(tf=t, pairs=[(a % 4, 0)]) for a, t in enumerate(tf)]
-    buckets = [mat + rows] if rhs == "same" else [mat, rows] if rhs == "other" else [mat]
+    rows = [dict(tf=t, pairs=[(a % 4, 0), (3, 0)][:2 if rhs == "apart" else 1]) for a, t in enumerate(tf)]
+    buckets = [mat + rows] if rhs == "same" else [mat] if rhs == "none" else [mat, rows]
     return Synthetic(buckets, nf * per_field, rng.random(nf * per_field) < 0.1, seed)
 
 
