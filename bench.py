@@ -1,7 +1,10 @@
 #!/usr/bin/env python3
-"""Benchmark: assembled nnz/s of the mixed-precision MFMA path vs the plain FP64
+"""Benchmark: assembled nnz/s of the mixed-precision path vs the plain FP64
 GPU path on the 3D linear-elasticity workload (h1xyz P2 on 64^3 x 6 Kuhn
-tetrahedra, jittered, E lognormal per element, nu = 0.3).
+tetrahedra, jittered, E lognormal per element, nu = 0.3).  These tetrahedra have
+constant coefficients and are assembled row by row: FP32 products summed in FP64
+in every reduced mode, FP64 in the FP64 mode, and no MFMA work in either; the
+other problems run the mode's MFMA kernels.
 
 One step = one numeric assembly (Jacobians, Gauss-point coefficients, element
 contractions, deterministic FP64 reduction into the cached CSR pattern + rhs)
@@ -176,7 +179,7 @@ def main():
     for mode in [v for v in args.variants.split(",") if v and v != args.mixed]:
         ms_v, _ = timed(mode)
         entry = {"ms_per_step": ms_v, "nnz_per_s": nnz / (ms_v * 1e-3), "ratio_vs_fp64": ms64 / ms_v,
-                 "kernels": plan.kernel_counts(mode)}
+                 "kernels": dict(plan.kernel_counts(mode), row_wise=plan.routes(mode)["row_wise"])}
         if ref is not None:
             vcsr = csr_now()
             entry["rel_err_vs_fp64_gpu"] = {"global_frobenius": glob_err(vcsr), "rhs": rel(vcsr.rhs, ref.rhs)}
@@ -228,8 +231,16 @@ def main():
             sd = bd.slices[s_]
             if not sd.is_rhs:
                 con_bytes += bd.n_elem * sd.n_tf * sd.n_dof * 4.0
-    kname = ("factor_contract_kernel" if args.problem == "hppoisson3d" else "mfma_contract_kernel") \
-        if prof_mix["mfma"] > 0 else "elem_cols"
+    routes = plan.routes(args.mixed)
+    rowwise = routes["row_wise"]
+    if prof_mix["mfma"] == 0:
+        kname = "slx_elem" if routes["elem_fused"] else "elem_cols"
+    elif plan.kernel_counts(args.mixed)["factorized"]:
+        kname = "factor_contract_kernel"
+    elif plan.tile_count(args.mixed):
+        kname = "slx_tile" if routes["tile_compiled"] else "tile_qv_kernel"
+    else:
+        kname = "mfma_contract_kernel"
     if t_contract >= prof_mix["reduce"]:
         # the roofline that bounds the kernel: the larger of the two ideal times
         t_flop = flops / (peak_elem * 1e12)
@@ -246,10 +257,7 @@ def main():
                     "kernel_ms": round(t_contract, 4), "algorithmic": con_bytes,
                     "mfma_tflops": round(flops / (t_contract * 1e-3) / 1e12, 3)}
     else:
-        # constant coefficients and no contraction launch: the row-wise kernel
-        # assembles straight into the CSR values, without element matrices
-        rowwise = prof_mix["mfma"] == 0 and all(d.buckets[b].q_invariant for b in range(d.n_buckets)
-                                                if any(not d.buckets[b].slices[s_].is_rhs for s_ in range(d.buckets[b].n_slices)))
+        # the row-wise kernel assembles straight into the CSR values, without element matrices
         if rowwise:
             ke_roundtrip = 0
         achieved = red_bytes / (prof_mix["reduce"] * 1e-3) / 1e9
@@ -298,7 +306,9 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": {"f16split": "f16x2-split/f32acc/f64reduce", "bf16split": "bf16x3-split/f32acc/f64reduce",
+        # reduced modes without MFMA work (row-wise plans, small elements) compute FP32 products
+        "dtype": "f32/f64reduce" if prof_mix["mfma"] == 0 and args.mixed != "fp64" else
+                 {"f16split": "f16x2-split/f32acc/f64reduce", "bf16split": "bf16x3-split/f32acc/f64reduce",
                   "fp32": "f32/f64reduce"}.get(args.mixed, args.mixed),
         "data": "synthetic",
         "config": {"workload": workload_name(args, n_elem),

@@ -592,7 +592,7 @@ class Plan:
     COEF_MODES = {"auto": 0, "interpreter": 1, "compiled": 2}
 
     def coef_mode(self, mode):
-        """Coefficient programs: "auto" (compiled for buckets of >= 4096 elements),
+        """Coefficient programs: "auto" (compiled for programs that at least 512 elements run),
         "interpreter" or "compiled"; returns the compiled kernels in use."""
         n = C.c_int32()
         check(lib().slx_plan_coef_mode(self.h, self.COEF_MODES[mode], C.byref(n)))

@@ -585,9 +585,9 @@ __global__ void reduce_rhs(DevReduce rd, const KT* __restrict__ ke, double* __re
 
 // one: a bucket of the launch (they agree but for their elements), by value
 // where it is the only one: the interpreter reads the description for every
-// instruction, and through memory one launch took 12 to 28 us more (P2
-// elasticity 162 elements 145 vs 170 us, orders 1 to 5 of 64 hexahedra 337 vs
-// 395 us an assembly).  max_elem: the largest bucket's elements.
+// instruction.  Through memory an assembly of 250 order-1 prisms took 148 us, by
+// value 136, orders 1 to 5 of 64 hexahedra 395 and 340, Newton on 288 triangles 159
+// and 136.  max_elem: the largest bucket's elements.
 hipError_t launch_coef(const DevJob& one, const DevJob* jobs, int n_jobs, int max_elem, const DevInputs& in, bool fp64, void* cbase,
                        hipStream_t st, int qfast, const DevPack& pk) {
     const DevBucket& b = one.b;

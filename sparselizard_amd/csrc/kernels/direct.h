@@ -14,10 +14,11 @@ namespace slx {
 #define SLX_DIRECT_PAD 16                // segments and slot blocks readable past the last row
 
 // One plan's row-wise description.  A segment (element e, group a, tf function
-// i) is the 32-bit word e << (ib + ab) | a << ib | i; its entries are
+// i) is the 32-bit word (e * na + a) << ib | i; its entries are
 //   Ke(b, j) = sum_p C(e)[a][b][p] Phi_p[i][j],   b < nb, j < n_dof
-// with C the element's coefficient record ([a][rec], rec = nb * P rounded up to
-// 4, zeros in the padding) and Phi the Gauss-point sums of the table products.
+// with C the element's coefficient record ([a][rec]: nb * P values rounded up to
+// 4, then the group's share of the bucket's right-hand-side coefficients rounded up
+// to 4; zeros in the padding) and Phi the Gauss-point sums of the table products.
 struct DirectDev {
     int32_t n_tf, n_dof, na, nb;
     int32_t P, JL, G;                       // pairs rounded up to a kernel's; columns per lane, lanes per row

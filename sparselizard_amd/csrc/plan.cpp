@@ -1610,10 +1610,11 @@ int bits_for(int64_t n) {
 // The right-hand side joins the launch when its slices sit in one such bucket
 // with one term each; otherwise it keeps its kernels (and then must not share
 // the matrix bucket).  Measured against the element kernels with the
-// reduction, whole assemblies: 48^3 x 6 P2 elasticity 1.19 vs 1.90 ms (FP16
-// split), 21^3 x 6 in FP64 0.145 vs 0.72 ms, 200^2 x 2 P1 Poisson 0.011 vs
-// 0.040 ms (three launches instead of six and no side stream); no class
-// measured slower.
+// reduction, whole assemblies, us: P2 elasticity FP16 split 48^3 x 6 1180 and 1900,
+// 24^3 x 6 from host memory 288 and 420, 8^3 x 6 42 and 245, 3^3 x 6 (interpreted
+// coefficients) 207 and 208; 21^3 x 6 in FP64 137 and 720; P1 Poisson 200^2 x 2 13 and
+// 54, 10^2 x 2 14 and 53.  Orders 3 and higher of these elements come in several
+// orientation buckets and do not take it.
 // SLX_TUNE_DIRECT=0 and SLX_TUNE_TABLE=none keep the element kernels.
 void choose_direct(slx_plan_s& P, const slx_plan_desc& d, const KeLayout& L) {
     P.direct = false;
@@ -2060,10 +2061,14 @@ void upload_buckets(slx_plan_s& P, const slx_plan_desc& d, const KeLayout& L) {
 // Compiled coefficient programs for the buckets the mode selects (auto: programs
 // that at least SLX_COEF_JIT_MIN elements run, over all buckets: the
 // interpreter's scratch registers cost the same per element whatever its
-// bucket); unique programs compiled in parallel.  At 4096 hp Poisson 9^3 (729
-// hexahedra, orders 1 to 5) took 565 us a call on the interpreter and the general
-// kernels, at 512 443 us; P2 elasticity on 750 tetrahedra 115 and 22 us.  Below,
-// the calls are launches and the compiler's half second is not earned back.
+// bucket); unique programs compiled in parallel.  Interpreted and compiled, us an
+// assembly: orders 1 to 5 of 512 hexahedra 401 and 248, P2 elasticity on 750
+// tetrahedra 229 and 40, Newton on 512 triangles 137 and 53.  The first plan of a
+// process that needs a program waits for the compiler: 0.3 s (Poisson), 0.6 s
+// (elasticity), 0.7 to 1.2 s (Newton, prisms), 1.7 s (Maxwell, 24 buckets), 3.2 s (five
+// orders, 25 kernels), against 0.01 to 0.07 s.  The smallest plans, where the launches
+// and the interpreter's fixed 100 to 200 us are all there is, don't ask for that:
+// 0.6 s are 4000 assemblies of 162 tetrahedra.
 #define SLX_COEF_JIT_MIN 512
 //
 // Element kernels: a bucket whose slices all run on the VALU element kernel in
