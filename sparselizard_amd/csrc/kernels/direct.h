@@ -36,8 +36,7 @@ struct DirectDev {
     const int64_t* rptr;                    // [nrows + 1]
     const uint32_t* rseg;
     const int64_t* rbase;
-    const float* rphi32;
-    const double* rphi64;
+    const double* rphi;
     const int64_t* free_dofs;
 };
 

@@ -195,14 +195,9 @@ hipError_t launch_direct(const DirectDev& d, bool fp64, const void* ctab, const 
 // One thread per element-matrix entry, the sums of direct_rows.
 template <typename KT>
 __global__ void direct_ke_kernel(DirectDev d, DirectBuild b, const KT* __restrict__ ctab, const KT* __restrict__ rtab, KT* __restrict__ ke) {
-    const KT *phi, *rphi;
-    if constexpr (sizeof(KT) == 4) {
-        phi = (const KT*)d.phi32;
-        rphi = (const KT*)d.rphi32;
-    } else {
-        phi = (const KT*)d.phi64;
-        rphi = (const KT*)d.rphi64;
-    }
+    const KT* phi;
+    if constexpr (sizeof(KT) == 4) phi = (const KT*)d.phi32;
+    else phi = (const KT*)d.phi64;
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int per = d.nb * d.n_dof;
     const int64_t nmat = (int64_t)d.na * b.n_elem * d.n_tf * per;
@@ -225,7 +220,7 @@ __global__ void direct_ke_kernel(DirectDev d, DirectBuild b, const KT* __restric
             if (u < n) {
                 const int64_t e = u / b.rgroup_ntf[g];
                 const int k = b.rgroup_k[g] + (int)(u - e * b.rgroup_ntf[g]);
-                ke[b.rgroup_base[g] + u] = -(rtab[d.rbase[k] + e * d.rstride] * rphi[k]);
+                ke[b.rgroup_base[g] + u] = (KT)-((double)rtab[d.rbase[k] + e * d.rstride] * d.rphi[k]);
                 break;
             }
             u -= n;

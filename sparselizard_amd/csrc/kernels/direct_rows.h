@@ -38,24 +38,26 @@ __device__ inline void direct_load(const KT* p, KT (&v)[N]) {
 }
 
 // The right-hand side of one free row: its entries in accumulation order
-// (rawvec.cpp:216-254), four loads in flight.
+// (rawvec.cpp:216-254), four loads in flight.  The products are FP64 in every
+// mode: with FP32 ones the rounded Gauss-point sums, the same in all entries, made
+// the sums of FP32 coefficients 1.3 times as far off as a sum over the Gauss points.
 template <typename KT>
-__device__ inline void direct_rhs_row(const DirectDev& d, const KT* __restrict__ rtab, const KT* __restrict__ rphi, int64_t r,
+__device__ inline void direct_rhs_row(const DirectDev& d, const KT* __restrict__ rtab, const double* __restrict__ rphi, int64_t r,
                                       double* __restrict__ rhs) {
     const uint32_t kmask = (1u << d.rib) - 1u;
     double s = 0.0;
     int64_t k = d.rptr[r];
     const int64_t k1 = d.rptr[r + 1];
     for (; k < k1; k += 4) {
-        KT v[4];
+        double v[4];
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             const uint32_t w = k + u < k1 ? d.rseg[k + u] : 0u;
             const uint32_t f = w & kmask;
-            v[u] = k + u < k1 ? -(rtab[d.rbase[f] + (int64_t)(w >> d.rib) * d.rstride] * rphi[f]) : (KT)0;
+            v[u] = k + u < k1 ? -((double)rtab[d.rbase[f] + (int64_t)(w >> d.rib) * d.rstride] * rphi[f]) : 0.0;
         }
 #pragma unroll
-        for (int u = 0; u < 4; u++) s += (double)v[u];
+        for (int u = 0; u < 4; u++) s += v[u];
     }
     rhs[d.free_dofs[r]] = s;
 }
@@ -162,17 +164,11 @@ __global__ void __launch_bounds__((256 * direct_waves<KT, NB, P>()), (direct_wav
     constexpr int NBUF = NB * P * (int)sizeof(KT) <= 48 ? 4 : sizeof(KT) == 4 ? 3 : 2;
     extern __shared__ __attribute__((aligned(16))) unsigned char direct_lds[];
     const KT* phi_g;
-    const KT* rphi;
-    if constexpr (sizeof(KT) == 4) {
-        phi_g = (const KT*)d.phi32;
-        rphi = (const KT*)d.rphi32;
-    } else {
-        phi_g = (const KT*)d.phi64;
-        rphi = (const KT*)d.rphi64;
-    }
+    if constexpr (sizeof(KT) == 4) phi_g = (const KT*)d.phi32;
+    else phi_g = (const KT*)d.phi64;
     if (blockIdx.x >= mat_blocks) {
         const int64_t r = (int64_t)(blockIdx.x - mat_blocks) * blockDim.x + threadIdx.x;
-        if (r < d.nrows) direct_rhs_row<KT>(d, rtab, rphi, r, rhs);
+        if (r < d.nrows) direct_rhs_row<KT>(d, rtab, d.rphi, r, rhs);
         return;
     }
     const int nphi = d.n_tf * G * PJ;

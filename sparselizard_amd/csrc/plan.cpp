@@ -1773,10 +1773,8 @@ void choose_direct(slx_plan_s& P, const slx_plan_desc& d, const KeLayout& L) {
                 rbase.push_back(rb == mb ? pack.pos[sd.terms[0].coef] : (int64_t)sd.terms[0].coef * rd.n_elem);
             }
         }
-        const std::vector<float> rphi32(rphi.begin(), rphi.end());
         P.dd.rstride = rb == mb ? pack.erec : 1;
-        P.dd.rphi64 = P.dev(rphi.data(), rphi.size());
-        P.dd.rphi32 = P.dev(rphi32.data(), rphi32.size());
+        P.dd.rphi = P.dev(rphi.data(), rphi.size());
         P.dd.rbase = P.dev(rbase.data(), rbase.size());
     }
     std::vector<int32_t> pads(pack.pads.begin(), pack.pads.end());

@@ -60,6 +60,17 @@ def test_rows_match_oracle(ctx, kind, spec, precision, tol):
     assert np.array_equal(a.Aval, b.Aval) and np.array_equal(a.Dval, b.Dval) and np.array_equal(a.rhs, b.rhs)
 
 
+@pytest.mark.parametrize("precision", ["f16split", "fp32"])
+@pytest.mark.parametrize("spec", ["n=6", "n=25"])
+def test_rhs_rounds_only_its_coefficients(ctx, spec, precision):
+    """The reduced modes' right-hand side sums FP64 products of FP32 coefficients: an entry of a row is off
+    by 2^-24 / sqrt(3) (root mean square) at most, and rows have six of them or more: 1.4e-8."""
+    prob = sa.Problem(ctx, "poisson2d", spec)
+    ref = prob.generate("fp64").csr(prob.info()["ndofs"]).rhs
+    got = prob.generate(precision).csr(prob.info()["ndofs"]).rhs
+    assert relerr(got, ref) <= 1.5e-8
+
+
 @pytest.mark.parametrize("kind,spec", [("poisson2d", "n=9"), ("elasticity3d", "n=3")])
 @pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("fp32", 1e-6)])
 def test_compiled_records(ctx, kind, spec, precision, tol):
