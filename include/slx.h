@@ -361,9 +361,9 @@ slx_status slx_selftest_mfma_layout(slx_ctx ctx, float* out256);
  * and 3 (v_mfma_f64_16x16x4_f64) on A[m][k] = (m + 2k) % 7 - 3,
  * B[k][n] = (3k + n) % 5 - 2 (kind 0 is slx_selftest_mfma_layout). */
 slx_status slx_selftest_mfma_layout_kind(slx_ctx ctx, int32_t kind, float* out256);
-/* Test hook: the streaming FP32 CSR product of slx_plan_solve's inner
- * iteration on a host CSR (square, nrows rows; values and x rounded to FP32):
- * y = A x and xy = x . y (FP64 sum of the FP32 products). */
+/* Test hook: the FP32 CSR product of slx_plan_solve's inner iteration (by rows
+ * or streamed, as the rule of the solve chooses) on a host CSR (square, nrows
+ * rows; values and x rounded to FP32): y = A x and xy = x . y (FP64 sum of the FP32 products). */
 slx_status slx_selftest_spmv_stream(slx_ctx ctx, int64_t nrows, const int64_t* rowp, const int32_t* col,
                                     const double* val, const double* x, double* y, double* xy);
 /* Test hook: a device allocation of more bytes than any device has; *kept = the

@@ -178,7 +178,7 @@ def mfma_layout_probe(ctx, kind=0):
 
 
 def spmv_stream_probe(ctx, rowp, col, val, x):
-    """The solve's streaming FP32 CSR product on a host CSR: (y, x.y)."""
+    """The FP32 CSR product of the solve's inner iterations on a host CSR: (y, x.y)."""
     rowp = np.ascontiguousarray(rowp, np.int64)
     col = np.ascontiguousarray(col, np.int32)
     val = np.ascontiguousarray(val, np.float64)

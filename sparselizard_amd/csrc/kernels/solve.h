@@ -77,7 +77,7 @@ hipError_t eliminate_system(const SolveSystem& s, const double* b, double* out, 
 // y[free] = A x[free] + D x[constrained], y[constrained] = x[constrained]
 // (x, y: n_dofs entries; xa, ya: nfree work; xd: ncons work)
 hipError_t matvec_system(const SolveSystem& s, const double* x, double* y, double* xa, double* xd, double* ya, hipStream_t st);
-// y = A x with the streaming FP32 product on any CSR; sc[1] = x.y
+// y = A x with the inner iterations' FP32 product on any CSR; sc[1] = x.y
 hipError_t spmv_stream_probe(int64_t nrows, const int64_t* rowp, const int32_t* col, const float* val, int64_t nnz,
                              int max_row, const int64_t* blk, int64_t nblk, const float* x, float* y, double* part, double* sc, hipStream_t st);
 

@@ -54,7 +54,7 @@ __device__ inline void split(const float (&v)[8], tj_u4 (&qp)[NPL]) {
             }
         }
     } else {
-// v - hi and its rounding in one instruction (v_fma_mixlo/mixhi_f16; a
+        // v - hi and its rounding in one instruction (v_fma_mixlo/mixhi_f16; a
         // constant -1 would fold to a conversion and a subtraction)
         float neg = -1.f;
         asm("" : "+s"(neg));
